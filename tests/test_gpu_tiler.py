@@ -48,3 +48,37 @@ def test_tiled_generation_writes_loadable_trees(tmp_path):
         d = os.path.join(str(tmp_path), f"grid_{x}_{y}_{z}")
         p = oracle.pool_load(d, slots=(8, 8, 8))
         assert p.blocks >= 1
+
+
+def _soup(ntri, seed, dim, spread):
+    """Triangles over a dim[0] x dim[1] tile grid of unit tiles: most within
+    a tile or across an edge, one in eight with edges of `spread` tiles."""
+    rng = np.random.default_rng(seed)
+    c = rng.uniform(-0.5, 1.0, (ntri, 1, 3)) + rng.uniform(0, 1, (ntri, 1, 3)) * (dim[0], dim[1], 1)
+    e = np.where(rng.random((ntri, 1, 1)) < 0.125, spread, 0.2)
+    return (c + rng.normal(size=(ntri, 3, 3)) * e).astype(np.float32)
+
+
+# counts around a group of 64, a workgroup's run and two of them; grids of one
+# tile, ragged ones, the largest whose counters fit LDS (1024 tiles) and the
+# next (sorted instead)
+@pytest.mark.parametrize("ntri,dim,spread", [
+    (1, (1, 1), 0.2), (63, (3, 1), 1.0), (64, (1, 5), 1.0), (65, (7, 5), 2.0), (256, (4, 4), 9.0),
+    (257, (31, 33), 3.0), (700, (32, 32), 40.0), (700, (33, 32), 40.0), (3001, (5, 3), 1.0)])
+def test_device_assignment_sizes(ntri, dim, spread):
+    from voxvizthesis_amd import _lib
+    verts = _soup(ntri, ntri, dim, spread)
+    g = _lib.VoxTileGrid()
+    g.origin[:], g.size[:], g.border[:], g.dim[:] = (0.0, 0.0), (1.0, 1.0), (0.1, 0.1), dim
+    print(f"[tiler] {ntri} triangles on {dim}", flush=True)
+    a = TileAssignment(verts, g)
+    ref = ot.assign(verts, (0.0, 0.0), (1.0, 1.0), (0.1, 0.1), dim)
+    assert a.start[0] == 0 and a.start[-1] == a.tris.size == sum(map(len, ref.values()))
+    for t in range(dim[0] * dim[1]):
+        want = ref.get(t, [])
+        assert a.tile(t).tolist() == want, f"tile {t}"
+        z = verts[want][:, :, 2]
+        if want:
+            assert a.zmin[t] == z.min() and a.zmax[t] == z.max(), f"tile {t}"
+        else:
+            assert np.isnan(a.zmin[t]) and np.isnan(a.zmax[t]), f"tile {t}"
