@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 from oracle.server import NONE
-from voxvizthesis_amd import scenes
+from voxvizthesis_amd import _lib, scenes
 from voxvizthesis_amd.terrain import DeviceTerrain, TerrainPager, c5_height_fn
 from voxvizthesis_amd.voxelizer import Voxelizer
 
@@ -52,6 +52,34 @@ def test_device_heights_with_ridged_term():
         assert z[0] == want[0, 0] and z[1] == want[128, 128]
         assert z[2] == want[int(np.floor(2000 / 32 + 0.5)), int(np.floor(1000 / 32 + 0.5))]
     finally:
+        t.close()
+
+
+# windows of one cell, around a workgroup's 256 cells and of several rows;
+# outputs 16-byte aligned and one float off
+@pytest.mark.parametrize("x0,y0,cw,ch,off", [(299, 299, 1, 1, 0), (0, 0, 255, 1, 0),
+                                             (3, 7, 256, 1, 4), (40, 0, 257, 1, 0),
+                                             (5, 9, 51, 37, 4), (0, 0, 300, 300, 0)])
+def test_device_tile_windows(x0, y0, cw, ch, off):
+    print(f"[terrain] window {x0} {y0} {cw}x{ch} offset {off}", flush=True)
+    t = DeviceTerrain(300, 1.0, 11)
+    nt = 2 * cw * ch
+    bufs = [_lib.DeviceArray.alloc(4 * k * nt + off) for k in (9, 9, 6)]
+    try:
+        ref = scenes.heightfield_terrain(300, 11)
+        g = t.grid()
+        win = g[y0:y0 + ch + 1, x0:x0 + cw + 1]
+        assert t.range(x0, y0, cw + 1, ch + 1) == (win.min(), win.max())
+        assert t._L.vox_terrain_tile(t.heights.ptr, t.n1, 1.0, x0, y0, cw, ch, t.lo, t.hi, 256,
+                                     *(b.ptr + off for b in bufs))
+        for b, k, want in zip(bufs, (9, 9, 6), (ref.verts, ref.vnormals, ref.uvs)):
+            a = np.empty(nt * k, np.float32)
+            assert t._L.vox_device_download(a.ctypes.data, b.ptr, off, a.nbytes)
+            w = want.reshape(300, 300, 2, -1)[y0:y0 + ch, x0:x0 + cw]
+            assert np.array_equal(a, w.reshape(-1))
+    finally:
+        for b in bufs:
+            b.close()
         t.close()
 
 

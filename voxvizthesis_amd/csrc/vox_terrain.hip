@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -120,80 +121,147 @@ __global__ void k_heights(float* __restrict__ out, uint32_t n1, double extent, d
     out[k] = (float)h;
 }
 
-// Triangles of cells [x0, x0 + cw) x [y0, y0 + ch), row by row, two per
-// cell: (v00, v10, v11), (v00, v11, v01).
-__global__ void k_tile(const float* __restrict__ H, uint32_t n1, double step, float dxf,
-                       uint32_t x0, uint32_t y0, uint32_t cw, uint32_t ch, double lo, double hi,
-                       uint32_t texW, float* __restrict__ verts, float* __restrict__ vn,
-                       float* __restrict__ uv) {
-    const uint64_t c = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= (uint64_t)cw * ch) return;
-    const uint32_t cj = (uint32_t)(c / cw), ci = (uint32_t)(c - (uint64_t)cj * cw);
-    const uint32_t i = x0 + ci, j = y0 + cj;
-    // corners (x, y): 00 = (i, j), 10 = (i+1, j), 11 = (i+1, j+1), 01 = (i, j+1)
-    const uint32_t ix[4] = {i, i + 1, i + 1, i}, iy[4] = {j, j, j + 1, j + 1};
-    float p[4][3], nrm[4][3];
-    const float two = 2.0f;
-    for (int q = 0; q < 4; ++q) {
-        const uint32_t a = ix[q], b = iy[q];
-        p[q][0] = (float)((double)a * step);
-        p[q][1] = (float)((double)b * step);
-        p[q][2] = H[(uint64_t)b * n1 + a];
-        // central differences, the rim padded with the edge value
-        const uint32_t am = a > 0 ? a - 1 : 0, ap = a + 1 < n1 ? a + 1 : n1 - 1;
-        const uint32_t bm = b > 0 ? b - 1 : 0, bp = b + 1 < n1 ? b + 1 : n1 - 1;
-        const float dhdx = (H[(uint64_t)b * n1 + ap] - H[(uint64_t)b * n1 + am]) / (two * dxf);
-        const float dhdy = (H[(uint64_t)bp * n1 + a] - H[(uint64_t)bm * n1 + a]) / (two * dxf);
-        const float nx = -dhdx, ny = -dhdy, nz = 1.0f;
-        const float l = sqrtf((nx * nx + ny * ny) + nz * nz);
-        nrm[q][0] = nx / l;
-        nrm[q][1] = ny / l;
-        nrm[q][2] = nz / l;
+// The workgroup's run of `count` floats from LDS to dst, whole 16-byte words
+// where dst is aligned.
+constexpr int kTileBlock = 256;
+__device__ __forceinline__ void store_run(const float* s, float* __restrict__ dst, uint32_t count) {
+    const uint32_t tid = threadIdx.x;
+    uint32_t done = 0;
+    if ((reinterpret_cast<uintptr_t>(dst) & 15u) == 0u) {
+        const float4* s4 = reinterpret_cast<const float4*>(s);
+        float4* d4 = reinterpret_cast<float4*>(dst);
+        for (uint32_t k = tid; k < count / 4u; k += kTileBlock) d4[k] = s4[k];
+        done = count & ~3u;
     }
-    const int tri[2][3] = {{0, 1, 2}, {0, 2, 3}};
-    for (int t = 0; t < 2; ++t) {
-        const uint64_t o = 2 * c + t;
-        double hs = 0.0;
-        for (int k = 0; k < 3; ++k) {
-            const int q = tri[t][k];
-            for (int a = 0; a < 3; ++a) {
-                verts[9 * o + 3 * k + a] = p[q][a];
-                vn[9 * o + 3 * k + a] = nrm[q][a];
-            }
-            hs = k == 0 ? (double)p[q][2] : hs + (double)p[q][2];
-        }
-        const double hmean = hs / 3.0;
-        const double span = hi - lo > 1e-12 ? hi - lo : 1e-12;
-        const double tt = (hmean - lo) / span;
-        int64_t idx = (int64_t)(tt * (double)texW);
-        idx = idx < 0 ? 0 : (idx > (int64_t)texW - 1 ? (int64_t)texW - 1 : idx);
-        const float u = ((float)idx + 0.5f) / (float)texW;
-        for (int k = 0; k < 3; ++k) {
-            uv[6 * o + 2 * k] = u;
-            uv[6 * o + 2 * k + 1] = 0.5f;
-        }
-    }
+    for (uint32_t k = done + tid; k < count; k += kTileBlock) dst[k] = s[k];
 }
 
-// Min and max of a window of the grid: one block per row, atomics on the
-// order-preserving integer images of the floats.
-// (negative floats map below every non-negative one, in order; the map is
-// its own inverse on the bit patterns)
+// Triangles of cells [x0, x0 + cw) x [y0, y0 + ch), row by row, two per
+// cell: (v00, v10, v11), (v00, v11, v01).  A thread computes one cell; the
+// workgroup's 256 cells are consecutive in every output, so each output
+// goes through LDS and out in consecutive 16-byte words (bound by the 192
+// bytes written per cell; a thread storing its own cell's words left the
+// 72-byte strides to the cache: 71 us for 1023 x 1021 cells, 34 us so, 6.1
+// TB/s).
+__global__ __launch_bounds__(kTileBlock) void k_tile(
+    const float* __restrict__ H, uint32_t n1, double step, float dxf, uint32_t x0, uint32_t y0,
+    uint32_t cw, uint32_t ch, double lo, double hi, uint32_t texW, float* __restrict__ verts,
+    float* __restrict__ vn, float* __restrict__ uv) {
+    __shared__ __align__(16) float s_out[kTileBlock * 18];
+    const uint64_t n = (uint64_t)cw * ch, c0 = (uint64_t)blockIdx.x * kTileBlock;
+    const uint64_t c = c0 + threadIdx.x;
+    const uint32_t cells = (uint32_t)(n - c0 < (uint64_t)kTileBlock ? n - c0 : (uint64_t)kTileBlock);
+    float p[4][3] = {}, nrm[4][3] = {}, tu[2] = {};
+    constexpr int tri[2][3] = {{0, 1, 2}, {0, 2, 3}};
+    if (c < n) {
+        const uint32_t cj = (uint32_t)(c / cw), ci = (uint32_t)(c - (uint64_t)cj * cw);
+        const uint32_t i = x0 + ci, j = y0 + cj;
+        // corners (x, y): 00 = (i, j), 10 = (i+1, j), 11 = (i+1, j+1), 01 = (i, j+1)
+        const uint32_t ix[4] = {i, i + 1, i + 1, i}, iy[4] = {j, j, j + 1, j + 1};
+        const float two = 2.0f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t a = ix[q], b = iy[q];
+            p[q][0] = (float)((double)a * step);
+            p[q][1] = (float)((double)b * step);
+            p[q][2] = H[(uint64_t)b * n1 + a];
+            // central differences, the rim padded with the edge value
+            const uint32_t am = a > 0 ? a - 1 : 0, ap = a + 1 < n1 ? a + 1 : n1 - 1;
+            const uint32_t bm = b > 0 ? b - 1 : 0, bp = b + 1 < n1 ? b + 1 : n1 - 1;
+            const float dhdx = (H[(uint64_t)b * n1 + ap] - H[(uint64_t)b * n1 + am]) / (two * dxf);
+            const float dhdy = (H[(uint64_t)bp * n1 + a] - H[(uint64_t)bm * n1 + a]) / (two * dxf);
+            const float nx = -dhdx, ny = -dhdy, nz = 1.0f;
+            const float l = sqrtf((nx * nx + ny * ny) + nz * nz);
+            nrm[q][0] = nx / l;
+            nrm[q][1] = ny / l;
+            nrm[q][2] = nz / l;
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            double hs = 0.0;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const int q = tri[t][k];
+                hs = k == 0 ? (double)p[q][2] : hs + (double)p[q][2];
+            }
+            const double hmean = hs / 3.0;
+            const double span = hi - lo > 1e-12 ? hi - lo : 1e-12;
+            const double tt = (hmean - lo) / span;
+            int64_t idx = (int64_t)(tt * (double)texW);
+            idx = idx < 0 ? 0 : (idx > (int64_t)texW - 1 ? (int64_t)texW - 1 : idx);
+            tu[t] = ((float)idx + 0.5f) / (float)texW;
+        }
+    }
+    auto corners = [&](const float (&v)[4][3], float* __restrict__ dst) {
+        float* s = s_out + 18 * threadIdx.x;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+#pragma unroll
+                for (int a = 0; a < 3; ++a) s[9 * t + 3 * k + a] = v[tri[t][k]][a];
+        __syncthreads();
+        store_run(s_out, dst + 18 * c0, 18u * cells);
+        __syncthreads();
+    };
+    corners(p, verts);
+    corners(nrm, vn);
+    float* s = s_out + 12 * threadIdx.x;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            s[6 * t + 2 * k] = tu[t];
+            s[6 * t + 2 * k + 1] = 0.5f;
+        }
+    __syncthreads();
+    store_run(s_out, uv + 12 * c0, 12u * cells);
+}
+
+// Min and max of a window of the grid, as order-preserving integer images of
+// the floats (negative floats map below every non-negative one, in order;
+// the map is its own inverse on the bit patterns): one pair per workgroup,
+// out[2b] and out[2b + 1], each written once (the caller takes the extremes
+// of the pairs), so there is nothing to set first and no atomic (two atomics
+// per thread on one pair: 98 us for 1024 x 1022 heights; so: 4.3 us).
+constexpr uint32_t kRangeBlocks = 512;
 __device__ __forceinline__ int32_t ordered(float f) {
     const int32_t b = __float_as_int(f);
     return b >= 0 ? b : (int32_t)(0x80000000u - (uint32_t)b - 1u);
 }
-__global__ void k_range(const float* __restrict__ H, uint32_t n1, uint32_t x0, uint32_t y0,
-                        uint32_t w, uint32_t h, int32_t* __restrict__ out) {
+__global__ __launch_bounds__(256) void k_range(const float* __restrict__ H, uint32_t n1,
+                                               uint32_t x0, uint32_t y0, uint32_t w, uint32_t h,
+                                               int32_t* __restrict__ out) {
+    __shared__ int32_t s_lo[4], s_hi[4];
     int32_t lo = INT32_MAX, hi = INT32_MIN;
-    for (uint32_t r = blockIdx.x; r < h; r += gridDim.x)
-        for (uint32_t q = threadIdx.x; q < w; q += blockDim.x) {
-            const int32_t v = ordered(H[(uint64_t)(y0 + r) * n1 + x0 + q]);
+    // a wave takes whole rows, four values of a lane in flight
+    for (uint32_t r = blockIdx.x * 4u + (threadIdx.x >> 6); r < h; r += gridDim.x * 4u) {
+        const float* row = H + (uint64_t)(y0 + r) * n1 + x0;
+#pragma unroll 4
+        for (uint32_t q = threadIdx.x & 63u; q < w; q += 64u) {
+            const int32_t v = ordered(row[q]);
             lo = v < lo ? v : lo;
             hi = v > hi ? v : hi;
         }
-    atomicMin(&out[0], lo);
-    atomicMax(&out[1], hi);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        const int32_t a = __shfl_xor(lo, o), b = __shfl_xor(hi, o);
+        lo = a < lo ? a : lo;
+        hi = b > hi ? b : hi;
+    }
+    if ((threadIdx.x & 63u) == 0u) {
+        s_lo[threadIdx.x >> 6] = lo;
+        s_hi[threadIdx.x >> 6] = hi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < 4; ++k) {
+            lo = s_lo[k] < lo ? s_lo[k] : lo;
+            hi = s_hi[k] > hi ? s_hi[k] : hi;
+        }
+        out[2 * blockIdx.x] = lo;
+        out[2 * blockIdx.x + 1] = hi;
+    }
 }
 float from_ordered(int32_t o) {
     const int32_t b = o >= 0 ? o : (int32_t)(0x80000000u - (uint32_t)o - 1u);
@@ -243,24 +311,33 @@ int vox_terrain_range(const float* heights, uint32_t n1, uint32_t x0, uint32_t y
     if (!heights || !out_minmax || w == 0 || h == 0 || (uint64_t)x0 + w > n1 ||
         (uint64_t)y0 + h > n1)
         return fail("vox_terrain_range: window outside the grid"), 0;
-    // the result words: one pair per calling thread, allocated on its first
-    // call and kept (no hipFree, which would wait for the whole device)
-    thread_local int32_t* d = nullptr;
-    if (!d && !check(hipMalloc(&d, 8), "vox_terrain_range")) return 0;
-    const int32_t init[2] = {INT32_MAX, INT32_MIN};
-    int32_t r[2] = {0, 0};
+    // the workgroups' pairs, in pinned host memory that the kernel writes
+    // itself: one buffer per calling thread, given back when it ends
+    struct Pairs {
+        int32_t* p = nullptr;
+        ~Pairs() {
+            if (p) (void)hipHostFree(p);
+        }
+    };
+    thread_local Pairs pairs;
+    if (!pairs.p && !check(hipHostMalloc(reinterpret_cast<void**>(&pairs.p), 8 * kRangeBlocks,
+                                         hipHostMallocDefault),
+                           "vox_terrain_range"))
+        return 0;
+    const uint32_t blocks = (h + 3u) / 4u < kRangeBlocks ? (h + 3u) / 4u : kRangeBlocks;
     // on the null stream, which the library's non-blocking streams do not
     // wait for and which waits for none of them
-    bool ok = check(hipMemcpyAsync(d, init, 8, hipMemcpyHostToDevice, nullptr), "vox_terrain_range");
-    if (ok) {
-        k_range<<<h < 4096u ? h : 4096u, 256>>>(heights, n1, x0, y0, w, h, d);
-        ok = check(hipGetLastError(), "vox_terrain_range") &&
-             check(hipMemcpyAsync(r, d, 8, hipMemcpyDeviceToHost, nullptr), "vox_terrain_range") &&
-             check(hipStreamSynchronize(nullptr), "vox_terrain_range");
+    k_range<<<blocks, 256>>>(heights, n1, x0, y0, w, h, pairs.p);
+    if (!check(hipGetLastError(), "vox_terrain_range") ||
+        !check(hipStreamSynchronize(nullptr), "vox_terrain_range"))
+        return 0;
+    int32_t lo = INT32_MAX, hi = INT32_MIN;
+    for (uint32_t b = 0; b < blocks; ++b) {
+        lo = std::min(lo, pairs.p[2 * b]);
+        hi = std::max(hi, pairs.p[2 * b + 1]);
     }
-    if (!ok) return 0;
-    out_minmax[0] = from_ordered(r[0]);
-    out_minmax[1] = from_ordered(r[1]);
+    out_minmax[0] = from_ordered(lo);
+    out_minmax[1] = from_ordered(hi);
     return 1;
 }
 
@@ -275,7 +352,7 @@ int vox_terrain_tile(const float* heights, uint32_t n1, double extent, uint32_t 
     const double step = extent / (double)(n1 - 1);
     const float dxf = (float)step;
     const uint64_t n = (uint64_t)cw * ch;
-    k_tile<<<blocks_for(n), 256>>>(heights, n1, step, dxf, x0, y0, cw, ch, (double)hmin,
+    k_tile<<<blocks_for(n), kTileBlock>>>(heights, n1, step, dxf, x0, y0, cw, ch, (double)hmin,
                                    (double)hmax, tex_width, verts, vnormals, uvs);
     // waits for this launch only (the null stream), not for the device
     if (!check(hipGetLastError(), "vox_terrain_tile") ||
