@@ -84,7 +84,7 @@ typedef struct vox_frame_view {
     uint32_t  nrequests;        /* capped at max_requests                    */
     uint32_t  nrequests_total;  /* distinct ids before the cap               */
     double    ms_raycast;       /* HIP-event time of the ray-cast kernel     */
-    double    ms_requests;      /* HIP-event time of the deduplication       */
+    double    ms_requests;      /* 0: the cast lists its requests itself     */
     const float* rgba_f32;      /* device, width*height*4 floats: FragColor  */
 } vox_frame_view;
 

@@ -461,31 +461,92 @@ __device__ __forceinline__ bool cast_pixel(const RayUniforms& U, gu32 __restrict
     return hit;
 }
 
+// A frame's list of distinct requested node ids.
+struct RequestList {
+    uint32_t* stamp;              // node texel -> tag of the frame that listed it
+    uint32_t* list;
+    unsigned long long* times;    // device clock when each was appended
+    uint32_t* counts;             // appended (capped), distinct
+    uint32_t tag, cap;
+};
+
+// Append a wave's node ids of one usage slot to the request list: lanes
+// holding the same id elect one leader (ballot loop), leaders claim the node
+// texel's frame stamp, the claimants' ids are appended with one count per
+// wave.  Every lane of the wave calls it (id 0: none).
+__device__ __forceinline__ void append_requests(const RequestList& R, const uint32_t* ndim,
+                                                uint32_t id) {
+    uint64_t pending = __ballot(id != 0u);
+    if (!pending) return;
+    const int lane = (int)(threadIdx.x & 63u);
+    uint64_t leaders = 0ull;
+    while (pending) {
+        const int l = __ffsll((unsigned long long)pending) - 1;
+        leaders |= 1ull << l;
+        pending &= ~__ballot(id == (uint32_t)__builtin_amdgcn_readlane((int)id, l));
+    }
+    bool claimed = false;
+    if ((leaders >> lane) & 1ull) {
+        const uint32_t x = ((id >> 20) & 1023u) - 1u;
+        const uint32_t y = ((id >> 10) & 1023u) - 1u;
+        const uint32_t z = (id & 1023u) - 1u;
+        if (x < ndim[0] && y < ndim[1] && z < ndim[2]) {
+            const uint32_t t = __umul24(__umul24(z, ndim[1]) + y, ndim[0]) + x;
+            // a plain read first: most leaders meet a node another wave has
+            // claimed already, and skip the atomic on its (hot) stamp word
+            claimed = R.stamp[t] != R.tag && atomicExch(&R.stamp[t], R.tag) != R.tag;
+        }
+    }
+    const uint64_t won = __ballot(claimed);
+    if (!won) return;
+    const int first = __ffsll((unsigned long long)won) - 1;
+    uint32_t base = 0u;
+    if (lane == first) base = atomicAdd(&R.counts[1], (uint32_t)__popcll(won));
+    base = (uint32_t)__builtin_amdgcn_readlane((int)base, first);
+    const uint32_t k = base + (uint32_t)__popcll(won & ((1ull << lane) - 1ull));
+    const bool put = claimed && k < R.cap;
+    if (put) {
+        R.list[k] = id;
+        R.times[k] = (unsigned long long)wall_clock64();  // emitted
+    }
+    const uint64_t kept = __ballot(put);
+    if (kept && lane == first) atomicAdd(&R.counts[0], (uint32_t)__popcll(kept));
+}
+
+// One octree's frame, one thread per pixel, 16 x 4 pixels a wave; the wave
+// that has cast its pixels lists their distinct node ids itself (the same
+// pass over the usage lists in a kernel of its own read 100 MB back at
+// 1080p and met few equal ids per wave: 154 us beside a cast of 0.91 ms).
 __global__ void __launch_bounds__(256)
 k_raycast(RayUniforms U, const uint32_t* __restrict__ tex, const uint32_t* __restrict__ pool,
           const float* __restrict__ jitter, uint32_t* __restrict__ rgbaOut,
-          float4* __restrict__ rgbaF, uint32_t* __restrict__ usageOut) {
+          float4* __restrict__ rgbaF, uint32_t* __restrict__ usageOut, RequestList R) {
     const int i = U.rx0 + (int)blockIdx.x * 16 + (int)(threadIdx.x & 15);
     const int j = U.ry0 + (int)blockIdx.y * 16 + (int)(threadIdx.x >> 4);
-    if (i >= U.rx1 || j >= U.ry1) return;
     uint32_t usage[kMaxUsage];
-    float dst[4];
-    cast_pixel(U, (gu32)tex, (gu32)pool, jitter, i, j, dst, usage);
-    const uint64_t pix = (uint64_t)j * U.W + i;
-    if (rgbaOut) {
+    if (i < U.rx1 && j < U.ry1) {
+        float dst[4];
+        cast_pixel(U, (gu32)tex, (gu32)pool, jitter, i, j, dst, usage);
+        const uint64_t pix = (uint64_t)j * U.W + i;
         uint32_t o = 0;
+#pragma unroll
         for (int c = 0; c < 4; ++c) {
             float v = dst[c] * 255.0f;
             v = v > 255.0f ? 255.0f : (v > 0.0f ? v : 0.0f);
             o |= (uint32_t)v << (8 * c);
         }
         rgbaOut[pix] = o;
+        rgbaF[pix] = make_float4(dst[0], dst[1], dst[2], dst[3]);  // FragColor
+        uint4* u4 = reinterpret_cast<uint4*>(usageOut + pix * kMaxUsage);
+        u4[0] = make_uint4(usage[0], usage[1], usage[2], usage[3]);
+        u4[1] = make_uint4(usage[4], usage[5], usage[6], usage[7]);
+        u4[2] = make_uint4(usage[8], usage[9], usage[10], usage[11]);
+    } else {
+#pragma unroll
+        for (int q = 0; q < kMaxUsage; ++q) usage[q] = 0u;
     }
-    if (rgbaF) rgbaF[pix] = make_float4(dst[0], dst[1], dst[2], dst[3]);  // FragColor
-    uint4* u4 = reinterpret_cast<uint4*>(usageOut + pix * kMaxUsage);
-    u4[0] = make_uint4(usage[0], usage[1], usage[2], usage[3]);
-    u4[1] = make_uint4(usage[4], usage[5], usage[6], usage[7]);
-    u4[2] = make_uint4(usage[8], usage[9], usage[10], usage[11]);
+#pragma unroll
+    for (int q = 0; q < kMaxUsage; ++q) append_requests(R, U.ndim, usage[q]);
 }
 
 // One octree of a front-to-back frame over several octrees: its uniforms
@@ -494,42 +555,8 @@ struct TreeCast {
     RayUniforms U;
     const uint32_t* tex;
     const uint32_t* pool;
-    uint32_t* stamp;              // node texel -> tag of the frame that listed it
-    uint32_t* list;
-    unsigned long long* times;
-    uint32_t* counts;             // appended (capped), distinct
-    uint32_t tag, cap;
+    RequestList R;
 };
-
-// Append a wave's node ids of one usage slot to the octree's request list:
-// lanes holding the same id elect one leader (ballot loop), leaders claim
-// the node texel's frame stamp, the first claimant appends the id.
-__device__ __forceinline__ void append_requests(const TreeCast& tc, uint32_t id) {
-    uint64_t pending = __ballot(id != 0u);
-    bool leader = false;
-    while (pending) {
-        const int l = __ffsll((unsigned long long)pending) - 1;
-        const uint32_t lid = __shfl(id, l);
-        const uint64_t same = __ballot(id == lid);
-        if ((int)(threadIdx.x & 63) == l) leader = true;
-        pending &= ~same;
-    }
-    if (!leader) return;
-    const uint32_t x = ((id >> 20) & 1023u) - 1u;
-    const uint32_t y = ((id >> 10) & 1023u) - 1u;
-    const uint32_t z = (id & 1023u) - 1u;
-    const uint32_t* nd = tc.U.ndim;
-    if (x >= nd[0] || y >= nd[1] || z >= nd[2]) return;
-    const uint64_t t = ((uint64_t)z * nd[1] + y) * nd[0] + x;
-    if (tc.stamp[t] != tc.tag && atomicExch(&tc.stamp[t], tc.tag) != tc.tag) {
-        const uint32_t k = atomicAdd(&tc.counts[1], 1u);
-        if (k < tc.cap) {
-            tc.list[k] = id;
-            tc.times[k] = (unsigned long long)wall_clock64();  // emitted
-            atomicAdd(&tc.counts[0], 1u);
-        }
-    }
-}
 
 // Front to back over n octrees listed in an order every ray meets them in
 // (boxes that tile space; the caller's order): each pixel casts its ray
@@ -583,66 +610,11 @@ k_raycast_multi(const TreeCast* __restrict__ trees, uint32_t n, const float* __r
             T = T * (1.0f - a);
         }
 #pragma unroll
-        for (int q = 0; q < kMaxUsage; ++q) append_requests(tc, usage[q]);
+        for (int q = 0; q < kMaxUsage; ++q) append_requests(tc.R, U.ndim, usage[q]);
     }
     if (in) {
         frame[pix] = make_float4(acc[0], acc[1], acc[2], acc[3]);
         if (trans) trans[pix] = T;
-    }
-}
-
-
-// Distinct node ids of the frame's pixel rectangle: lanes of a wave
-// holding the same id elect one leader (ballot loop), leaders claim the node
-// texel's frame stamp, the first claimant appends the id.  counts[0] =
-// appended (capped), counts[1] = distinct ids.  Entry e of the rectangle is
-// list slot e % 12 of its pixel e / 12 (row by row).
-__global__ void __launch_bounds__(256)
-k_requests(const uint32_t* __restrict__ usage, uint32_t W, int32_t rx0, int32_t ry0, uint32_t rw,
-           uint64_t n, uint32_t tag, uint32_t ndx, uint32_t ndy, uint32_t ndz,
-           uint32_t* __restrict__ stamp, uint32_t* __restrict__ list,
-           unsigned long long* __restrict__ times, uint32_t cap,
-           uint32_t* __restrict__ counts) {
-    for (uint64_t base = (uint64_t)blockIdx.x * blockDim.x; base < n;
-         base += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t e = base + threadIdx.x;
-        uint32_t id = 0u;
-        if (e < n) {
-            // n < 2^32 (checked at launch): 32-bit index arithmetic
-            const uint32_t e32 = (uint32_t)e;
-            const uint32_t p = e32 / (uint32_t)kMaxUsage;
-            const uint32_t k = e32 - p * (uint32_t)kMaxUsage;
-            const uint32_t prow = p / rw;
-            const uint64_t px = (uint64_t)rx0 + (p - prow * rw), py = (uint64_t)ry0 + prow;
-            id = usage[(py * W + px) * kMaxUsage + k];
-        }
-        // wave-level deduplication
-        uint64_t pending = __ballot(id != 0u);
-        bool leader = false;
-        while (pending) {
-            const int l = __ffsll((unsigned long long)pending) - 1;
-            const uint32_t lid = __shfl(id, l);
-            const uint64_t same = __ballot(id == lid);
-            if ((int)(threadIdx.x & 63) == l) leader = true;
-            pending &= ~same;
-        }
-        if (leader) {
-            const uint32_t x = ((id >> 20) & 1023u) - 1u;
-            const uint32_t y = ((id >> 10) & 1023u) - 1u;
-            const uint32_t z = (id & 1023u) - 1u;
-            const uint64_t t = ((uint64_t)z * ndy + y) * ndx + x;
-            // a plain read first: most leaders meet a node another wave has
-            // claimed already, and skip the atomic on its (hot) stamp word
-            if (x < ndx && y < ndy && z < ndz && stamp[t] != tag &&
-                atomicExch(&stamp[t], tag) != tag) {
-                const uint32_t k = atomicAdd(&counts[1], 1u);
-                if (k < cap) {
-                    list[k] = id;
-                    times[k] = (unsigned long long)wall_clock64();  // emitted
-                    atomicAdd(&counts[0], 1u);
-                }
-            }
-        }
     }
 }
 
@@ -971,20 +943,17 @@ int vox_raycast_frame(vox_raycaster* rc, const vox_camera* cam, const vox_raycas
     launch_fill_u32(st, rc->counts.as<uint32_t>(), 2, 0u);
     (void)hipEventRecord(rc->ev[0], st);
     dim3 grid((rw + 15) / 16, (rh + 15) / 16);
+    const RequestList R{rc->stamp.as<uint32_t>(), rc->req.as<uint32_t>(),
+                        rc->reqTime.as<unsigned long long>(), rc->counts.as<uint32_t>(), rc->tag,
+                        rc->maxReq};
     k_raycast<<<grid, 256, 0, st>>>(U, tex, o.poolCol, rc->jitter.as<float>(), rc->rgba.as<uint32_t>(),
-                                    rc->rgbaF.as<float4>(), rc->usage.as<uint32_t>());
+                                    rc->rgbaF.as<float4>(), rc->usage.as<uint32_t>(), R);
     rc->rect[0] = U.rx0;
     rc->rect[1] = U.ry0;
     rc->rect[2] = U.rx1;
     rc->rect[3] = U.ry1;
+    // the requests are listed by the cast itself: no time of their own
     (void)hipEventRecord(rc->ev[1], st);
-    const uint64_t nent = npix * kMaxUsage;
-    const unsigned rgrid = (unsigned)std::min<uint64_t>((nent + 255) / 256, 8192);
-    k_requests<<<rgrid, 256, 0, st>>>(rc->usage.as<uint32_t>(), (uint32_t)rc->W, U.rx0, U.ry0, rw,
-                                      nent, rc->tag, nd[0], nd[1],
-                                      nd[2], rc->stamp.as<uint32_t>(), rc->req.as<uint32_t>(),
-                                      rc->reqTime.as<unsigned long long>(), rc->maxReq,
-                                      rc->counts.as<uint32_t>());
     (void)hipEventRecord(rc->ev[2], st);
     if (!rc->check(hipGetLastError(), "raycast kernels") ||
         !rc->check(hipEventRecord(rc->done, st), "event record"))
@@ -1039,12 +1008,9 @@ int vox_raycast_frame_multi(vox_raycaster* const* rcs, uint32_t n, const vox_cam
         launch_fill_u32(st, rc->counts.as<uint32_t>(), 2, 0u);
         tc.tex = o.tex;
         tc.pool = o.poolCol;
-        tc.stamp = rc->stamp.as<uint32_t>();
-        tc.list = rc->req.as<uint32_t>();
-        tc.times = rc->reqTime.as<unsigned long long>();
-        tc.counts = rc->counts.as<uint32_t>();
-        tc.tag = rc->tag;
-        tc.cap = rc->maxReq;
+        tc.R = RequestList{rc->stamp.as<uint32_t>(), rc->req.as<uint32_t>(),
+                           rc->reqTime.as<unsigned long long>(), rc->counts.as<uint32_t>(),
+                           rc->tag, rc->maxReq};
         rc->W = cam->width;
         rc->H = cam->height;
         rc->rect[0] = tc.U.rx0;
