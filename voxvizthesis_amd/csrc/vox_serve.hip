@@ -513,16 +513,21 @@ __device__ __forceinline__ void append_requests(const RequestList& R, const uint
     if (kept && lane == first) atomicAdd(&R.counts[0], (uint32_t)__popcll(kept));
 }
 
-// One octree's frame, one thread per pixel, 16 x 4 pixels a wave; the wave
+// One octree's frame, one thread per pixel, 16 x 4 pixels a wave and a wave
+// per workgroup, so that a wave's place is free again when its own rays end
+// (four waves a workgroup: 1.11 ms where this takes 1.05; 8 x 8 pixels:
+// 1.06; neighbouring workgroups on one XCD: 1.4 to 1.5, as the rays of one
+// part of the image are longer than another's); the wave
 // that has cast its pixels lists their distinct node ids itself (the same
 // pass over the usage lists in a kernel of its own read 100 MB back at
 // 1080p and met few equal ids per wave: 154 us beside a cast of 0.91 ms).
-__global__ void __launch_bounds__(256)
+constexpr int kCastW = 16, kCastH = 4;   // pixels of a wave
+__global__ void __launch_bounds__(kCastW * kCastH)
 k_raycast(RayUniforms U, const uint32_t* __restrict__ tex, const uint32_t* __restrict__ pool,
           const float* __restrict__ jitter, uint32_t* __restrict__ rgbaOut,
           float4* __restrict__ rgbaF, uint32_t* __restrict__ usageOut, RequestList R) {
-    const int i = U.rx0 + (int)blockIdx.x * 16 + (int)(threadIdx.x & 15);
-    const int j = U.ry0 + (int)blockIdx.y * 16 + (int)(threadIdx.x >> 4);
+    const int i = U.rx0 + (int)blockIdx.x * kCastW + (int)(threadIdx.x % kCastW);
+    const int j = U.ry0 + (int)blockIdx.y * kCastH + (int)(threadIdx.x / kCastW);
     uint32_t usage[kMaxUsage];
     if (i < U.rx1 && j < U.ry1) {
         float dst[4];
@@ -570,13 +575,13 @@ struct TreeCast {
 // requests for it.  With resume the pass continues a frame: acc from frame,
 // T from trans (a pass over the octrees in front wrote both); trans, when
 // given, receives each pixel's T for the next pass.
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kCastW * kCastH)
 k_raycast_multi(const TreeCast* __restrict__ trees, uint32_t n, const float* __restrict__ jitter,
                 int32_t W, int32_t x0, int32_t y0, int32_t x1, int32_t y1, float tStop,
                 float4* __restrict__ frame, float* __restrict__ trans, int resume) {
     // pixels of the union of the octrees' rectangles, [x0, x1) x [y0, y1)
-    const int i = x0 + (int)blockIdx.x * 16 + (int)(threadIdx.x & 15);
-    const int j = y0 + (int)blockIdx.y * 16 + (int)(threadIdx.x >> 4);
+    const int i = x0 + (int)blockIdx.x * kCastW + (int)(threadIdx.x % kCastW);
+    const int j = y0 + (int)blockIdx.y * kCastH + (int)(threadIdx.x / kCastW);
     const bool in = i < x1 && j < y1;
     const uint64_t pix = (uint64_t)j * W + i;
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -942,11 +947,11 @@ int vox_raycast_frame(vox_raycaster* rc, const vox_camera* cam, const vox_raycas
     }
     launch_fill_u32(st, rc->counts.as<uint32_t>(), 2, 0u);
     (void)hipEventRecord(rc->ev[0], st);
-    dim3 grid((rw + 15) / 16, (rh + 15) / 16);
+    dim3 grid((rw + kCastW - 1) / kCastW, (rh + kCastH - 1) / kCastH);
     const RequestList R{rc->stamp.as<uint32_t>(), rc->req.as<uint32_t>(),
                         rc->reqTime.as<unsigned long long>(), rc->counts.as<uint32_t>(), rc->tag,
                         rc->maxReq};
-    k_raycast<<<grid, 256, 0, st>>>(U, tex, o.poolCol, rc->jitter.as<float>(), rc->rgba.as<uint32_t>(),
+    k_raycast<<<grid, kCastW * kCastH, 0, st>>>(U, tex, o.poolCol, rc->jitter.as<float>(), rc->rgba.as<uint32_t>(),
                                     rc->rgbaF.as<float4>(), rc->usage.as<uint32_t>(), R);
     rc->rect[0] = U.rx0;
     rc->rect[1] = U.ry0;
@@ -1067,8 +1072,9 @@ int vox_raycast_frame_multi(vox_raycaster* const* rcs, uint32_t n, const vox_cam
         !r0->check(hipEventRecord(r0->tableCopied[b], st), "event record"))
         return 0;
     (void)hipEventRecord(r0->ev[0], st);
-    dim3 grid((unsigned)(ux1 - ux0 + 15) / 16, (unsigned)(uy1 - uy0 + 15) / 16);
-    k_raycast_multi<<<grid, 256, 0, st>>>(r0->multiTable.as<TreeCast>(), n, r0->jitter.as<float>(),
+    dim3 grid((unsigned)(ux1 - ux0 + kCastW - 1) / kCastW,
+              (unsigned)(uy1 - uy0 + kCastH - 1) / kCastH);
+    k_raycast_multi<<<grid, kCastW * kCastH, 0, st>>>(r0->multiTable.as<TreeCast>(), n, r0->jitter.as<float>(),
                                           cam->width, ux0, uy0, ux1, uy1, t_stop,
                                           reinterpret_cast<float4*>(frame), transmittance,
                                           resume ? 1 : 0);
