@@ -2,15 +2,19 @@
 
 The device decides a node's level-of-detail test from a range of voxel half
 sizes (lod_range) and a node's step count from products with reciprocals
-(exit_steps) wherever rounding cannot change the outcome, and takes c / 255
-from a fused product.  Restated here in fp32 and compared with the stated
+(exit_steps) wherever rounding cannot change the outcome, and takes c / 255,
+quotients by the pool's sides and the trilinear weights from products.  Restated here in fp32 and compared with the stated
 arithmetic on drawn rays."""
+import ctypes
 import math
 
 import numpy as np
 import pytest
 
 f = np.float32
+LIBM = ctypes.CDLL("libm.so.6")
+LIBM.fmaf.restype = ctypes.c_float
+LIBM.fmaf.argtypes = [ctypes.c_float] * 3
 U24 = 2.0 ** -24
 
 
@@ -110,9 +114,34 @@ def test_exit_steps_equal_the_divided_ones(levels):
             assert sure[n // 4:].mean() > 0.74
 
 
+def fma(a, b, c):
+    """Fused multiply-add in fp32 of scalars (the C library's)."""
+    return LIBM.fmaf(float(a), float(b), float(c))
+
+
 def test_unorm8_is_the_rounded_quotient():
-    c = np.arange(256)
-    k = float.fromhex("0x1.010102p-16")
-    # the product and the sum are exact in float64, which rounds once
-    got = (c * k + c * 2.0 ** -8).astype(f)
-    assert (got == (c.astype(f) / f(255))).all()
+    k = float.fromhex("0x1.010102p-8")
+    for c in range(256):
+        assert f(fma(c, k, c)) == f(256) * (f(c) / f(255))
+
+
+# brick texels per axis of wide pools (B + 2) and of texture pools
+@pytest.mark.parametrize("b", [3, 6, 9, 18, 34, 66, 100, 144, 288, 720, 1023, 1024])
+def test_div_by_is_the_rounded_quotient(b):
+    rng = np.random.default_rng(b)
+    r = f(1) / f(b)
+    a = np.concatenate([rng.random(4000) * 16, np.exp2(rng.uniform(-80, 10, 4000)),
+                        np.arange(1024)]).astype(f)
+    for x in a:
+        q = x * r
+        assert f(fma(fma(-q, b, x), r, q)) == x / f(b)
+
+
+def test_weight_products_are_exact():
+    w = np.arange(257)
+    rng = np.random.default_rng(1)
+    x, y, z = (rng.choice(w, 20000) for _ in range(3))
+    want = ((x / 256).astype(f) * (y / 256).astype(f)) * (z / 256).astype(f)
+    got = (x.astype(f) * y.astype(f)) * (z.astype(f) * f(2.0 ** -32))
+    assert (got * f(256) == want).all()
+    assert (want.astype(np.float64) == x * y * z / 2.0 ** 24).all()

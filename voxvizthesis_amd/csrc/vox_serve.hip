@@ -163,17 +163,18 @@ __device__ __forceinline__ void lod_range(const RayUniforms& U, v3 p, v3 cam, fl
     }
 }
 
-// c / 255 for a channel c = 0 .. 255: the correctly rounded quotient, from
-// one fused product (all 256 compared with the division; c / 256 is exact).
-__device__ __forceinline__ float unorm8(uint32_t c) {
+// 256 (c / 255) for a channel c = 0 .. 255, c / 255 the correctly rounded
+// quotient: one fused product (all 256 compared with the division; the scale
+// changes no rounding).
+__device__ __forceinline__ float unorm8_256(uint32_t c) {
     const float f = (float)c;
-    return __builtin_fmaf(f, 0x1.010102p-16f, f * 0x1p-8f);
+    return __builtin_fmaf(f, 0x1.010102p-8f, f);
 }
 __device__ __forceinline__ void unpack_rgba(uint32_t c, float o[4]) {
-    o[0] = unorm8(c & 255u);
-    o[1] = unorm8((c >> 8) & 255u);
-    o[2] = unorm8((c >> 16) & 255u);
-    o[3] = unorm8(c >> 24);
+    o[0] = unorm8_256(c & 255u) * 0x1p-8f;
+    o[1] = unorm8_256((c >> 8) & 255u) * 0x1p-8f;
+    o[2] = unorm8_256((c >> 16) & 255u) * 0x1p-8f;
+    o[3] = unorm8_256(c >> 24) * 0x1p-8f;
 }
 
 // texture(BrickSampler, s): trilinear, clamp to edge.  unorm8 channel c
@@ -194,32 +195,37 @@ struct pair32 {
 } __attribute__((packed, aligned(4)));
 typedef const __attribute__((address_space(1))) pair32* gpair;
 
-// Loads of one sample: eight texels t in corner order and the weights w.
+// Loads of one sample: eight texels t in corner order and the weights w,
+// whole 256ths.
+// Coordinates are clamped as floats (the texel numbers are whole and below
+// 2^24); a pool has at most 1024 texels per axis, so indices are 24-bit
+// products.  (No coordinate is NaN: a ray that is cast has a direction of
+// numbers, and a volume so small that its brick step would not be one has
+// none, its rays' directions overflowing before.)
 __device__ __forceinline__ void load_sample(gu32 __restrict__ col, const RayUniforms& U, v3 s,
                                             uint32_t (&t)[8], float (&w)[3]) {
     const float c[3] = {s.x, s.y, s.z};
-    int i0[3];
+    float f[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        float u = c[a];
-        if (!(u == u)) u = 0.0f;
-        const float b = u * U.poolDim[a] - 0.5f;
-        const float f = floorf(b);
-        w[a] = rintf((b - f) * 256.0f) * 0x1p-8f;
-        i0[a] = (int)fmaxf(fminf(f, 1.0e9f), -1.0e9f);
+        const float b = c[a] * U.poolDim[a] - 0.5f;
+        f[a] = floorf(b);
+        w[a] = rintf((b - f[a]) * 256.0f);
     }
-    const int dx = (int)U.pdim[0], dy = (int)U.pdim[1], dz = (int)U.pdim[2];
-    const int xp = max(min(i0[0], dx - 2), 0);   // (a pool has B + 2 >= 3 texels per axis)
-    const bool left = i0[0] < 0, right = i0[0] > dx - 2;
-    const int y0 = max(min(i0[1], dy - 1), 0), y1 = max(min(i0[1] + 1, dy - 1), 0);
-    const int z0 = max(min(i0[2], dz - 1), 0), z1 = max(min(i0[2] + 1, dz - 1), 0);
-    const uint32_t r0 = (uint32_t)z0 * U.pdim[1], r1 = (uint32_t)z1 * U.pdim[1];
-    const uint32_t row[4] = {(r0 + (uint32_t)y0) * U.pdim[0], (r0 + (uint32_t)y1) * U.pdim[0],
-                             (r1 + (uint32_t)y0) * U.pdim[0], (r1 + (uint32_t)y1) * U.pdim[0]};
+    const float mx = U.poolDim[0] - 2.0f, my = U.poolDim[1] - 1.0f, mz = U.poolDim[2] - 1.0f;
+    const bool left = f[0] < 0.0f, right = f[0] > mx;   // (a pool has B + 2 >= 3 texels per axis)
+    const uint32_t x = (uint32_t)__builtin_amdgcn_fmed3f(f[0], 0.0f, mx);
+    const float y0 = __builtin_amdgcn_fmed3f(f[1], 0.0f, my);
+    const float z0 = __builtin_amdgcn_fmed3f(f[2], 0.0f, mz);
+    const uint32_t o = __umul24(__umul24((uint32_t)z0, U.pdim[1]) + (uint32_t)y0, U.pdim[0]) + x;
+    // the next row and slice where they lie inside the edge, else the same
+    const uint32_t oy = f[1] >= 0.0f && f[1] < my ? U.pdim[0] : 0u;
+    const uint32_t oz = f[2] >= 0.0f && f[2] < mz ? U.pdim[0] * U.pdim[1] : 0u;
+    const uint32_t at[4] = {o, o + oy, o + oz, o + oy + oz};
     pair32 q[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        gpair g = (gpair)(col + (row[k] + (uint32_t)xp));
+        gpair g = (gpair)(col + at[k]);
         q[k].a = g->a;
         q[k].b = g->b;
     }
@@ -230,22 +236,36 @@ __device__ __forceinline__ void load_sample(gu32 __restrict__ col, const RayUnif
     }
 }
 
+// a / b for a whole b below 2^23 whose rounded reciprocal r is at hand: the
+// product a r is within one unit in the last place of the quotient, and one
+// fused remainder step then rounds it correctly (Markstein 1990; b's
+// significand is not all ones).  A numerator so small that the remainder
+// would be subnormal is divided out.
+__device__ __forceinline__ float div_by(float a, float b, float r) {
+    if (fabsf(a) < 0x1p-80f && a != 0.0f) return a / b;
+    const float q = a * r;
+    return __builtin_fmaf(__builtin_fmaf(-q, b, a), r, q);
+}
+__device__ __forceinline__ v3 div_pool(const RayUniforms& U, v3 a) {
+    return {div_by(a.x, U.poolDim[0], U.firstTexel[0]), div_by(a.y, U.poolDim[1], U.firstTexel[1]),
+            div_by(a.z, U.poolDim[2], U.firstTexel[2])};
+}
+
+// The products of three weights are whole 2^24ths (at most 24 bits) and so
+// exact in any order; the channels' scale of 256 is taken out with theirs.
 __device__ __forceinline__ void weigh_sample(const uint32_t (&t)[8], const float (&w)[3],
                                              float r[4]) {
-    r[0] = r[1] = r[2] = r[3] = 0.0f;
+    const float z[2] = {(256.0f - w[2]) * 0x1p-32f, w[2] * 0x1p-32f};
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-        const int dx = k & 1, dy = (k >> 1) & 1, dz = k >> 2;
-        const float wx = dx ? w[0] : 1.0f - w[0];
-        const float wy = dy ? w[1] : 1.0f - w[1];
-        const float wz = dz ? w[2] : 1.0f - w[2];
-        const float wk = (wx * wy) * wz;
-        float c[4];
-        unpack_rgba(t[k], c);
-        r[0] = r[0] + wk * c[0];
-        r[1] = r[1] + wk * c[1];
-        r[2] = r[2] + wk * c[2];
-        r[3] = r[3] + wk * c[3];
+        const float wx = (k & 1) ? w[0] : 256.0f - w[0];
+        const float wy = ((k >> 1) & 1) ? w[1] : 256.0f - w[1];
+        const float wk = (wx * wy) * z[k >> 2];
+        const uint32_t v = t[k];
+        const float c[4] = {wk * unorm8_256(v & 255u), wk * unorm8_256((v >> 8) & 255u),
+                            wk * unorm8_256((v >> 16) & 255u), wk * unorm8_256(v >> 24)};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = k == 0 ? c[i] : r[i] + c[i];
     }
 }
 
@@ -412,16 +432,16 @@ __device__ __forceinline__ bool cast_pixel(const RayUniforms& U, gu32 __restrict
                     // pool's normalised coordinates or, in a wide pool, the brick's
                     const v3 bp = U.wide
                         ? ld3(U.firstTexel)
-                        : mk((float)((curBrickPtr.y >> 20) & 1023u) / U.poolDim[0],
-                             (float)((curBrickPtr.y >> 10) & 1023u) / U.poolDim[1],
-                             (float)(curBrickPtr.y & 1023u) / U.poolDim[2]);
+                        : div_pool(U, mk((float)((curBrickPtr.y >> 20) & 1023u),
+                                         (float)((curBrickPtr.y >> 10) & 1023u),
+                                         (float)(curBrickPtr.y & 1023u)));
                     // (a path with no resident brick keeps the root's word 1,
                     // which need not be a slot: slot 0 is read then, where the
                     // reference reads whatever texel those bits name)
                     const uint32_t slot = curBrickPtr.y < U.wideSlots ? curBrickPtr.y : 0u;
                     gu32 bpool =
                         U.wide ? pool + (uint64_t)slot * (U.pdim[0] * U.pdim[1] * U.pdim[2]) : pool;
-                    v3 cbr = add(bp, divv(mul(curBrickRayPos, ld3(U.brickDim)), ld3(U.poolDim)));
+                    v3 cbr = add(bp, div_pool(U, mul(curBrickRayPos, ld3(U.brickDim))));
                     const v3 ws = muls(muls(rayDir, U.rayStep), ratio);
                     for (int s = 0; s < ns; ++s) {
                         rayPos = add(rayPos, ws);
