@@ -63,6 +63,39 @@ void block_flush() {
 
 namespace {
 
+// Pinned words of a handle (kPinWords), kept for the next handle when one is
+// destroyed (allocating them takes 70 us): at most kPinKept, the rest freed.
+constexpr size_t kPinWords = 256, kPinKept = 64;
+std::mutex g_pinMu;
+std::vector<uint32_t*> g_pins;
+uint32_t* pin_take() {
+    {
+        std::lock_guard<std::mutex> lk(g_pinMu);
+        if (!g_pins.empty()) {
+            uint32_t* p = g_pins.back();
+            g_pins.pop_back();
+            return p;
+        }
+    }
+    void* p = nullptr;
+    if (hipHostMalloc(&p, kPinWords * 4, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return static_cast<uint32_t*>(p);
+}
+void pin_give(uint32_t* p) {
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lk(g_pinMu);
+        if (g_pins.size() < kPinKept) {
+            g_pins.push_back(p);
+            return;
+        }
+    }
+    (void)hipHostFree(p);
+}
+
 struct HostGroup {
     vox_group desc;
     bool device = false;
@@ -75,7 +108,7 @@ struct LevelBufs {
     LevelMap map{};
     uint64_t active = 0;
     int aliasOf = -1;     // level whose tiles hold this level's voxels
-    DevBuf mark, excl, tileIdx, list, col, qn, nrm;
+    DevBuf tileIdx, list, col, qn, nrm;
 };
 
 // A level as the kernels see it.  In the reference's mip recursion level
@@ -167,6 +200,9 @@ struct vox_ctx {
     std::vector<DepthBufs> tree;
     DevBuf bitmap;
     DevBuf counters;  // small host-read counters
+    // Pinned words the kernels leave their counts in for the host (kPin*).
+    uint32_t* pin = nullptr;
+    std::vector<int32_t> fillFlags;   // what grpFill holds
     vox_stats stats{};
     std::vector<TimedLaunch> timed;
     std::vector<hipEvent_t> eventPool;
@@ -247,9 +283,13 @@ inline uint64_t trunc_u(float f) {
     return (uint64_t)f;
 }
 
-// Word of h->counters where the scans of a generate report a wait that
-// timed out (zeroed by the setup pass, read at the generate's last sync).
-constexpr uint32_t kScanErrWord = 128;
+// Words of h->counters, zeroed together by the setup pass: active tiles per
+// level (first), with several chunks the bricks per depth, where the scans of a generate report a wait
+// that timed out, and the collapse's ticket.
+constexpr uint32_t kChunkBricksWord = 64, kScanErrWord = 128, kCollapseWord = 129,
+                   kCounterWords = 160;
+// Words of h->pin: what launch_map_counts and launch_generate_counts leave.
+constexpr uint32_t kPinTiles = 0, kPinCounts = 32;
 
 bool scan(vox_ctx* h, const uint32_t* in, uint32_t* out, uint64_t n) {
     if (!ensure_scan_tmp(h->scanTmp, n, h->st, h->err, "scan scratch")) return false;
@@ -414,6 +454,7 @@ void vox_destroy(vox_ctx* h) {
     if (h->evJoin) (void)hipEventDestroy(h->evJoin);
     if (h->side) (void)hipStreamDestroy(h->side);
     if (h->st) (void)hipStreamDestroy(h->st);
+    pin_give(h->pin);   // the handle's streams are idle
     delete h;
 }
 
@@ -473,6 +514,7 @@ int vox_init(vox_ctx* h) {
         !h->check(hipEventCreateWithFlags(&h->evFork, hipEventDisableTiming), "hipEventCreate") ||
         !h->check(hipEventCreateWithFlags(&h->evJoin, hipEventDisableTiming), "hipEventCreate"))
         return 0;
+    if (!h->pin && !(h->pin = pin_take())) return h->fail("no pinned memory for counters"), 0;
     (void)hipEventCreate(&h->evStart);
     (void)hipEventCreate(&h->evStop);
     int cus = 0;
@@ -493,6 +535,7 @@ int vox_allocate_voxel_memory(vox_ctx* h) {
         P.TG[a] = (h->S[a] + kTile - 1) / kTile;
         P.C[a] = h->C[a];
     }
+    for (int a = 0; a < 2; ++a) P.invTG[a] = 1.0 / P.TG[a];
     P.numTiles = (uint64_t)P.TG[0] * P.TG[1] * P.TG[2];
     h->lv.assign(h->L, LevelBufs());
     for (int k = 0; k < h->L; ++k) {
@@ -503,11 +546,11 @@ int vox_allocate_voxel_memory(vox_ctx* h) {
             l.map.dims[a] = k == 0 ? h->S[a] : h->nc[a] * (h->C[a] >> k);
             l.map.TG[a] = (l.map.dims[a] + kTile - 1) / kTile;
         }
+        // (a level of no tiles on an axis is never divided by)
+        for (int a = 0; a < 2; ++a) l.map.invTG[a] = l.map.TG[a] ? 1.0 / l.map.TG[a] : 0.0;
         l.map.numTiles = (uint64_t)l.map.TG[0] * l.map.TG[1] * l.map.TG[2];
         uint64_t nt = l.map.numTiles;
-        if (!l.mark.ensure(nt * 4, h->err, "tile marks") ||
-            !l.excl.ensure((nt + 1) * 4, h->err, "tile scan") ||
-            !l.tileIdx.ensure(nt * 4, h->err, "tile map") ||
+        if (!l.tileIdx.ensure(nt * 4, h->err, "tile map") ||
             !l.list.ensure(nt * 4, h->err, "tile list"))
             return 0;
         l.map.tileIdx = l.tileIdx.as<int32_t>();
@@ -577,13 +620,14 @@ void vox_deallocate_voxel_memory(vox_ctx* h) {
     if (!h || !idle(h)) return;
     if (h->st) (void)hipStreamSynchronize(h->st);
     for (auto& l : h->lv) {
-        l.mark.release(); l.excl.release(); l.tileIdx.release(); l.list.release();
+        l.tileIdx.release(); l.list.release();
         l.col.release(); l.qn.release(); l.nrm.release();
     }
     h->lv.clear();
     for (auto& t : h->tree) {
         t.types.release(); t.cc.release(); t.bidx.release();
         t.brickNode.release(); t.bcol.release(); t.bnrm.release();
+        t.ccol.release(); t.cnrm.release();
     }
     h->tree.clear();
     h->nodeFlag.release(); h->nodeExcl.release();
@@ -618,6 +662,7 @@ int vox_allocate_triangle_memory(vox_ctx* h) {
         !h->img.ensure(nimg, h->err, "images") ||
         !h->grpFill.ensure(h->groups.size() * 4 + 4, h->err, "group flags"))
         return 0;
+    h->fillFlags.clear();
     // Concatenate groups (allocateTriangleMemory, Voxelizer.cu 346-457).
     uint64_t to = 0, vo = 0, uo = 0, io = 0;
     h->gargs.clear();
@@ -707,6 +752,7 @@ void vox_deallocate_triangle_memory(vox_ctx* h) {
     if (h->st) (void)hipStreamSynchronize(h->st);
     h->verts.release(); h->fnorm.release(); h->bbox.release(); h->vn.release(); h->gbounds.release();
     h->uv.release(); h->img.release(); h->grpFill.release();
+    h->fillFlags.clear();
     h->groups.clear();
     h->gargs.clear();
     h->T = 0;
@@ -759,10 +805,14 @@ int vox_compute_edges_face_normals_and_bounds(vox_ctx* h) {
         fill[g] = (ga.overlaps && ga.textured && ga.terrain) ? 1 : 0;
     }
     // (replay: the flags are already on the device from the eager pass)
-    if (!h->replay &&
-        !h->check(hipMemcpyAsync(h->grpFill.p, fill.data(), 4 * (G + 1), hipMemcpyHostToDevice, h->st),
-                  "group flags"))
-        return 0;
+    if (!h->replay && fill != h->fillFlags) {
+        if (!h->check(hipMemcpyAsync(h->grpFill.p, fill.data(), 4 * (G + 1), hipMemcpyHostToDevice,
+                                     h->st),
+                      "group flags") ||
+            !h->check(hipStreamSynchronize(h->st), "group flags"))
+            return 0;
+        h->fillFlags = fill;
+    }
     h->numBins = (uint64_t)std::max(G, 1) * P.numTiles;
     if (!h->binCount.ensure((h->numBins + 1) * 4, h->err, "bin counts") ||
         !h->binStart.ensure((h->numBins + 1) * 4, h->err, "bin offsets"))
@@ -771,7 +821,7 @@ int vox_compute_edges_face_normals_and_bounds(vox_ctx* h) {
     uint32_t* start = h->binStart.as<uint32_t>();
     h->run("fill", [&] {
         const FillSeg z[2] = {{cnt, h->numBins, 0u},
-                              {h->counters.as<uint32_t>() + kScanErrWord, 1, 0u}};
+                              {h->counters.as<uint32_t>(), kCounterWords, 0u}};
         launch_fill_segs(h->st, z, 2);
     });
     h->run("setup", [&] {
@@ -784,22 +834,7 @@ int vox_compute_edges_face_normals_and_bounds(vox_ctx* h) {
         launch_scan_clear(h->st, cnt, start, h->numBins, h->scanTmp.as<uint32_t>(),
                           h->counters.as<uint32_t>() + kScanErrWord);
     });
-    uint32_t total = 0;
-    if (h->replay) {
-        total = (uint32_t)h->planPairs;
-    } else {
-        if (!h->check(hipMemcpyAsync(&total, start + h->numBins, 4, hipMemcpyDeviceToHost, h->st),
-                      "bin total") ||
-            !h->check(hipStreamSynchronize(h->st), "setup"))
-            return 0;
-        h->planPairs = total;
-    }
-    h->pairs = total;
-    if (!h->binTri.ensure((uint64_t)total * 4, h->err, "bin entries")) return 0;
-    h->run("scatter", [&] {
-        launch_scatter(h->st, P, h->gargs, h->bbox.as<uint32_t>(), start, cnt,
-                       h->binTri.as<uint32_t>());
-    });
+    if (!h->check(hipGetLastError(), "setup")) return 0;
     h->prepared = true;
     return 1;
 }
@@ -833,52 +868,59 @@ int gen_front(vox_ctx* h) {
         (void)hipEventRecord(h->evStart, st);
     }
 
+    // the setup pass's counters and counts serve one generate
+    h->prepared = false;
     // Active tiles: level 0 from the bins, level k from level src(k).
     LevelBufs& l0 = h->lv[0];
-    h->run("activity", [&] {
-        launch_activity0(st, P, G, h->grpFill.as<int32_t>(), h->binStart.as<uint32_t>(),
-                         l0.mark.as<uint32_t>());
+    uint32_t* ctr = h->counters.as<uint32_t>();
+    h->run("tile_map", [&] {
+        launch_map_tiles0(st, P, G, h->grpFill.as<int32_t>(), h->binStart.as<uint32_t>(),
+                          l0.tileIdx.as<int32_t>(), l0.list.as<int32_t>(), ctr);
     });
+    l0.aliasOf = -1;
     const bool chain = (h->options & VOX_OPT_MIP_CHAIN) != 0;
     auto srcOf = [&](int k) { return chain ? k - 1 : (k == 1 ? 0 : k - 2); };
-    uint32_t* ctr = h->counters.as<uint32_t>();
-    // Each level is compacted before the next one marks its parents; the
-    // dense tile list is sized for every tile of the level.
-    for (int k = 0; k < L; ++k) {
+    // Each level is mapped from its source level's map; the dense tile list
+    // is sized for every tile of the level.
+    for (int k = 1; k < L; ++k) {
         LevelBufs& l = h->lv[k];
         // (each chunk has its own chain: level 2j is not level 2j - 1 then)
         l.aliasOf = (!chain && !h->multi && k >= 2 && (k % 2) == 0) ? k - 1 : -1;
         if (l.aliasOf >= 0) continue;
-        if (k > 0) {
-            LevelView s = view(h, srcOf(k));
-            MipShift shift;
-            if (h->multi && mip_shift_for(s.map, l.map, chunkGeom(h), srcOf(k), k, shift))
-                h->run("mark", [&] {
-                    launch_mark_children_shifted(st, s.map, l.map, shift, l.mark.as<uint32_t>());
-                });
-            else if (h->multi)
-                h->run("mark", [&] {
-                    launch_chunk_mark(st, s.map, l.map, chunkGeom(h), srcOf(k), k,
-                                      l.mark.as<uint32_t>());
-                });
+        const LevelView s = view(h, srcOf(k));
+        MipShift shift{};
+        const bool general =
+            h->multi && !mip_shift_for(s.map, l.map, chunkGeom(h), srcOf(k), k, shift);
+        h->run("tile_map", [&] {
+            if (general)
+                launch_chunk_map(st, s.map, l.map, chunkGeom(h), srcOf(k), k,
+                                 l.tileIdx.as<int32_t>(), l.list.as<int32_t>(), ctr + k);
             else
-                h->run("mark", [&] { launch_mark_children(st, s.map, l.map, l.mark.as<uint32_t>()); });
-        }
-        h->run("scan", [&] { scan(h, l.mark.as<uint32_t>(), l.excl.as<uint32_t>(), l.map.numTiles); });
-        h->run("compact", [&] {
-            launch_compact(st, l.map.numTiles, l.mark.as<uint32_t>(), l.excl.as<uint32_t>(),
-                           l.tileIdx.as<int32_t>(), l.list.as<int32_t>(), ctr + k);
+                launch_map_children(st, s.map, l.map, shift, l.tileIdx.as<int32_t>(),
+                                    l.list.as<int32_t>(), ctr + k);
         });
     }
     uint32_t act[VOX_MAX_LEVELS] = {0};
     if (h->replay) {
         std::memcpy(act, h->planAct, sizeof(act));
+        h->pairs = h->planPairs;
     } else {
-        if (!h->check(hipMemcpyAsync(act, ctr, 4 * L, hipMemcpyDeviceToHost, st), "tile counts") ||
+        h->run("tile_map", [&] {
+            launch_map_counts(st, ctr, L, h->binStart.as<uint32_t>() + h->numBins,
+                              h->pin + kPinTiles);
+        });
+        if (!h->check(hipGetLastError(), "tile maps") ||
             !h->check(hipStreamSynchronize(st), "tile maps"))
             return 0;
+        std::memcpy(act, h->pin + kPinTiles, 4 * L);
         std::memcpy(h->planAct, act, sizeof(act));
+        h->pairs = h->planPairs = h->pin[kPinTiles + kMaxLevels];
     }
+    if (!h->binTri.ensure(h->pairs * 4, h->err, "bin entries")) return 0;
+    h->run("scatter", [&] {
+        launch_scatter(st, P, h->gargs, h->bbox.as<uint32_t>(), h->binStart.as<uint32_t>(),
+                       h->binCount.as<uint32_t>(), h->binTri.as<uint32_t>());
+    });
     for (int k = 0; k < L; ++k) {
         LevelBufs& l = h->lv[k];
         if (l.aliasOf >= 0) {
@@ -897,22 +939,29 @@ int gen_front(vox_ctx* h) {
         (1ull << 32))
         return h->fail("more hit records than 32-bit indices address; use fewer persistent "
                        "workgroups or a smaller grid"), 0;
+    // work lists of kGroupSet overlapping groups at a time; counters per group
+    uint64_t overlapping = 0;
+    for (const GroupArgs& ga : h->gargs) overlapping += ga.overlaps ? 1 : 0;
+    const uint64_t lists = std::min<uint64_t>(std::max<uint64_t>(overlapping, 1), kGroupSet);
+    const uint64_t counts = std::max<uint64_t>(overlapping, 1);
     if (!h->occ0.ensure((uint64_t)l0.active * kTileWords * 4, h->err, "occupancy words") ||
         !h->fill0.ensure((uint64_t)l0.active * kTileWords * 4, h->err, "filled-voxel words") ||
         !h->hit0.ensure((uint64_t)l0.active * kTileWords * 4, h->err, "hit words") ||
-        !h->work.ensure((uint64_t)l0.active * 16, h->err, "tile work list") ||
-        !h->workCount.ensure(4, h->err, "tile work count") ||
+        !h->work.ensure(lists * l0.active * 16, h->err, "tile work lists") ||
+        !h->workCount.ensure(4 * counts, h->err, "tile work counts") ||
         !h->rec.ensure(kRecSegs * rec_seg_cap(l0.active, vox_grid(l0.active, h->persistentBlocks)) *
                            32,
                        h->err, "hit records") ||
-        !h->recCount.ensure(4 * kRecSegs, h->err, "hit record counts"))
+        !h->recCount.ensure(4 * kRecSegs * counts, h->err, "hit record counts"))
         return 0;
     unsigned long long* satc = h->sat.as<unsigned long long>();
     h->run("fill", [&] {
-        const FillSeg z[3] = {{h->occ0.as<uint32_t>(), l0.active * kTileWords, 0u},
+        const FillSeg z[5] = {{h->occ0.as<uint32_t>(), l0.active * kTileWords, 0u},
                               {h->fill0.as<uint32_t>(), l0.active * kTileWords, 0u},
-                              {reinterpret_cast<uint32_t*>(satc), 2, 0u}};
-        launch_fill_segs(st, z, 3);
+                              {reinterpret_cast<uint32_t*>(satc), 2, 0u},
+                              {h->workCount.as<uint32_t>(), counts, 0u},
+                              {h->recCount.as<uint32_t>(), kRecSegs * counts, 0u}};
+        launch_fill_segs(st, z, 5);
     });
     // Level 0 stores only hit or filled voxels: the others read as zero
     // wherever level 0 is read (LevelMap::defOcc / defFill), so no tile is
@@ -923,35 +972,62 @@ int gen_front(vox_ctx* h) {
     return 1;
 }
 
-void gen_group_tiles(vox_ctx* h, int g) {
+// Place of group g among the overlapping ones: its counters, and (modulo
+// kGroupSet) its work list.
+uint64_t group_place(const vox_ctx* h, int g) {
+    uint64_t k = 0;
+    for (int i = 0; i < g; ++i) k += h->gargs[i].overlaps ? 1 : 0;
+    return k;
+}
+struct GroupBufs {
+    uint4* work;
+    uint32_t* workCount;
+    uint32_t* recCount;
+};
+GroupBufs group_bufs(vox_ctx* h, int g) {
+    const uint64_t k = group_place(h, g);
+    return {h->work.as<uint4>() + (k % kGroupSet) * h->lv[0].active,
+            h->workCount.as<uint32_t>() + k, h->recCount.as<uint32_t>() + k * kRecSegs};
+}
+
+// The work lists of n overlapping groups (at most kGroupSet, consecutive
+// among the overlapping ones).
+void gen_group_tiles(vox_ctx* h, const int* g, int n) {
     LevelBufs& l0 = h->lv[0];
+    WorkSet W{};
+    W.n = n;
+    for (int i = 0; i < n; ++i) {
+        const GroupBufs b = group_bufs(h, g[i]);
+        W.work[i] = b.work;
+        W.count[i] = b.workCount;
+        W.g[i] = g[i];
+    }
     h->run("group_tiles", [&] {
-        launch_group_tiles(h->st, h->P, g, l0.active, l0.list.as<int32_t>(),
-                           h->binStart.as<uint32_t>(), h->work.as<uint4>(),
-                           h->workCount.as<uint32_t>(), h->recCount.as<uint32_t>());
+        launch_group_tiles(h->st, h->P, W, l0.active, l0.list.as<int32_t>(),
+                           h->binStart.as<uint32_t>());
     });
 }
 
 void gen_voxelize(vox_ctx* h, int g) {
     LevelBufs& l0 = h->lv[0];
+    const GroupBufs b = group_bufs(h, g);
     h->run("voxelize_g" + std::to_string(g), [&] {
         launch_voxelize(h->st, h->P, h->gargs[g], g, g == first_overlap(h) ? 1 : 0, l0.active,
                         l0.list.as<int32_t>(), h->verts.as<float>(), h->fnorm.as<float>(),
                         h->bbox.as<uint32_t>(), h->binStart.as<uint32_t>(),
                         h->binTri.as<uint32_t>(), h->occ0.as<uint32_t>(), h->hit0.as<uint32_t>(),
-                        h->sat.as<unsigned long long>(), h->work.as<uint4>(),
-                        h->workCount.as<uint32_t>(), h->rec.as<uint4>(),
-                        h->recCount.as<uint32_t>(), h->persistentBlocks);
+                        h->sat.as<unsigned long long>(), b.work, b.workCount, h->rec.as<uint4>(),
+                        b.recCount, h->persistentBlocks);
     });
 }
 
 VoxUnitJob gen_voxelize_job(vox_ctx* h, int g) {
     LevelBufs& l0 = h->lv[0];
+    const GroupBufs b = group_bufs(h, g);
     return voxelize_job(h->P, h->gargs[g], g == first_overlap(h) ? 1 : 0, l0.active,
                         h->verts.as<float>(), h->fnorm.as<float>(), h->bbox.as<uint32_t>(),
                         h->binTri.as<uint32_t>(), h->occ0.as<uint32_t>(), h->hit0.as<uint32_t>(),
-                        h->work.as<uint4>(), h->workCount.as<uint32_t>(), h->rec.as<uint4>(),
-                        h->recCount.as<uint32_t>(), h->persistentBlocks);
+                        b.work, b.workCount, h->rec.as<uint4>(), b.recCount, h->persistentBlocks);
 }
 
 void gen_group_tail(vox_ctx* h, int g) {
@@ -961,7 +1037,7 @@ void gen_group_tail(vox_ctx* h, int g) {
     hipStream_t st = h->st;
     const VoxParams& P = h->P;
     h->run("colour_g" + std::to_string(g), [&] {
-        launch_colour(st, P, ga, init, l0.active, h->rec.as<uint4>(), h->recCount.as<uint32_t>(),
+        launch_colour(st, P, ga, init, l0.active, h->rec.as<uint4>(), group_bufs(h, g).recCount,
                       l0.list.as<int32_t>(), h->verts.as<float>(), h->fnorm.as<float>(),
                       l0.col.as<uint32_t>(), l0.qn.as<uint32_t>(), l0.nrm.as<float>(),
                       h->fill0.as<uint32_t>(), h->persistentBlocks);
@@ -1069,9 +1145,13 @@ int gen_back(vox_ctx* h, const char* out_dir, int binary) {
     std::vector<std::array<uint32_t, 3>> borders(L);
     // The samples of all depths in one launch, then each depth's comparison.
     static_assert(kMaxLevels >= VOX_MAX_LEVELS, "one sample entry per depth");
-    SampleDepths S{};
+    CompareDepths CD{};
+    SampleDepths& S = CD.S;
     S.L = L;
-    for (int a = 0; a < 3; ++a) S.B[a] = h->B[a];
+    for (int a = 0; a < 3; ++a) {
+        S.B[a] = h->B[a];
+        S.invB[a] = 1.0f / (float)h->B[a];
+    }
     for (int d = L - 1; d >= 0; --d) {
         LevelView l = view(h, L - 1 - d);
         DepthBufs& t = h->tree[d];
@@ -1092,17 +1172,29 @@ int gen_back(vox_ctx* h, const char* out_dir, int binary) {
     S.start[L] = h->allNodes;
     const uint64_t bvox = (uint64_t)(h->B[0] + 2) * (h->B[1] + 2) * (h->B[2] + 2);
     uint32_t nb[VOX_MAX_LEVELS] = {0};
+    DepthOut dout{};
+    dout.L = L;
+    for (int d = 0; d < L; ++d) {
+        dout.bidx[d] = h->tree[d].bidx.as<uint32_t>();
+        dout.types[d] = h->tree[d].types.as<uint8_t>();
+        dout.off[d] = h->tree[d].off;
+    }
+    dout.off[L] = h->allNodes;
+    // the counts the host needs, left in pinned memory
+    auto counts = [&](const uint32_t* excl, const uint64_t* offs, const uint32_t* cnt) {
+        if (h->replay) return;
+        h->run("scan", [&] {
+            launch_generate_counts(st, excl, offs, cnt, L, reinterpret_cast<uint32_t*>(satc),
+                                   ctr + kScanErrWord, h->pin + kPinCounts);
+        });
+    };
     if (h->multi) {
         // Several chunks: per-chunk samples and types OR-ed over chunks, and
         // bricks numbered in the order the brick writer writes them (the
         // chunk that completes a brick, inside one chunk before across
         // chunks, node order), by a key sort per depth.
         const ChunkGeom cg = chunkGeom(h);
-        uint32_t* bcount = ctr + 64;
-        h->run("fill", [&] {
-            const FillSeg z[1] = {{bcount, (uint64_t)L, 0u}};
-            launch_fill_segs(st, z, 1);
-        });
+        uint32_t* bcount = ctr + kChunkBricksWord;
         h->run("node_type", [&] {
             launch_chunk_node_type(st, S, cg);
             for (int d = L - 1; d >= 0; --d) {
@@ -1112,10 +1204,10 @@ int gen_back(vox_ctx* h, const char* out_dir, int binary) {
                                         h->nodesA.as<uint32_t>() + t.off, bcount + d);
             }
         });
+        counts(nullptr, nullptr, bcount);
         occupancy();
-        if (!h->check(hipMemcpyAsync(nb, bcount, 4 * L, hipMemcpyDeviceToHost, st), "brick counts") ||
-            !h->check(hipStreamSynchronize(st), "node typing"))
-            return 0;
+        if (!h->check(hipStreamSynchronize(st), "node typing")) return 0;
+        std::memcpy(nb, h->pin + kPinCounts, 4 * L);
         uint32_t rankBits = 0;
         while ((1ull << rankBits) < (uint64_t)h->nc[0] * h->nc[1] * h->nc[2]) ++rankBits;
         for (int d = 0; d < L; ++d) {
@@ -1154,11 +1246,14 @@ int gen_back(vox_ctx* h, const char* out_dir, int binary) {
     } else {
         h->run("node_type", [&] {
             launch_node_sample_all(st, S);
+            uint64_t end = 0;
             for (int d = L - 1; d >= 0; --d) {
-                LevelView l = view(h, L - 1 - d);
-                launch_node_compare(st, l.map, l.active, l.list, l.col, S.Rd[d], h->B, S.border[d],
-                                    S.xLimit[d], S.cc[d], S.flag[d]);
+                const LevelView l = view(h, L - 1 - d);
+                CD.list[d] = l.list;
+                end += l.active;
+                CD.tileEnd[d] = end;
             }
+            launch_node_compare_all(st, CD);
         });
         // One scan over the flags of every depth; a depth's brick addresses are
         // its scan values less the value at its first node.
@@ -1169,21 +1264,16 @@ int gen_back(vox_ctx* h, const char* out_dir, int binary) {
             uint64_t offs[VOX_MAX_LEVELS + 1];
             for (int d = 0; d < L; ++d) offs[d] = h->tree[d].off;
             offs[L] = h->allNodes;
-            h->run("scan", [&] {
-                launch_range_counts(st, h->nodeExcl.as<uint32_t>(), offs, L, ctr + 32);
-            });
+            counts(h->nodeExcl.as<uint32_t>(), offs, nullptr);
         }
         occupancy();
         if (h->replay) {
             std::memcpy(nb, h->planNb, sizeof(nb));
         } else {
-            if (!h->check(hipMemcpyAsync(nb, ctr + 32, 4 * L, hipMemcpyDeviceToHost, st), "brick counts") ||
-                !h->check(hipStreamSynchronize(st), "node typing"))
-                return 0;
+            if (!h->check(hipStreamSynchronize(st), "node typing")) return 0;
+            std::memcpy(nb, h->pin + kPinCounts, 4 * L);
             std::memcpy(h->planNb, nb, sizeof(nb));
         }
-        DepthOut dout{};
-        dout.L = L;
         for (int d = 0; d < L; ++d) {
             DepthBufs& t = h->tree[d];
             t.bricks = nb[d];
@@ -1192,24 +1282,15 @@ int gen_back(vox_ctx* h, const char* out_dir, int binary) {
                 !t.bcol.ensure((uint64_t)nb[d] * bvox * 4, h->err, "brick colours") ||
                 !t.bnrm.ensure((uint64_t)nb[d] * bvox * 4, h->err, "brick normals"))
                 return 0;
-            dout.bidx[d] = t.bidx.as<uint32_t>();
             dout.brickNode[d] = t.brickNode.as<uint32_t>();
-            dout.types[d] = t.types.as<uint8_t>();
-            dout.off[d] = t.off;
         }
-        dout.off[L] = h->allNodes;
         h->run("brick_assign", [&] {
             launch_brick_assign_all(st, h->nodeFlag.as<uint32_t>(), h->nodeExcl.as<uint32_t>(), dout);
         });
     }
     // CollapseConstantBranches (Voxelizer.cu 701-774): the types are final.
     if (overlap) side.fork();
-    for (int d = L - 2; d >= 0; --d) {
-        h->run("collapse", [&] {
-            launch_collapse(aux, h->tree[d].Rd, d + 1 == L - 1 ? 1 : 0,
-                            h->tree[d].types.as<uint8_t>(), h->tree[d + 1].types.as<uint8_t>());
-        });
-    }
+    h->run("collapse", [&] { launch_collapse_all(aux, dout, ctr + kCollapseWord); });
     // The bricks of all depths in one launch, the deepest (largest) first.
     GatherDepths GD{};
     for (int a = 0; a < 3; ++a) GD.B[a] = h->B[a];
@@ -1254,17 +1335,15 @@ int gen_back(vox_ctx* h, const char* out_dir, int binary) {
     h->workReleased = false;
     if (h->replay) {
         h->haveResult = true;
-        h->prepared = false;
         return firstOverlap >= 0 ? 1 : -1;
     }
     (void)hipEventRecord(h->evStop, st);
-    unsigned long long sat = 0;
-    uint32_t scanErr = 0;
-    if (!h->check(hipMemcpyAsync(&sat, satc, 8, hipMemcpyDeviceToHost, st), "counters") ||
-        !h->check(hipMemcpyAsync(&scanErr, ctr + kScanErrWord, 4, hipMemcpyDeviceToHost, st),
-                  "counters") ||
+    if (!h->check(hipGetLastError(), "generate kernels") ||
         !h->check(hipStreamSynchronize(st), "generate"))
         return 0;
+    unsigned long long sat = 0;
+    std::memcpy(&sat, h->pin + kPinCounts + kMaxLevels, 8);
+    const uint32_t scanErr = h->pin[kPinCounts + kMaxLevels + 2];
     if (scanErr)
         return h->fail("a device-wide prefix sum gave up waiting on a predecessor; the result is "
                        "not valid (run vox_generate again)"), 0;
@@ -1284,7 +1363,6 @@ int gen_back(vox_ctx* h, const char* out_dir, int binary) {
         return 0;
     if (h->options & VOX_OPT_TIMING) collect_timings(h);
     h->haveResult = true;
-    h->prepared = false;  // bins are consumed; a new generate re-runs setup
     if (out_dir) {
         if (!vox_write_files_impl(h, out_dir, h->p, h->dP, h->N, binary ? 1 : 0, h->extra, h->C,
                                   h->multi ? 1 : 0))
@@ -1306,11 +1384,14 @@ int vox_generate(vox_ctx* h, const char* out_dir, int binary, int compressed) {
     if (!h->prepared && !vox_compute_edges_face_normals_and_bounds(h)) return 0;
     if (!gen_front(h)) return 0;
     // Voxelize, colour and fill, group by group (Voxelizer.cu 2335-2553).
-    for (int g = 0; g < (int)h->gargs.size(); ++g) {
-        if (!h->gargs[g].overlaps) continue;
-        gen_group_tiles(h, g);
-        gen_voxelize(h, g);
-        gen_group_tail(h, g);
+    std::vector<int> over;
+    for (int g = 0; g < (int)h->gargs.size(); ++g)
+        if (h->gargs[g].overlaps) over.push_back(g);
+    for (size_t k = 0; k < over.size(); ++k) {
+        if (k % kGroupSet == 0)
+            gen_group_tiles(h, over.data() + k, (int)std::min<size_t>(kGroupSet, over.size() - k));
+        gen_voxelize(h, over[k]);
+        gen_group_tail(h, over[k]);
     }
     return gen_back(h, out_dir, binary);
 }
@@ -1477,7 +1558,7 @@ void buffer_list(vox_ctx* h, std::vector<void*>& out) {
                      &h->counters, &h->nodeFlag, &h->nodeExcl, &h->fill0};
     for (DevBuf* b : top) out.push_back(b->p);
     for (auto& l : h->lv) {
-        DevBuf* lb[] = {&l.mark, &l.excl, &l.tileIdx, &l.list, &l.col, &l.qn, &l.nrm};
+        DevBuf* lb[] = {&l.tileIdx, &l.list, &l.col, &l.qn, &l.nrm};
         for (DevBuf* b : lb) out.push_back(b->p);
     }
     for (auto& t : h->tree) {
@@ -1783,7 +1864,7 @@ int vox_batch_capture(vox_batch* b) {
             const size_t j = order[k];
             if (groupsOf[j].size() <= w) continue;
             vox_ctx* h = b->jobs[j];
-            gen_group_tiles(h, groupsOf[j][w]);
+            gen_group_tiles(h, &groupsOf[j][w], 1);
             table.push_back(gen_voxelize_job(h, groupsOf[j][w]));
             ok = b->check(hipEventRecord(b->preVox[j], b->branch[j]), "join") &&
                  b->check(hipStreamWaitEvent(b->st, b->preVox[j], 0), "join");

@@ -100,6 +100,7 @@ constexpr int kFillTiles = 3;       // ceil(19 / 8)
 struct VoxParams {
     uint32_t S[3];        // voxel space per axis (N + 4*extra)
     uint32_t TG[3];       // level-0 tile grid, ceil(S/8)
+    double invTG[2];      // 1 / TG[0], 1 / TG[1]
     uint64_t numTiles;    // TG[0]*TG[1]*TG[2]
     float offP[3];        // p - extra*delta
     float dP[3];          // delta
@@ -129,6 +130,7 @@ struct GroupArgs {
 struct LevelMap {         // sparse tiles of one mip level
     uint32_t dims[3];     // S_k
     uint32_t TG[3];       // tile grid
+    double invTG[2];      // 1 / TG[0], 1 / TG[1]
     uint64_t numTiles;
     const int32_t* tileIdx;   // dense map tile -> compact index or -1
     // Level 0 stores only the voxels that some group hit (defOcc, the
@@ -214,15 +216,25 @@ void launch_setup(hipStream_t st, const VoxParams& P, const std::vector<GroupArg
 void launch_scatter(hipStream_t st, const VoxParams& P, const std::vector<GroupArgs>& groups,
                     const uint32_t* bbox, const uint32_t* binStart, uint32_t* binFill,
                     uint32_t* binTri);
-void launch_activity0(hipStream_t st, const VoxParams& P, int ngroups, const int32_t* grpFill,
-                      const uint32_t* binStart, uint32_t* mark);
-// Also writes excl[n] (the number of marked tiles) to *count.
-void launch_compact(hipStream_t st, uint64_t n, const uint32_t* mark, const uint32_t* excl,
-                    int32_t* tileIdx, int32_t* list, uint32_t* count);
-// mark[t] = 1 when any of the (up to 8) source tiles under level tile t is
-// active, else 0: every mark written, no clearing first.
-void launch_mark_children(hipStream_t st, const LevelMap& src, const LevelMap& dst,
-                          uint32_t* markDst);
+// The chunked mip filter as the single-chunk one with a per-chunk source
+// offset (MipShift), where the chunk geometry allows it: every axis's chunk
+// extent at the level a multiple of the tile edge, the per-chunk offset a
+// multiple of two tiles and every source inside the source level.
+struct MipShift {
+    uint32_t cd[3];    // chunk extent at the level (0: one chunk, no shift)
+    uint32_t off[3];   // source offset per chunk: Cs - 2 Cd
+};
+// Tile maps: tileIdx[t] = the active tile's place in list, or -1; *count =
+// active tiles (zero before the launch).
+void launch_map_tiles0(hipStream_t st, const VoxParams& P, int ngroups, const int32_t* grpFill,
+                       const uint32_t* binStart, int32_t* tileIdx, int32_t* list, uint32_t* count);
+// A level tile is active when any of the (up to 8) source tiles under it is.
+void launch_map_children(hipStream_t st, const LevelMap& src, const LevelMap& dst,
+                         const MipShift& shift, int32_t* tileIdx, int32_t* list, uint32_t* count);
+// Into pinned host memory: host[k] = tiles[k] for k < n (n <= kMaxLevels),
+// host[kMaxLevels] = *pairs.
+void launch_map_counts(hipStream_t st, const uint32_t* tiles, int n, const uint32_t* pairs,
+                       uint32_t* host);
 void launch_voxelize(hipStream_t st, const VoxParams& P, const GroupArgs& G, int g, int init,
                      uint64_t nActive, const int32_t* list, const float* verts,
                      const float* fnorm, const uint32_t* bbox, const uint32_t* binStart,
@@ -259,9 +271,17 @@ VoxUnitJob voxelize_job(const VoxParams& P, const GroupArgs& G, int init, uint64
 // queue one.
 void launch_voxelize_batch(hipStream_t st, const VoxUnitJob* jobs, uint32_t njobs,
                            uint32_t* unitStart, uint32_t* queue, unsigned blocks);
-void launch_group_tiles(hipStream_t st, const VoxParams& P, int g, uint64_t nActive,
-                        const int32_t* list, const uint32_t* binStart, uint4* work,
-                        uint32_t* workCount, uint32_t* recCount);
+// The work lists of up to kGroupSet groups in one launch: entry i the tiles
+// holding triangles of group g[i], at work[i] (room for every active tile),
+// counted in *count[i] (zero before).
+struct WorkSet {
+    uint4* work[kGroupSet];
+    uint32_t* count[kGroupSet];
+    int32_t g[kGroupSet];
+    int n;
+};
+void launch_group_tiles(hipStream_t st, const VoxParams& P, const WorkSet& W, uint64_t nActive,
+                        const int32_t* list, const uint32_t* binStart);
 // fillw: level 0's filled-voxel words (a voxel neither hit before this group
 // nor filled holds no stored value and counts as zero).
 void launch_colour(hipStream_t st, const VoxParams& P, const GroupArgs& G, int init,
@@ -294,14 +314,20 @@ struct SampleDepths {
     uint32_t xLimit[kMaxLevels];
     uint64_t start[kMaxLevels + 1];
     uint32_t B[3];
+    float invB[3];        // 1 / B
     int L;
 };
 void launch_node_sample_all(hipStream_t st, const SampleDepths& S);
-// Node typing, second half: every voxel of the active tiles compared with the
-// samples of the nodes whose bricks hold it.
-void launch_node_compare(hipStream_t st, const LevelMap& lm, uint64_t nActive, const int32_t* list,
-                         const uint32_t* col, uint32_t Rd, const uint32_t B[3],
-                         const uint32_t border[3], uint32_t xLimit, uint32_t* cc, uint32_t* flag);
+// Node typing, second half, every depth in one launch: every voxel of the
+// active tiles compared with the samples of the nodes whose bricks hold it.
+// Depth d's level has the tiles list[d]; the launch walks the depths from the
+// deepest, depth d ending at tile tileEnd[d].
+struct CompareDepths {
+    SampleDepths S;
+    const int32_t* list[kMaxLevels];
+    uint64_t tileEnd[kMaxLevels];
+};
+void launch_node_compare_all(hipStream_t st, const CompareDepths& C);
 // Brick indices of every depth in one launch over the all-depth node array:
 // node n of depth d (off[d] <= n < off[d + 1]) gets type, brick index
 // (excl[n] - excl[off[d]]) and its brick's node.
@@ -318,9 +344,12 @@ void launch_brick_assign_all(hipStream_t st, const uint32_t* flag, const uint32_
 struct RangeOffs {
     uint64_t v[kMaxLevels + 1];
 };
-// out[d] = excl[offs[d + 1]] - excl[offs[d]] for d < n (n <= kMaxLevels).
-void launch_range_counts(hipStream_t st, const uint32_t* excl, const uint64_t* offs, int n,
-                         uint32_t* out);
+// Into pinned host memory: host[d] = counts[d], or without counts excl[offs[d
+// + 1]] - excl[offs[d]], for d < n (n <= kMaxLevels); the two words of sat
+// and the word at err after kMaxLevels of them.
+void launch_generate_counts(hipStream_t st, const uint32_t* excl, const uint64_t* offs,
+                            const uint32_t* counts, int n, const uint32_t* sat,
+                            const uint32_t* err, uint32_t* host);
 // The bricks of every depth in one launch: entry e (a depth with bricks)
 // covers workgroups start[e] <= w < start[e + 1], one brick each.
 struct GatherDepths {
@@ -337,8 +366,9 @@ struct GatherDepths {
     int n;
 };
 void launch_brick_gather_all(hipStream_t st, const GatherDepths& G);
-void launch_collapse(hipStream_t st, uint32_t Rd, int childIsLeaf, uint8_t* types,
-                     const uint8_t* childTypes);
+// LEAF-CONST marks of every depth from the final types (ticket: a device word,
+// zero before the launch).
+void launch_collapse_all(hipStream_t st, const DepthOut& D, uint32_t* ticket);
 
 // ---- several chunks (generateVoxelsAndOctTree's chunk loop, Voxelizer.cu
 // 2180-2814, with chunks smaller than the voxel space) ----
@@ -351,23 +381,13 @@ struct ChunkGeom {
     // visit rank of chunk (i, j, l) at [(l * nc[1] + j) * nc[0] + i]
     const uint32_t* rank;
 };
-// mark[t] = 1 when a voxel of level tile t reads an active source tile
-// (source voxels 2x, 2x + 1 of the same chunk, local coordinates).
-// (ks: the source level, kd: the level built from it.)
-void launch_chunk_mark(hipStream_t st, const LevelMap& src, const LevelMap& dst,
-                       const ChunkGeom& cg, int ks, int kd, uint32_t* markDst);
-// The chunked mip filter as the single-chunk one with a per-chunk source
-// offset (MipShift), where the chunk geometry allows it: every axis's chunk
-// extent at the level a multiple of the tile edge, the per-chunk offset a
-// multiple of two tiles and every source inside the source level.
-struct MipShift {
-    uint32_t cd[3];    // chunk extent at the level (0: one chunk, no shift)
-    uint32_t off[3];   // source offset per chunk: Cs - 2 Cd
-};
+// The tile map of a level: a tile is active when a voxel of it reads an active
+// source tile (source voxels 2x, 2x + 1 of the same chunk, local
+// coordinates; ks: the source level, kd: the level built from it).
+void launch_chunk_map(hipStream_t st, const LevelMap& src, const LevelMap& dst, const ChunkGeom& cg,
+                      int ks, int kd, int32_t* tileIdx, int32_t* list, uint32_t* count);
 bool mip_shift_for(const LevelMap& src, const LevelMap& dst, const ChunkGeom& cg, int ks, int kd,
                    MipShift& out);
-void launch_mark_children_shifted(hipStream_t st, const LevelMap& src, const LevelMap& dst,
-                                  const MipShift& shift, uint32_t* markDst);
 void launch_mip_shifted(hipStream_t st, const LevelMap& src, const LevelMap& dst,
                         const MipShift& shift, uint64_t nActive, const int32_t* listDst,
                         const uint32_t* colSrc, const float* nrmSrc, uint32_t* colDst,
@@ -408,7 +428,7 @@ void launch_occupancy(hipStream_t st, const VoxParams& P, uint64_t nActive, cons
 void launch_dense_level(hipStream_t st, const LevelMap& lm, const uint32_t* col,
                         const float* nrm, uint32_t* outCol, float* outNrm);
 void launch_fill_u32(hipStream_t st, uint32_t* p, uint64_t n, uint32_t v);
-// Up to four (pointer, words, value) fills in one launch.
+// Up to six (pointer, words, value) fills in one launch.
 struct FillSeg {
     uint32_t* p;
     uint64_t n;

@@ -78,15 +78,22 @@ __device__ __forceinline__ void fill_inv255(float* s_inv255) {
     for (int i = threadIdx.x; i < 256; i += blockDim.x) s_inv255[i] = (float)i / 255.0f;
 }
 
-// Linear tile index -> tile coordinates (32-bit arithmetic; tile grids hold
-// fewer than 2^31 tiles).
-__device__ __forceinline__ void tile_xyz(uint64_t tlin64, const uint32_t* TG, uint32_t& x,
-                                         uint32_t& y, uint32_t& z) {
+// t / d for t, d < 2^31 given inv = 1.0 / d: (t + 1/2) / d lies at least
+// 1 / (2 d) >= 2^-32 from a whole number, the product within 2^-20 of that
+// distance (an integer division takes some 40 instructions).
+__device__ __forceinline__ uint32_t udiv_inv(uint32_t t, double inv) {
+    return (uint32_t)(((double)t + 0.5) * inv);
+}
+// Linear tile index -> tile coordinates (tile grids hold fewer than 2^31
+// tiles), M a level map or the voxel parameters.
+template <class M>
+__device__ __forceinline__ void tile_xyz(uint64_t tlin64, const M& m, uint32_t& x, uint32_t& y,
+                                         uint32_t& z) {
     const uint32_t t = (uint32_t)tlin64;
-    const uint32_t q = t / TG[0];
-    x = t - q * TG[0];
-    z = q / TG[1];
-    y = q - z * TG[1];
+    const uint32_t q = udiv_inv(t, m.invTG[0]);
+    x = t - q * m.TG[0];
+    z = udiv_inv(q, m.invTG[1]);
+    y = q - z * m.TG[1];
 }
 // Node index at a depth with Rd = 2^ld nodes per axis.
 __device__ __forceinline__ void node_xyz(uint64_t n, uint32_t ld, uint32_t& x, uint32_t& y,
@@ -415,67 +422,145 @@ __global__ __launch_bounds__(kBlock) void k_scatter(VoxParams P, GroupSet S,
     }
 }
 
+// Until every memory operation of the wave has returned.
+__device__ __forceinline__ void wait_memory() {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+}
+
+// Tile maps.  A thread decides kMapRows (1 or 4) times kMapTiles consecutive
+// tiles of a level (active(t0): a bit per tile); a workgroup's active tiles take
+// consecutive places of the level's list in tile order, reserved with one
+// atomic, so neighbours along x stay neighbours there (the order of
+// workgroups is any: a tile's place changes no result).  Bound by the reads of
+// the bins (or the source map), and past some 2,000 workgroups by the atomics
+// on the one counter, hence 4096 tiles a workgroup.  Marks, a scan over them
+// and a compaction took three launches and passes a level: 43 us on level 0
+// of the 1024^3 workload, a fifth of the smallest calls' device time.
+// (Small maps take 1024 tiles a workgroup: 4096 left a few workgroups to a
+// long chain of reads.)
+constexpr int kMapTiles = 4;
+constexpr uint32_t kMapBlock = kBlock * kMapTiles;   // tiles of a workgroup, per row
+constexpr uint64_t kMapSmall = 512 * kMapBlock;      // up to here one row
+template <int kMapRows, class Active>
+__device__ __forceinline__ void map_tiles(uint64_t n, Active active, int32_t* __restrict__ tileIdx,
+                                          int32_t* __restrict__ list,
+                                          uint32_t* __restrict__ count) {
+    constexpr int kParts = kMapRows * (kBlock / 64);
+    static_assert(kParts <= 64, "one wave scans the parts");
+    __shared__ uint32_t s_part[kParts];
+    __shared__ uint32_t s_base;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint64_t b0 =
+        (uint64_t)blockIdx.x * (kMapBlock * kMapRows) + (uint64_t)tid * kMapTiles;
+    uint32_t m[kMapRows], e[kMapRows];
+#pragma unroll
+    for (int j = 0; j < kMapRows; ++j) {
+        const uint64_t t0 = b0 + (uint64_t)j * kBlock * kMapTiles;
+        m[j] = t0 < n ? active(t0) : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < kMapRows; ++j) {
+        const uint32_t c = (uint32_t)__popc(m[j]), inc = wave_incl_scan(c);
+        e[j] = inc - c;
+        if (lane == 63) s_part[j * (kBlock / 64) + wave] = inc;
+    }
+    __syncthreads();
+    if (tid < 64) {
+        const uint32_t v = tid < kParts ? s_part[tid] : 0u, inc = wave_incl_scan(v);
+        if (tid < kParts) s_part[tid] = inc - v;
+        const uint32_t total = __shfl(inc, 63, 64);
+        if (tid == 0) s_base = total ? atomicAdd(count, total) : 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kMapRows; ++j) {
+        const uint64_t t0 = b0 + (uint64_t)j * kBlock * kMapTiles;
+        uint32_t at = s_base + s_part[j * (kBlock / 64) + wave] + e[j];
+        int32_t v[kMapTiles];
+#pragma unroll
+        for (int k = 0; k < kMapTiles; ++k) {
+            const bool on = (m[j] >> k) & 1u;
+            v[k] = on ? (int32_t)at : -1;
+            if (on) list[at++] = (int32_t)(t0 + k);
+        }
+        if (t0 + kMapTiles <= n) {
+            *reinterpret_cast<int4*>(tileIdx + t0) = make_int4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < kMapTiles; ++k)
+                if (t0 + k < n) tileIdx[t0 + k] = v[k];
+        }
+    }
+}
+
 // A level-0 tile is active when any group has triangles binned to it, or when
 // a terrain group with a texture has triangles up to three tiles above it
 // (the fill reaches 19 voxels down, VoxelizerKernels.cu 888-917).
-__global__ void k_activity0(VoxParams P, int ngroups, const int32_t* __restrict__ grpFill,
-                            const uint32_t* __restrict__ binStart, uint32_t* __restrict__ mark) {
-    uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= P.numTiles) return;
-    uint32_t tx_, ty_, tz;
-    tile_xyz(t, P.TG, tx_, ty_, tz);
-    uint32_t on = 0;
-    for (int g = 0; g < ngroups && !on; ++g) {
-        uint64_t key = (uint64_t)g * P.numTiles + t;
-        if (binStart[key + 1] > binStart[key]) on = 1;
-        if (!on && grpFill[g]) {
-            for (int q = 1; q <= kFillTiles; ++q) {
-                if (tz + q >= P.TG[2]) break;
-                uint64_t k2 = key + (uint64_t)q * P.TG[0] * P.TG[1];
-                if (binStart[k2 + 1] > binStart[k2]) { on = 1; break; }
+template <int kMapRows>
+__global__ __launch_bounds__(kBlock) void k_map_tiles0(VoxParams P, int ngroups,
+                                                       const int32_t* __restrict__ grpFill,
+                                                       const uint32_t* __restrict__ binStart,
+                                                       int32_t* __restrict__ tileIdx,
+                                                       int32_t* __restrict__ list,
+                                                       uint32_t* __restrict__ count) {
+    const uint64_t n = P.numTiles, slab = (uint64_t)P.TG[0] * P.TG[1];
+    map_tiles<kMapRows>(n, [&](uint64_t t0) {
+        uint32_t m = 0u;
+        for (int g = 0; g < ngroups; ++g) {
+            const uint32_t* start = binStart + (uint64_t)g * n;
+            const int up = grpFill[g] ? kFillTiles : 0;
+            for (int q = 0; q <= up; ++q) {
+                // (past the grid's last tile both ends are the group's end,
+                // an empty bin; a tile q above is past it when outside in z)
+                const uint64_t t = t0 + (uint64_t)q * slab;
+                uint32_t b[kMapTiles + 1];
+#pragma unroll
+                for (int k = 0; k <= kMapTiles; ++k) b[k] = start[t + k < n ? t + k : n];
+#pragma unroll
+                for (int k = 0; k < kMapTiles; ++k) m |= (b[k + 1] > b[k] ? 1u : 0u) << k;
             }
         }
-    }
-    mark[t] = on;
-}
-
-__global__ void k_compact(uint64_t n, const uint32_t* __restrict__ mark,
-                          const uint32_t* __restrict__ excl, int32_t* __restrict__ tileIdx,
-                          int32_t* __restrict__ list, uint32_t* __restrict__ count) {
-    uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) *count = excl[n];   // the scan's total: active tiles
-    if (t >= n) return;
-    if (mark[t]) {
-        uint32_t e = excl[t];
-        tileIdx[t] = (int32_t)e;
-        list[e] = (int32_t)t;
-    } else {
-        tileIdx[t] = -1;
-    }
+        return t0 + kMapTiles <= n ? m : m & ((1u << (n - t0)) - 1u);
+    }, tileIdx, list, count);
 }
 
 // Level-k tile (a,b,c) reads source voxels [16a, 16a+16), i.e. source tiles
 // 2a and 2a+1 on each axis, shifted by the tile's chunk offset (MipShift,
 // whole tile pairs) with several chunks.
-__global__ void k_mark_children(LevelMap src, LevelMap dst, MipShift shift,
-                                uint32_t* __restrict__ markDst) {
-    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= dst.numTiles) return;
-    uint32_t px, py, pz;
-    tile_xyz(t, dst.TG, px, py, pz);
-    const uint32_t ox = shift.cd[0] ? (px * kTile) / shift.cd[0] * shift.off[0] / kTile : 0u;
-    const uint32_t oy = shift.cd[1] ? (py * kTile) / shift.cd[1] * shift.off[1] / kTile : 0u;
-    const uint32_t oz = shift.cd[2] ? (pz * kTile) / shift.cd[2] * shift.off[2] / kTile : 0u;
-    uint32_t m = 0u;
+template <int kMapRows>
+__global__ __launch_bounds__(kBlock) void k_map_children(LevelMap src, LevelMap dst,
+                                                         MipShift shift,
+                                                         int32_t* __restrict__ tileIdx,
+                                                         int32_t* __restrict__ list,
+                                                         uint32_t* __restrict__ count) {
+    map_tiles<kMapRows>(dst.numTiles, [&](uint64_t t0) {
+        uint32_t m = 0u, px, py, pz;
+        tile_xyz(t0, dst, px, py, pz);
 #pragma unroll
-    for (uint32_t c = 0; c < 8u; ++c) {
-        const uint32_t x = 2 * px + ox + (c & 1u), y = 2 * py + oy + ((c >> 1) & 1u),
-                       z = 2 * pz + oz + (c >> 2);
-        if (x < src.TG[0] && y < src.TG[1] && z < src.TG[2] &&
-            src.tileIdx[((uint64_t)z * src.TG[1] + y) * src.TG[0] + x] >= 0)
-            m = 1u;
-    }
-    markDst[t] = m;
+        for (int k = 0; k < kMapTiles; ++k) {
+            const uint32_t ox = shift.cd[0] ? (px * kTile) / shift.cd[0] * shift.off[0] / kTile : 0u;
+            const uint32_t oy = shift.cd[1] ? (py * kTile) / shift.cd[1] * shift.off[1] / kTile : 0u;
+            const uint32_t oz = shift.cd[2] ? (pz * kTile) / shift.cd[2] * shift.off[2] / kTile : 0u;
+            // the eight loads independent of each other (one outside the
+            // source reads its tile 0 and does not count)
+            const bool in = t0 + k < dst.numTiles;
+            uint32_t on = 0u;
+#pragma unroll
+            for (uint32_t c = 0; c < 8u; ++c) {
+                const uint32_t x = 2 * px + ox + (c & 1u), y = 2 * py + oy + ((c >> 1) & 1u),
+                               z = 2 * pz + oz + (c >> 2);
+                const bool ok = in & (x < src.TG[0]) & (y < src.TG[1]) & (z < src.TG[2]);
+                const int32_t v = src.tileIdx[ok ? ((uint64_t)z * src.TG[1] + y) * src.TG[0] + x : 0u];
+                on |= (ok & (v >= 0)) ? 1u : 0u;
+            }
+            m |= on << k;
+            if (++px == dst.TG[0]) {
+                px = 0u;
+                if (++py == dst.TG[1]) { py = 0u; ++pz; }
+            }
+        }
+        return m;
+    }, tileIdx, list, count);
 }
 
 // ---------------------------------------------------------------------------
@@ -732,7 +817,7 @@ __device__ __forceinline__ uint32_t voxelize_unit(
     if ((uint32_t)tid < nt) {
         const uint4 wk = work[w0 + tid];
         uint32_t tx, ty, tz;
-        tile_xyz(wk.y, P.TG, tx, ty, tz);
+        tile_xyz(wk.y, P, tx, ty, tz);
         s_org[tid] = make_uint4(tx * kTile, ty * kTile, tz * kTile, wk.x);
         s_bin[tid] = make_uint2(wk.z, wk.w);
     }
@@ -1241,33 +1326,42 @@ __global__ __launch_bounds__(kBlock) void k_colour(
     }
 }
 
-// Tiles holding triangles of group g, appended in any order (the tiles are
-// independent, so the order does not change any result), each with what
-// the voxelize pass needs first: (active tile, tile index, first bin entry,
-// entries), so a workgroup starts a tile with one load.
-__global__ void k_group_tiles(VoxParams P, int g, uint64_t nActive, const int32_t* __restrict__ list,
-                              const uint32_t* __restrict__ binStart, uint4* __restrict__ work,
-                              uint32_t* __restrict__ workCount) {
-    const uint64_t a = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t tlin = 0, b0 = 0, b1 = 0;
-    if (a < nActive) {
-        tlin = (uint32_t)list[a];
-        const uint64_t key = (uint64_t)g * P.numTiles + tlin;
-        b0 = binStart[key];
-        b1 = binStart[key + 1];
+// Tiles holding triangles of each group of the set (blockIdx.y), appended in
+// any order (the tiles are independent, so the order does not change any
+// result), each with what the voxelize pass needs first: (active tile, tile
+// index, first bin entry, entries), so a workgroup starts a tile with one
+// load.  One atomic per 1024 active tiles (one per wave of 64 met the same
+// word 1,600 times on the 1024^3 workload: 20 us a group).
+__global__ __launch_bounds__(kBlock) void k_group_tiles(uint64_t numTiles, WorkSet W,
+                                                        uint64_t nActive,
+                                                        const int32_t* __restrict__ list,
+                                                        const uint32_t* __restrict__ binStart) {
+    __shared__ uint32_t s_w[kBlock / 64];
+    __shared__ uint32_t s_base;
+    const int i = (int)blockIdx.y;
+    const uint64_t a0 = (uint64_t)blockIdx.x * kBlock * kMapTiles + threadIdx.x;
+    uint4 e[kMapTiles];
+    uint32_t cnt = 0;
+#pragma unroll
+    for (int k = 0; k < kMapTiles; ++k) {
+        const uint64_t a = a0 + (uint64_t)k * kBlock;
+        e[k] = make_uint4((uint32_t)a, 0u, 0u, 0u);
+        if (a < nActive) {
+            e[k].y = (uint32_t)list[a];
+            const uint64_t key = (uint64_t)W.g[i] * numTiles + e[k].y;
+            e[k].z = binStart[key];
+            e[k].w = binStart[key + 1] - e[k].z;
+        }
+        cnt += e[k].w ? 1u : 0u;
     }
-    // one atomic per wave on the shared counter; lanes take consecutive slots
-    const bool take = a < nActive && b1 > b0;
-    const uint64_t mask = __ballot(take);
-    if (!mask) return;
-    const int lane = (int)(threadIdx.x & 63u);
-    const int leader = __ffsll((unsigned long long)mask) - 1;
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(workCount, (uint32_t)__popcll(mask));
-    base = __shfl(base, leader);
-    if (take)
-        work[base + (uint32_t)__popcll(mask & ((1ull << lane) - 1ull))] =
-            make_uint4((uint32_t)a, tlin, b0, b1 - b0);
+    uint32_t total;
+    uint32_t o = block_excl_scan(cnt, s_w, &total);
+    if (threadIdx.x == 0) s_base = total ? atomicAdd(W.count[i], total) : 0u;
+    __syncthreads();
+    o += s_base;
+#pragma unroll
+    for (int k = 0; k < kMapTiles; ++k)
+        if (e[k].w) W.work[i][o++] = e[k];
 }
 
 // ---------------------------------------------------------------------------
@@ -1301,7 +1395,7 @@ __global__ __launch_bounds__(kBlock) void k_fill(VoxParams P, int g, int init, u
     if (a >= nActive) return;   // whole waves
     const uint64_t tlin = (uint64_t)list[a];
     uint32_t tx_, ty_, tz;
-    tile_xyz(tlin, P.TG, tx_, ty_, tz);
+    tile_xyz(tlin, P, tx_, ty_, tz);
     const uint64_t slab = (uint64_t)P.TG[0] * P.TG[1];
     const uint32_t q = (uint32_t)lane >> 4, wd = (uint32_t)lane & 15u;
     int32_t idx = -1;
@@ -1396,7 +1490,7 @@ __global__ __launch_bounds__(kBlock) void k_mip(LevelMap src, LevelMap dst, MipS
     const uint64_t b = blockIdx.x;
     const uint64_t tlin = (uint64_t)listDst[b];
     uint32_t tx, ty, tz;
-    tile_xyz(tlin, dst.TG, tx, ty, tz);
+    tile_xyz(tlin, dst, tx, ty, tz);
     // source offsets of this tile's chunk (multiples of 16 voxels)
     const uint32_t ox = shift.cd[0] ? (tx * kTile) / shift.cd[0] * shift.off[0] : 0u;
     const uint32_t oy = shift.cd[1] ? (ty * kTile) / shift.cd[1] * shift.off[1] : 0u;
@@ -1526,7 +1620,7 @@ __global__ void k_mip_source_count(LevelMap src, LevelMap dst, uint64_t nActive,
     unsigned long long n = 0;
     if (b < nActive) {
         uint32_t tx, ty, tz;
-        tile_xyz((uint64_t)listDst[b], dst.TG, tx, ty, tz);
+        tile_xyz((uint64_t)listDst[b], dst, tx, ty, tz);
         for (uint32_t c = 0; c < 8u; ++c) {
             const uint32_t sx = 2 * tx + (c & 1u), sy = 2 * ty + ((c >> 1) & 1u), sz = 2 * tz + (c >> 2);
             if (sx >= src.TG[0] || sy >= src.TG[1] || sz >= src.TG[2]) continue;
@@ -1571,7 +1665,7 @@ __device__ __forceinline__ bool stored(const LevelMap& lm, uint64_t a, uint32_t 
 //                sample is non-zero and the brick reaches an inactive tile
 //                (whose voxels are all zero);
 //   node_compare per active tile: every voxel is read once and compared with
-//                the samples of the (at most 8) nodes whose bricks hold it.
+//                the samples of the nodes whose bricks hold it.
 __device__ __forceinline__ void node_sample_at(const LevelMap& lm, const uint32_t* __restrict__ col,
                                                uint32_t Rd, uint32_t Bx, uint32_t By, uint32_t Bz,
                                                uint32_t bx, uint32_t by, uint32_t bz,
@@ -1625,100 +1719,150 @@ __global__ void k_node_sample_all(SampleDepths S) {
                    n - S.start[d]);
 }
 
-// nodes n whose stored brick [n*B + b - 1, n*B + b + B] holds coordinate X
-__device__ __forceinline__ void node_span(uint32_t X, uint32_t B, uint32_t b, uint32_t Rd,
-                                          int32_t& lo, int32_t& hi) {
+// nodes n whose stored brick [n*B + b - 1, n*B + b + B] holds coordinate X:
+// (X - b - 1) / B <= n <= (X - b + 1) / B, rounded down (invB = 1 / B)
+__device__ __forceinline__ void node_span(uint32_t X, uint32_t B, float invB, uint32_t b,
+                                          uint32_t Rd, int32_t& lo, int32_t& hi) {
     const int32_t x = (int32_t)X - (int32_t)b;   // voxel relative to interior start
-    // n*B - 1 <= x <= n*B + B  <=>  (x - B)/B <= n <= (x + 1)/B
-    int32_t l = x - (int32_t)B;
-    lo = l >= 0 ? (l + (int32_t)B - 1) / (int32_t)B : -((-l) / (int32_t)B);
-    const int32_t h1 = x + 1;
-    hi = h1 >= 0 ? h1 / (int32_t)B : -((-h1 + (int32_t)B - 1) / (int32_t)B);
-    if (lo < 0) lo = 0;
+    lo = x >= 1 ? (int32_t)udiv_small((uint32_t)(x - 1), B, invB) : 0;
+    hi = x >= -1 ? (int32_t)udiv_small((uint32_t)(x + 1), B, invB) : -1;
     if (hi > (int32_t)Rd - 1) hi = (int32_t)Rd - 1;
 }
 
-// One wave per active tile, kBlock / 64 tiles per workgroup: lane l holds the
-// voxels (l & 7, l >> 3, z) for z = 0..7 in registers (eight coalesced
-// 256-byte loads). The wave then walks the nodes whose stored bricks reach
-// the tile (at most 8 for B >= 8): each node's sample is one wave-uniform
-// load, compared with the lane's voxels inside that brick, and one ballot
-// decides the node's flag. No LDS, no barrier.
+// One wave per active tile of any depth's level, kBlock / 64 tiles per
+// workgroup: lane l holds the voxels (l & 7, l >> 3, z) for z = 0..7 in
+// registers (eight coalesced 256-byte loads, of the stored voxels only).  The
+// voxels unequal to a value are then eight 64-bit masks, one per layer, that
+// every lane shares, and lane i decides the i-th node that reaches the tile
+// (27 at the most for B = 8, 8 for B = 16): its stored brick is a mask over x
+// and y and a range of layers.  One pass serves all nodes of one sample (most
+// samples are zero).  Nodes that another tile has flagged by then are left
+// out, and a tile all of whose nodes are is not read.  Bound by instruction
+// issue, scalar and vector alike: with the nodes one after the other in the
+// wave a 512^3 soup of 8^3 bricks took 498 us, so 122.
 constexpr int kNcTiles = kBlock / 64;
-__global__ __launch_bounds__(kBlock) void k_node_compare(
-    LevelMap lm, const int32_t* __restrict__ list, uint64_t nActive,
-    const uint32_t* __restrict__ col, uint32_t Rd, uint32_t Bx, uint32_t By, uint32_t Bz,
-    uint32_t bx, uint32_t by, uint32_t bz, uint32_t xLimit, const uint32_t* __restrict__ cc,
-    uint32_t* __restrict__ flag) {
+__global__ __launch_bounds__(kBlock) void k_node_compare_all(CompareDepths C) {
     const int lane = (int)(threadIdx.x & 63u);
-    const uint64_t a = (uint64_t)blockIdx.x * kNcTiles + (threadIdx.x >> 6);
-    if (a >= nActive) return;   // whole waves
+    const uint64_t w =
+        (uint64_t)blockIdx.x * kNcTiles + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const SampleDepths& S = C.S;
+    int d = S.L - 1;                       // deepest first
+    while (d >= 0 && w >= C.tileEnd[d]) --d;
+    if (d < 0) return;                     // whole waves
+    const uint64_t a = w - (d + 1 < S.L ? C.tileEnd[d + 1] : 0u);
+    const LevelMap& lm = S.lm[d];
+    const uint32_t Rd = S.Rd[d];
+    const uint32_t* __restrict__ cc = S.cc[d];
+    uint32_t* __restrict__ flag = S.flag[d];
     uint32_t tx, ty, tz;
-    tile_xyz((uint64_t)list[a], lm.TG, tx, ty, tz);
-    const uint32_t B3[3] = {Bx, By, Bz}, b3[3] = {bx, by, bz};
+    tile_xyz((uint64_t)C.list[d][a], lm, tx, ty, tz);
+    const uint32_t B3[3] = {S.B[0], S.B[1], S.B[2]};
+    const uint32_t b3[3] = {S.border[d][0], S.border[d][1], S.border[d][2]};
     const uint32_t o3[3] = {tx * kTile, ty * kTile, tz * kTile};
+    // voxels of the tile that the comparison examines, per axis
+    const uint32_t lim[3] = {min(S.xLimit[d], lm.dims[0]), lm.dims[1], lm.dims[2]};
     // nodes whose bricks reach the tile, per axis
     int32_t blo[3], bhi[3];
 #pragma unroll
     for (int ax = 0; ax < 3; ++ax) {
         int32_t lo, hi;
-        node_span(o3[ax], B3[ax], b3[ax], Rd, blo[ax], hi);
-        node_span(o3[ax] + kTile - 1, B3[ax], b3[ax], Rd, lo, bhi[ax]);
+        node_span(o3[ax], B3[ax], S.invB[ax], b3[ax], Rd, blo[ax], hi);
+        node_span(o3[ax] + kTile - 1, B3[ax], S.invB[ax], b3[ax], Rd, lo, bhi[ax]);
     }
     if (blo[0] > bhi[0] || blo[1] > bhi[1] || blo[2] > bhi[2]) return;
-    const uint32_t X = o3[0] + ((uint32_t)lane & 7u), Y = o3[1] + ((uint32_t)lane >> 3);
-    const bool colOk = X < xLimit && X < lm.dims[0] && Y < lm.dims[1];
-    // z layers inside the level
-    uint32_t zIn = 0u;
+    const uint32_t ex = (uint32_t)(bhi[0] - blo[0] + 1), ey = (uint32_t)(bhi[1] - blo[1] + 1);
+    const uint32_t nn = ex * ey * (uint32_t)(bhi[2] - blo[2] + 1);
+    const float invEx = __builtin_amdgcn_rcpf((float)ex), invEy = __builtin_amdgcn_rcpf((float)ey);
     uint32_t c[kTile];
-    const uint32_t* tc = col + a * kTileVox + (uint64_t)lane;
-    // stored-voxel words of the tile (level 0), lane w < 16 holding word w
-    uint32_t dw = 0xffffffffu;
-    if (lm.defOcc && lane < kTileWords)
-        dw = lm.defOcc[a * kTileWords + lane] | lm.defFill[a * kTileWords + lane];
+    bool read = false;                     // the tile's voxels are in c
+    for (uint32_t i0 = 0; i0 < nn; i0 += 64u) {
+        const uint32_t i = i0 + (uint32_t)lane;
+        const uint32_t q = udiv_small(i, ex, invEx), kz = udiv_small(q, ey, invEy);
+        const int32_t k3[3] = {blo[0] + (int32_t)(i - q * ex), blo[1] + (int32_t)(q - kz * ey),
+                               blo[2] + (int32_t)kz};
+        const uint64_t n = ((uint64_t)k3[2] * Rd + (uint32_t)k3[1]) * Rd + (uint32_t)k3[0];
+        bool open = i < nn;
+        uint32_t smp = 0u;
+        if (open) {
+            smp = cc[n];
+            open = flag[n] == 0u;
+        }
+        uint64_t pend = __ballot(open);
+        if (!pend) continue;
+        if (!read) {
+            read = true;
+            const uint32_t* tc = S.col[d] + a * kTileVox + (uint64_t)lane;
+            // stored-voxel words of the tile (level 0), lane w < 16 holding word w
+            uint32_t dw = 0xffffffffu;
+            if (lm.defOcc && lane < kTileWords)
+                dw = lm.defOcc[a * kTileWords + lane] | lm.defFill[a * kTileWords + lane];
 #pragma unroll
-    for (int lz = 0; lz < kTile; ++lz) {
-        bool st = true;
-        if (lm.defOcc)
-            st = (((uint32_t)__shfl((int)dw, lz * 2 + (lane >> 5)) >> (lane & 31)) & 1u) != 0u;
-        const uint32_t cv = tc[lz * 64];   // every voxel of the tile is allocated
-        c[lz] = st ? cv : 0u;
-        if (o3[2] + (uint32_t)lz < lm.dims[2]) zIn |= 1u << lz;
-    }
-    for (int32_t nz = blo[2]; nz <= bhi[2]; ++nz) {
-        // stored brick of node n on an axis: [n*B + b - 1, n*B + b + B]
-        const int32_t z0 = nz * (int32_t)Bz + (int32_t)bz - 1 - (int32_t)o3[2];
-        const int32_t z1 = z0 + (int32_t)Bz + 1;
-        uint32_t zm = 0u;
-#pragma unroll
-        for (int lz = 0; lz < kTile; ++lz)
-            if (lz >= z0 && lz <= z1) zm |= 1u << lz;
-        zm &= zIn;
-        if (!zm) continue;
-        for (int32_t ny = blo[1]; ny <= bhi[1]; ++ny) {
-            const int32_t y0 = ny * (int32_t)By + (int32_t)by - 1;
-            const bool inY = (int32_t)Y >= y0 && (int32_t)Y <= y0 + (int32_t)By + 1;
-            for (int32_t nx = blo[0]; nx <= bhi[0]; ++nx) {
-                const int32_t x0 = nx * (int32_t)Bx + (int32_t)bx - 1;
-                const bool inX = (int32_t)X >= x0 && (int32_t)X <= x0 + (int32_t)Bx + 1;
-                const uint64_t n = ((uint64_t)nz * Rd + ny) * Rd + nx;
-                const uint32_t s = cc[n];
-                uint32_t ne = 0u;
-#pragma unroll
-                for (int lz = 0; lz < kTile; ++lz) ne |= (c[lz] != s ? 1u : 0u) << lz;
-                const bool d = colOk && inX && inY && (ne & zm) != 0u;
-                if (__ballot(d) && lane == 0) flag[n] = 1u;
+            for (int lz = 0; lz < kTile; ++lz) {
+                bool st = true;
+                if (lm.defOcc)
+                    st = (((uint32_t)__shfl((int)dw, lz * 2 + (lane >> 5)) >> (lane & 31)) & 1u) != 0u;
+                c[lz] = 0u;
+                if (st) c[lz] = tc[lz * 64];
             }
         }
+        // the lane's node in the tile: bits [v0, v1] of each axis's eight
+        // voxels are those of its stored brick [k*B + b - 1, k*B + b + B]
+        // inside the limit
+        uint32_t m3[3];
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) {
+            const int32_t o = (int32_t)o3[ax];
+            int32_t v0 = k3[ax] * (int32_t)B3[ax] + (int32_t)b3[ax] - 1 - o;
+            int32_t v1 = min(v0 + (int32_t)B3[ax] + 1, (int32_t)lim[ax] - 1 - o);
+            v0 = max(v0, 0);
+            v1 = min(v1, kTile - 1);
+            m3[ax] = v0 <= v1 ? ((2u << v1) - 1u) & ~((1u << v0) - 1u) : 0u;
+        }
+        // rows 0..3 and 4..7 of a layer: bit y of the y mask to row y's byte
+        const uint32_t row = m3[0] * 0x01010101u;
+        const uint32_t xy0 = row & ((((m3[1] & 15u) * 0x00204081u) & 0x01010101u) * 255u);
+        const uint32_t xy1 = row & ((((m3[1] >> 4) * 0x00204081u) & 0x01010101u) * 255u);
+        bool hit = false;
+        while (pend) {
+            const int l = __ffsll((unsigned long long)pend) - 1;
+            const uint32_t s = (uint32_t)__builtin_amdgcn_readlane((int)smp, l);
+            const bool same = open && smp == s;
+            uint32_t ne0 = 0u, ne1 = 0u;
+#pragma unroll
+            for (int lz = 0; lz < kTile; ++lz) {
+                const uint64_t u = __ballot(c[lz] != s);
+                const bool in = (m3[2] >> lz) & 1u;
+                ne0 |= in ? (uint32_t)u : 0u;
+                ne1 |= in ? (uint32_t)(u >> 32) : 0u;
+            }
+            if (same) hit = ((ne0 & xy0) | (ne1 & xy1)) != 0u;
+            pend &= ~__ballot(same);
+        }
+        if (hit) flag[n] = 1u;
     }
 }
 
-// out[d] = excl[offs[d + 1]] - excl[offs[d]]: the flags set in each range of
-// an exclusive scan's input.
-__global__ void k_range_counts(const uint32_t* __restrict__ excl, RangeOffs offs, int n,
-                               uint32_t* __restrict__ out) {
+// What the host reads between the tile maps and their buffers, into pinned
+// memory: active tiles per level, then the bin entries.
+__global__ void k_map_counts(const uint32_t* __restrict__ tiles, int n,
+                             const uint32_t* __restrict__ pairs, uint32_t* __restrict__ host) {
+    const int k = (int)threadIdx.x;
+    if (k < n) host[k] = tiles[k];
+    if (k == n) host[kMaxLevels] = *pairs;
+}
+
+// What the host reads between node typing and the brick arrays, into pinned
+// memory (a kernel's store costs less than copies of a few bytes): the brick
+// counts of the depths (the flags set in each range of the scan's input, or
+// counts as given), then the overlap tests and the scans' time-out word.
+__global__ void k_generate_counts(const uint32_t* __restrict__ excl, RangeOffs offs,
+                                  const uint32_t* __restrict__ counts, int n,
+                                  const uint32_t* __restrict__ sat,
+                                  const uint32_t* __restrict__ err, uint32_t* __restrict__ host) {
     const int d = (int)threadIdx.x;
-    if (d < n) out[d] = excl[offs.v[d + 1]] - excl[offs.v[d]];
+    if (d < n) host[d] = counts ? counts[d] : excl[offs.v[d + 1]] - excl[offs.v[d]];
+    if (d < 2) host[kMaxLevels + d] = sat[d];
+    if (d == 2) host[kMaxLevels + 2] = *err;
 }
 
 __global__ void k_brick_assign_all(uint64_t allNodes, const uint32_t* __restrict__ flag,
@@ -1841,24 +1985,63 @@ __global__ __launch_bounds__(kBlock) void k_brick_gather_all(GatherDepths G) {
                     w - G.start[e]);
 }
 
-// CollapseConstantBranches (Voxelizer.cu 701-774), one level at a time,
-// leaves first.
-__global__ void k_collapse(uint32_t Rd, int childIsLeaf, uint8_t* __restrict__ types,
-                           const uint8_t* __restrict__ childTypes) {
-    uint64_t n = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t nn = (uint64_t)Rd * Rd * Rd;
-    if (n >= nn) return;
+// CollapseConstantBranches (Voxelizer.cu 701-774), leaves first, every depth
+// in one launch: a workgroup takes the subtree under one node kCollapse
+// depths above the leaves' parents, depth by depth; the last workgroup to end
+// (*ticket counts them, zero before the launch) goes on with the depths above.
+// A launch per depth took 2 to 3 us each, more than its work.
+constexpr int kCollapse = 3;
+// atRoot: the node is a subtree's root, whose mark another workgroup may
+// read; aboveRoot: its children are such roots.  Those go past the caches
+// (agent scope); the marks inside a subtree stay with its workgroup.
+__device__ __forceinline__ void collapse_node(uint32_t Rd, bool childIsLeaf, bool atRoot,
+                                              bool aboveRoot, uint8_t* __restrict__ types,
+                                              const uint8_t* childTypes, uint32_t x, uint32_t y,
+                                              uint32_t z) {
+    const uint64_t n = ((uint64_t)z * Rd + y) * Rd + x;
     if (types[n] != 0) return;
-    uint32_t x, y, z;
-    node_xyz(n, (uint32_t)(__ffs(Rd) - 1), x, y, z);
     const uint32_t Rc = Rd * 2;
     bool all = true;
+#pragma unroll
     for (uint32_t c = 0; c < 8; ++c) {
         const uint32_t cx = 2 * x + (c & 1u), cy = 2 * y + ((c >> 1) & 1u), cz = 2 * z + (c >> 2);
-        const uint8_t t = childTypes[((uint64_t)cz * Rc + cy) * Rc + cx];
+        const uint8_t* q = childTypes + ((uint64_t)cz * Rc + cy) * Rc + cx;
+        const uint8_t t =
+            aboveRoot ? __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *q;
         all = all && (childIsLeaf ? (t == 0) : (t == 2));
     }
-    if (all) types[n] = 2;
+    if (!all) return;
+    if (atRoot)
+        __hip_atomic_store(types + n, (uint8_t)2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else
+        types[n] = 2;
+}
+__global__ __launch_bounds__(kBlock) void k_collapse_all(DepthOut D, uint32_t* __restrict__ ticket) {
+    __shared__ bool s_last;
+    const int top = D.L - 2 - kCollapse > 0 ? D.L - 2 - kCollapse : 0;   // the subtrees' roots
+    uint32_t rx, ry, rz;
+    node_xyz(blockIdx.x, (uint32_t)top, rx, ry, rz);
+    for (int d = D.L - 2; d >= top; --d) {
+        const uint32_t k = (uint32_t)(d - top), m = (1u << k) - 1u;   // 2^k nodes an axis here
+        for (uint32_t i = threadIdx.x; i < 1u << (3 * k); i += kBlock)
+            collapse_node(1u << d, d + 1 == D.L - 1, d == top, false, D.types[d], D.types[d + 1],
+                          (rx << k) + (i & m), (ry << k) + ((i >> k) & m), (rz << k) + (i >> (2 * k)));
+        __syncthreads();   // (and its release and acquire at workgroup scope)
+    }
+    if (top == 0) return;
+    if (threadIdx.x == 0) {
+        wait_memory();     // this thread wrote the root's mark
+        s_last = atomicAdd(ticket, 1u) == gridDim.x - 1u;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    for (int d = top - 1; d >= 0; --d) {
+        const uint32_t m = (1u << d) - 1u;
+        for (uint32_t i = threadIdx.x; i < 1u << (3 * d); i += kBlock)
+            collapse_node(1u << d, false, false, d == top - 1, D.types[d], D.types[d + 1], i & m,
+                          (i >> d) & m, i >> (2 * d));
+        __syncthreads();
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void k_occupancy(VoxParams P, const int32_t* __restrict__ list,
@@ -1867,7 +2050,7 @@ __global__ __launch_bounds__(kBlock) void k_occupancy(VoxParams P, const int32_t
     const uint64_t a = blockIdx.x;
     const uint64_t tlin = (uint64_t)list[a];
     uint32_t tx, ty, tz;
-    tile_xyz(tlin, P.TG, tx, ty, tz);
+    tile_xyz(tlin, P, tx, ty, tz);
     if ((P.S[0] & 7u) == 0u) {
         // a tile row of 8 voxels is one byte of the bitmap
         const uint32_t r = threadIdx.x;
@@ -2279,8 +2462,9 @@ __global__ void k_copy_scattered(const uint4* __restrict__ src, uint4* __restric
     }
 }
 
+constexpr int kFillSegs = 6;
 struct FillSegs {
-    FillSeg s[4];
+    FillSeg s[kFillSegs];
     int k;
 };
 // Grid-stride over the words of all segments, one after the other.
@@ -2347,12 +2531,11 @@ __device__ __forceinline__ void chunk_src(uint32_t X, uint32_t Cd, uint32_t Cs, 
     s1 = i * Cs + min(2u * x + 1u, Cs - 1u);
 }
 
-__global__ void k_chunk_mark(LevelMap src, LevelMap dst, ChunkGeom cg, int ks, int kd,
-                             uint32_t* __restrict__ markDst) {
-    const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= dst.numTiles) return;
+__device__ __forceinline__ uint32_t chunk_tile_active(const LevelMap& src, const LevelMap& dst,
+                                                       const ChunkGeom& cg, int ks, int kd,
+                                                       uint64_t t) {
     uint32_t p[3];
-    tile_xyz(t, dst.TG, p[0], p[1], p[2]);
+    tile_xyz(t, dst, p[0], p[1], p[2]);
     // per axis the distinct source tiles the tile's voxels read (at most 8:
     // a voxel's two sources share a tile)
     uint32_t st[3][kTile], ns[3] = {0u, 0u, 0u};
@@ -2367,15 +2550,24 @@ __global__ void k_chunk_mark(LevelMap src, LevelMap dst, ChunkGeom cg, int ks, i
             if (ns[a] == 0u || st[a][ns[a] - 1u] != tt) st[a][ns[a]++] = tt;
         }
     }
-    uint32_t m = 0u;
-    for (uint32_t k = 0; k < ns[2] && !m; ++k)
-        for (uint32_t j = 0; j < ns[1] && !m; ++j)
+    for (uint32_t k = 0; k < ns[2]; ++k)
+        for (uint32_t j = 0; j < ns[1]; ++j)
             for (uint32_t i = 0; i < ns[0]; ++i)
-                if (src.tileIdx[((uint64_t)st[2][k] * src.TG[1] + st[1][j]) * src.TG[0] + st[0][i]] >= 0) {
-                    m = 1u;
-                    break;
-                }
-    markDst[t] = m;
+                if (src.tileIdx[((uint64_t)st[2][k] * src.TG[1] + st[1][j]) * src.TG[0] + st[0][i]] >= 0)
+                    return 1u;
+    return 0u;
+}
+__global__ __launch_bounds__(kBlock) void k_chunk_map(LevelMap src, LevelMap dst, ChunkGeom cg,
+                                                      int ks, int kd,
+                                                      int32_t* __restrict__ tileIdx,
+                                                      int32_t* __restrict__ list,
+                                                      uint32_t* __restrict__ count) {
+    map_tiles<1>(dst.numTiles, [&](uint64_t t0) {
+        uint32_t m = 0u;
+        for (int k = 0; k < kMapTiles; ++k)
+            if (t0 + k < dst.numTiles && chunk_tile_active(src, dst, cg, ks, kd, t0 + k)) m |= 1u << k;
+        return m;
+    }, tileIdx, list, count);
 }
 
 // ComputeVoxelMipMap8 (VoxelizerKernels.cu 1520-1663) inside each chunk:
@@ -2392,7 +2584,7 @@ __global__ __launch_bounds__(kBlock) void k_chunk_mip(LevelMap src, LevelMap dst
     const uint64_t b = blockIdx.x;
     const uint64_t tlin = (uint64_t)listDst[b];
     uint32_t tx, ty, tz;
-    tile_xyz(tlin, dst.TG, tx, ty, tz);
+    tile_xyz(tlin, dst, tx, ty, tz);
     __shared__ float s_inv255[256];
     fill_inv255(s_inv255);
     __syncthreads();
@@ -2808,7 +3000,7 @@ void launch_fill_segs(hipStream_t st, const FillSeg* segs, int nseg) {
     FillSegs F{};
     uint64_t total = 0;
     F.k = 0;
-    for (int i = 0; i < nseg && F.k < 4; ++i) {
+    for (int i = 0; i < nseg && F.k < kFillSegs; ++i) {
         if (segs[i].n == 0 || !segs[i].p) continue;
         F.s[F.k++] = segs[i];
         total += (segs[i].n + 3) / 4;
@@ -2863,26 +3055,24 @@ void launch_scatter(hipStream_t st, const VoxParams& P, const std::vector<GroupA
                                                                binTri);
                       });
 }
-void launch_activity0(hipStream_t st, const VoxParams& P, int ngroups, const int32_t* grpFill,
-                      const uint32_t* binStart, uint32_t* mark) {
-    k_activity0<<<grid_for(P.numTiles, kBlock), kBlock, 0, st>>>(P, ngroups, grpFill, binStart, mark);
+void launch_map_tiles0(hipStream_t st, const VoxParams& P, int ngroups, const int32_t* grpFill,
+                       const uint32_t* binStart, int32_t* tileIdx, int32_t* list, uint32_t* count) {
+    if (P.numTiles <= kMapSmall)
+        k_map_tiles0<1><<<grid_for(P.numTiles, kMapBlock), kBlock, 0, st>>>(
+            P, ngroups, grpFill, binStart, tileIdx, list, count);
+    else
+        k_map_tiles0<4><<<grid_for(P.numTiles, 4 * kMapBlock), kBlock, 0, st>>>(
+            P, ngroups, grpFill, binStart, tileIdx, list, count);
 }
-void launch_compact(hipStream_t st, uint64_t n, const uint32_t* mark, const uint32_t* excl,
-                    int32_t* tileIdx, int32_t* list, uint32_t* count) {
-    if (n == 0) {
-        launch_fill_u32(st, count, 1, 0u);
-        return;
-    }
-    k_compact<<<grid_for(n, kBlock), kBlock, 0, st>>>(n, mark, excl, tileIdx, list, count);
-}
-void launch_mark_children(hipStream_t st, const LevelMap& src, const LevelMap& dst,
-                          uint32_t* markDst) {
-    launch_mark_children_shifted(st, src, dst, MipShift{}, markDst);
-}
-void launch_mark_children_shifted(hipStream_t st, const LevelMap& src, const LevelMap& dst,
-                                  const MipShift& shift, uint32_t* markDst) {
+void launch_map_children(hipStream_t st, const LevelMap& src, const LevelMap& dst,
+                         const MipShift& shift, int32_t* tileIdx, int32_t* list, uint32_t* count) {
     if (dst.numTiles == 0) return;
-    k_mark_children<<<grid_for(dst.numTiles, kBlock), kBlock, 0, st>>>(src, dst, shift, markDst);
+    if (dst.numTiles <= kMapSmall)
+        k_map_children<1><<<grid_for(dst.numTiles, kMapBlock), kBlock, 0, st>>>(
+            src, dst, shift, tileIdx, list, count);
+    else
+        k_map_children<4><<<grid_for(dst.numTiles, 4 * kMapBlock), kBlock, 0, st>>>(
+            src, dst, shift, tileIdx, list, count);
 }
 void launch_voxelize(hipStream_t st, const VoxParams& P, const GroupArgs& G, int g, int init,
                      uint64_t nActive, const int32_t* list, const float* verts,
@@ -2926,14 +3116,11 @@ void launch_voxelize_batch(hipStream_t st, const VoxUnitJob* jobs, uint32_t njob
     k_voxelize_batch_units<<<1, kBlock, 0, st>>>(jobs, njobs, unitStart, queue);
     k_voxelize_batch<<<blocks, kBlock, 0, st>>>(jobs, njobs, unitStart, queue);
 }
-void launch_group_tiles(hipStream_t st, const VoxParams& P, int g, uint64_t nActive,
-                        const int32_t* list, const uint32_t* binStart, uint4* work,
-                        uint32_t* workCount, uint32_t* recCount) {
-    const FillSeg z[2] = {{workCount, 1, 0u}, {recCount, kRecSegs, 0u}};
-    launch_fill_segs(st, z, 2);
-    if (nActive == 0) return;
-    k_group_tiles<<<grid_for(nActive, kBlock), kBlock, 0, st>>>(P, g, nActive, list, binStart,
-                                                                 work, workCount);
+void launch_group_tiles(hipStream_t st, const VoxParams& P, const WorkSet& W, uint64_t nActive,
+                        const int32_t* list, const uint32_t* binStart) {
+    if (nActive == 0 || W.n == 0) return;
+    k_group_tiles<<<dim3(grid_for(nActive, kBlock * kMapTiles), (unsigned)W.n), kBlock, 0, st>>>(
+        P.numTiles, W, nActive, list, binStart);
 }
 void launch_colour(hipStream_t st, const VoxParams& P, const GroupArgs& G, int init,
                    uint64_t nActive, const uint4* rec, const uint32_t* recCount,
@@ -2986,20 +3173,22 @@ void launch_node_sample_all(hipStream_t st, const SampleDepths& S) {
     if (S.L <= 0 || S.start[S.L] == 0) return;
     k_node_sample_all<<<grid_for(S.start[S.L], kBlock), kBlock, 0, st>>>(S);
 }
-void launch_node_compare(hipStream_t st, const LevelMap& lm, uint64_t nActive, const int32_t* list,
-                         const uint32_t* col, uint32_t Rd, const uint32_t B[3],
-                         const uint32_t border[3], uint32_t xLimit, uint32_t* cc, uint32_t* flag) {
-    if (nActive == 0) return;
-    k_node_compare<<<(unsigned)((nActive + kNcTiles - 1) / kNcTiles), kBlock, 0, st>>>(
-        lm, list, nActive, col, Rd, B[0], B[1], B[2], border[0], border[1], border[2], xLimit, cc,
-        flag);
+void launch_node_compare_all(hipStream_t st, const CompareDepths& C) {
+    const uint64_t n = C.S.L > 0 ? C.tileEnd[0] : 0u;
+    if (n == 0) return;
+    k_node_compare_all<<<grid_for(n, kNcTiles), kBlock, 0, st>>>(C);
 }
-void launch_range_counts(hipStream_t st, const uint32_t* excl, const uint64_t* offs, int n,
-                         uint32_t* out) {
-    if (n <= 0) return;
+void launch_map_counts(hipStream_t st, const uint32_t* tiles, int n, const uint32_t* pairs,
+                       uint32_t* host) {
+    k_map_counts<<<1, 64, 0, st>>>(tiles, n < kMaxLevels ? n : kMaxLevels, pairs, host);
+}
+void launch_generate_counts(hipStream_t st, const uint32_t* excl, const uint64_t* offs,
+                            const uint32_t* counts, int n, const uint32_t* sat,
+                            const uint32_t* err, uint32_t* host) {
     RangeOffs o{};
-    for (int d = 0; d <= n && d <= kMaxLevels; ++d) o.v[d] = offs[d];
-    k_range_counts<<<1, 64, 0, st>>>(excl, o, n < kMaxLevels ? n : kMaxLevels, out);
+    for (int d = 0; offs && d <= n && d <= kMaxLevels; ++d) o.v[d] = offs[d];
+    k_generate_counts<<<1, 64, 0, st>>>(excl, o, counts, n < kMaxLevels ? n : kMaxLevels, sat, err,
+                                        host);
 }
 void launch_brick_assign_all(hipStream_t st, const uint32_t* flag, const uint32_t* excl,
                              const DepthOut& D) {
@@ -3012,10 +3201,10 @@ void launch_brick_gather_all(hipStream_t st, const GatherDepths& G) {
     if (G.n <= 0 || G.start[G.n] == 0) return;
     k_brick_gather_all<<<(unsigned)G.start[G.n], kBlock, 0, st>>>(G);
 }
-void launch_collapse(hipStream_t st, uint32_t Rd, int childIsLeaf, uint8_t* types,
-                     const uint8_t* childTypes) {
-    const uint64_t nn = (uint64_t)Rd * Rd * Rd;
-    k_collapse<<<grid_for(nn, kBlock), kBlock, 0, st>>>(Rd, childIsLeaf, types, childTypes);
+void launch_collapse_all(hipStream_t st, const DepthOut& D, uint32_t* ticket) {
+    if (D.L < 2) return;
+    const int top = std::max(0, D.L - 2 - kCollapse);
+    k_collapse_all<<<1u << (3 * top), kBlock, 0, st>>>(D, ticket);
 }
 void launch_occupancy(hipStream_t st, const VoxParams& P, uint64_t nActive, const int32_t* list,
                       const uint32_t* occ, uint32_t* bitmap) {
@@ -3075,10 +3264,11 @@ void launch_mip_source_count(hipStream_t st, const LevelMap& src, const LevelMap
                                                                     out);
 }
 
-void launch_chunk_mark(hipStream_t st, const LevelMap& src, const LevelMap& dst,
-                       const ChunkGeom& cg, int ks, int kd, uint32_t* markDst) {
+void launch_chunk_map(hipStream_t st, const LevelMap& src, const LevelMap& dst, const ChunkGeom& cg,
+                      int ks, int kd, int32_t* tileIdx, int32_t* list, uint32_t* count) {
     if (dst.numTiles == 0) return;
-    k_chunk_mark<<<grid_for(dst.numTiles, kBlock), kBlock, 0, st>>>(src, dst, cg, ks, kd, markDst);
+    k_chunk_map<<<grid_for(dst.numTiles, kMapBlock), kBlock, 0, st>>>(src, dst, cg, ks, kd, tileIdx,
+                                                                      list, count);
 }
 void launch_chunk_mip(hipStream_t st, const LevelMap& src, const LevelMap& dst,
                       const ChunkGeom& cg, int ks, int kd, uint64_t nActive,
