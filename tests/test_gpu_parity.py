@@ -102,3 +102,10 @@ def test_brick_wider_than_the_gather_tile_table():
     # B = 64: a stored brick of 66^3 spans 9 tiles per axis, more than the
     # brick gather stages in LDS (6), so it reads the tile map directly
     _check(scenes.scene_terrain_n(64, 128, 64))
+
+
+# bricks of one wave's batch (10 voxels an axis), one voxel more, the largest
+# whose tiles are staged (39) and the next, which reads the maps per voxel
+@pytest.mark.parametrize("N,B", [(32, 8), (36, 9), (78, 39), (80, 40)])
+def test_brick_sizes_at_the_gather_s_edges(N, B):
+    _check(scenes.scene_mixed(seed=21, N=N, B=B))
