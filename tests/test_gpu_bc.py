@@ -36,3 +36,24 @@ def test_compressed_bricks_match_oracle(scene, tmp_path):
         assert total > 0
     finally:
         vz.close()
+
+
+@pytest.mark.parametrize("B", [(3,) * 3, (5,) * 3, (6,) * 3, (7,) * 3, (1022, 2, 2), (1026, 2, 2)],
+                         ids=str)
+def test_block_rows_of_every_width(B):
+    """Rows of 5, 7, 8 and 9 texels: single texels where rows are odd, pairs
+    where they are even, the edge texel repeated 3, 1, 0 and 3 times; the widest
+    rows that a workgroup stages, and wider ones."""
+    cube = scenes.scene_mixed(seed=3, N=B[-1] * 8, B=B[-1])
+    scene = scenes.Scene(meshes=cube.meshes, N=tuple(8 * b for b in B), B=B, name=f"rows_{B[0]}")
+    print(f"[bc] {scene.name}", flush=True)
+    vz = voxelize_scene(scene, options=VOX_OPT_MIP_CHAIN, compressed=True)
+    try:
+        comp, total = vz.compressed(), 0
+        for d, tr in enumerate(vz.result()["tree"]):
+            oc, on = oracle.bc_encode_bricks(tr["bcol"], tr["bnrm"], tuple(b + 2 for b in B))
+            assert (comp[d][0] == oc).all() and (comp[d][1] == on).all(), f"depth {d}"
+            total += tr["nb"]
+        assert total > 0
+    finally:
+        vz.close()
