@@ -89,3 +89,11 @@ def test_terrain_256_b8_mip_chain():
 def test_full_octree_generator_512_chunks(chunk):
     ref = _check(scenes.scene_full_octree(cells=512, N=512, B=16), chunk)
     assert sum(t["nb"] for t in ref.tree) > 0
+
+
+@pytest.mark.parametrize("N,B,chunk", [(8, 2, 4), (128, 64, 32), (132, 66, 44), (40, 10, 24)])
+def test_node_windows_at_the_tables_edges(N, B, chunk):
+    """The smallest bricks and chunks; windows of 66 voxels, 10 tiles and 4
+    chunks an axis, which fill the tables of a wave; wider ones; extents that
+    end inside a tile."""
+    _check(scenes.scene_mixed(seed=3, N=N, B=B), chunk)

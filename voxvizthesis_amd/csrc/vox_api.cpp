@@ -284,9 +284,11 @@ inline uint64_t trunc_u(float f) {
 }
 
 // Words of h->counters, zeroed together by the setup pass: active tiles per
-// level (first), with several chunks the bricks per depth, where the scans of a generate report a wait
-// that timed out, and the collapse's ticket.
-constexpr uint32_t kChunkBricksWord = 64, kScanErrWord = 128, kCollapseWord = 129,
+// level (first), with several chunks the bricks per depth and in all and the
+// nodes over active tiles, where the scans of a generate report a wait that
+// timed out, and the collapse's ticket.
+constexpr uint32_t kChunkBricksWord = 64, kChunkBricksAllWord = 126,
+                   kChunkNodesWord = 127, kScanErrWord = 128, kCollapseWord = 129,
                    kCounterWords = 160;
 // Words of h->pin: what launch_map_counts and launch_generate_counts leave.
 constexpr uint32_t kPinTiles = 0, kPinCounts = 32;
@@ -595,19 +597,17 @@ int vox_allocate_voxel_memory(vox_ctx* h) {
                         q.push_back({n[0], n[1], n[2]});
                     }
         }
-        uint64_t maxNodes = 0;
-        for (int d = 0; d < h->L; ++d) maxNodes = std::max(maxNodes, h->tree[d].nodes);
         if (!h->chunkRank.ensure(rank.size() * 4, h->err, "chunk ranks") ||
             !h->check(hipMemcpy(h->chunkRank.p, rank.data(), rank.size() * 4, hipMemcpyHostToDevice),
                       "chunk ranks") ||
             !h->keysA.ensure(h->allNodes * 8, h->err, "brick keys") ||
-            !h->keysB.ensure(maxNodes * 8, h->err, "brick keys") ||
+            !h->keysB.ensure(h->allNodes * 8, h->err, "brick keys") ||
             !h->nodesA.ensure(h->allNodes * 4, h->err, "brick nodes") ||
-            !h->nodesB.ensure(maxNodes * 4, h->err, "brick nodes"))
+            !h->nodesB.ensure(h->allNodes * 4, h->err, "brick nodes"))
             return 0;
         size_t tmpBytes = 0;
         if (!h->check(chunk_sort_pairs(h->st, nullptr, &tmpBytes, nullptr, nullptr, nullptr, nullptr,
-                                       (uint32_t)maxNodes, 64),
+                                       (uint32_t)h->allNodes, 64),
                       "sort size") ||
             !h->sortTmp.ensure(tmpBytes, h->err, "sort scratch"))
             return 0;
@@ -1192,57 +1192,57 @@ int gen_back(vox_ctx* h, const char* out_dir, int binary) {
         // Several chunks: per-chunk samples and types OR-ed over chunks, and
         // bricks numbered in the order the brick writer writes them (the
         // chunk that completes a brick, inside one chunk before across
-        // chunks, node order), by a key sort per depth.
+        // chunks, node order), by one key sort.
         const ChunkGeom cg = chunkGeom(h);
         uint32_t* bcount = ctr + kChunkBricksWord;
+        uint32_t rankBits = 0, depthBits = 0;
+        while ((1ull << rankBits) < (uint64_t)h->nc[0] * h->nc[1] * h->nc[2]) ++rankBits;
+        while ((1 << depthBits) < L) ++depthBits;
+        const uint32_t depthShift = 3u * (uint32_t)(L - 1) + 1u + rankBits;
         h->run("node_type", [&] {
-            launch_chunk_node_type(st, S, cg);
-            for (int d = L - 1; d >= 0; --d) {
-                DepthBufs& t = h->tree[d];
-                launch_chunk_brick_keys(st, S.flag[d], cg, L - 1 - d, t.Rd, h->B, S.border[d],
-                                        h->keysA.as<unsigned long long>() + t.off,
-                                        h->nodesA.as<uint32_t>() + t.off, bcount + d);
-            }
+            launch_chunk_node_type(st, S, cg, h->nodesB.as<uint32_t>(), ctr + kChunkNodesWord);
+            launch_chunk_brick_keys(st, S, cg, depthShift, h->keysA.as<unsigned long long>(),
+                                    h->nodesA.as<uint32_t>(), bcount, ctr + kChunkBricksAllWord);
         });
         counts(nullptr, nullptr, bcount);
         occupancy();
         if (!h->check(hipStreamSynchronize(st), "node typing")) return 0;
         std::memcpy(nb, h->pin + kPinCounts, 4 * L);
-        uint32_t rankBits = 0;
-        while ((1ull << rankBits) < (uint64_t)h->nc[0] * h->nc[1] * h->nc[2]) ++rankBits;
+        RangeOffs first{};
         for (int d = 0; d < L; ++d) {
             DepthBufs& t = h->tree[d];
             t.bricks = nb[d];
             h->stats.bricks_total += nb[d];
+            first.v[d + 1] = first.v[d] + nb[d];
             if (!t.brickNode.ensure((uint64_t)nb[d] * 4, h->err, "brick nodes") ||
                 !t.bcol.ensure((uint64_t)nb[d] * bvox * 4, h->err, "brick colours") ||
                 !t.bnrm.ensure((uint64_t)nb[d] * bvox * 4, h->err, "brick normals"))
                 return 0;
-            if (nb[d] > 1) {
-                const int bits = (int)(3 * d + 1 + rankBits);
-                size_t tb = 0;
-                if (!h->check(chunk_sort_pairs(st, nullptr, &tb, nullptr, nullptr, nullptr, nullptr,
-                                               nb[d], bits),
-                              "sort size") ||
-                    !h->sortTmp.ensure(tb, h->err, "sort scratch"))
-                    return 0;
-                tb = h->sortTmp.cap;
-                if (!h->check(chunk_sort_pairs(st, h->sortTmp.p, &tb,
-                                               h->keysA.as<unsigned long long>() + t.off,
-                                               h->keysB.as<unsigned long long>(),
-                                               h->nodesA.as<uint32_t>() + t.off,
-                                               h->nodesB.as<uint32_t>(), nb[d], bits),
-                              "brick order"))
-                    return 0;
-            }
-            const uint32_t* sorted =
-                nb[d] > 1 ? h->nodesB.as<uint32_t>() : h->nodesA.as<uint32_t>() + t.off;
-            h->run("brick_assign", [&] {
-                launch_chunk_brick_assign(st, t.nodes, S.flag[d], sorted, nb[d],
-                                          t.types.as<uint8_t>(), t.bidx.as<uint32_t>(),
-                                          t.brickNode.as<uint32_t>());
-            });
+            dout.brickNode[d] = t.brickNode.as<uint32_t>();
         }
+        const uint64_t bricks = first.v[L];
+        if (bricks > 1) {
+            const int bits = (int)(depthShift + depthBits);
+            size_t tb = 0;
+            if (!h->check(chunk_sort_pairs(st, nullptr, &tb, nullptr, nullptr, nullptr, nullptr,
+                                           bricks, bits),
+                          "sort size") ||
+                !h->sortTmp.ensure(tb, h->err, "sort scratch"))
+                return 0;
+            tb = h->sortTmp.cap;
+            if (!h->check(chunk_sort_pairs(st, h->sortTmp.p, &tb,
+                                           h->keysA.as<unsigned long long>(),
+                                           h->keysB.as<unsigned long long>(),
+                                           h->nodesA.as<uint32_t>(), h->nodesB.as<uint32_t>(),
+                                           bricks, bits),
+                          "brick order"))
+                return 0;
+        }
+        h->run("brick_assign", [&] {
+            launch_chunk_brick_assign(st, dout, first, h->nodeFlag.as<uint32_t>(),
+                                      bricks > 1 ? h->nodesB.as<uint32_t>()
+                                                 : h->nodesA.as<uint32_t>());
+        });
     } else {
         h->run("node_type", [&] {
             launch_node_sample_all(st, S);

@@ -400,25 +400,27 @@ void launch_chunk_mip(hipStream_t st, const LevelMap& src, const LevelMap& dst,
 // S.lm / S.col; S.cc, S.flag; nodes numbered from S.start[d]): flag[n] = 1
 // when a chunk the node's stored brick reaches holds a typed voxel of the
 // brick unequal to that chunk's sample; cc[n] = the sample of the last chunk
-// in visit order.
-void launch_chunk_node_type(hipStream_t st, const SampleDepths& S, const ChunkGeom& cg);
-// Brick keys of one depth: for each NON-CONST node whose stored brick lies
-// in processed chunks, key = (rank of the chunk that completes it << (1 +
-// 3d)) | (0 inside one chunk, 1 across chunks) << 3d | node; keys and nodes
-// appended at *count.
-void launch_chunk_brick_keys(hipStream_t st, const uint32_t* flag, const ChunkGeom& cg, int k,
-                             uint32_t Rd, const uint32_t B[3], const uint32_t border[3],
-                             unsigned long long* keys, uint32_t* nodes, uint32_t* count);
+// in visit order.  list (a word per node) and count (zero before) are
+// scratch.
+void launch_chunk_node_type(hipStream_t st, const SampleDepths& S, const ChunkGeom& cg,
+                            uint32_t* list, uint32_t* count);
+// Brick keys of every depth: for each NON-CONST node whose stored brick lies
+// in processed chunks, key = depth << depthShift | (rank of the chunk that
+// completes it << (1 + 3d)) | (0 inside one chunk, 1 across chunks) << 3d |
+// node; keys and nodes at *total on, in any order, count[d] of depth d.
+void launch_chunk_brick_keys(hipStream_t st, const SampleDepths& S, const ChunkGeom& cg,
+                             uint32_t depthShift, unsigned long long* keys, uint32_t* nodes,
+                             uint32_t* count, uint32_t* total);
 // Sort n (key, node) pairs by key (tmp: temporary storage; *tmpBytes is
 // its size on entry, or the size needed when tmp is null).
 hipError_t chunk_sort_pairs(hipStream_t st, void* tmp, size_t* tmpBytes,
                             const unsigned long long* keysIn, unsigned long long* keysOut,
                             const uint32_t* nodesIn, uint32_t* nodesOut, uint32_t n, int keyBits);
-// After the sort: types[node] = flag, bidx[node] = 0xffffffff, then
-// bidx[sorted[j]] = j and brickNode[j] = sorted[j].
-void launch_chunk_brick_assign(hipStream_t st, uint64_t nodes, const uint32_t* flag,
-                               const uint32_t* sorted, uint32_t nb, uint8_t* types,
-                               uint32_t* bidx, uint32_t* brickNode);
+// After the sort: types[node] = flag (of the nodes of every depth), bidx[node]
+// = 0xffffffff, then for brick j of depth d, the node n = sorted[first[d] + j]:
+// bidx[n] = j and brickNode[j] = n.
+void launch_chunk_brick_assign(hipStream_t st, const DepthOut& D, const RangeOffs& first,
+                               const uint32_t* flag, const uint32_t* sorted);
 // The whole bitmap (no clear needed) when S[0] is a multiple of 32 and a row
 // of tile indices fits in LDS; false (nothing launched) otherwise.
 bool launch_occupancy_rows(hipStream_t st, const VoxParams& P, const int32_t* tileIdx,

@@ -2679,7 +2679,7 @@ __device__ __forceinline__ uint32_t chunk_typed_limit(uint32_t Ck, uint32_t o, u
     if (tpb + o - bo > full) tpb = full - (o - bo) + 2u;
     if (tpb == 0u) return 0u;
     const uint64_t th = tpb < 8u ? tpb : 8u;
-    uint64_t nb = ((uint64_t)tpb + th - 1u) / th;
+    uint64_t nb = tpb < 8u ? 1u : ((uint64_t)tpb + 7u) >> 3;
     uint64_t cover = nb * th;
     if (xAxis && tpb > 128u) {
         nb >>= 1;
@@ -2690,38 +2690,106 @@ __device__ __forceinline__ uint32_t chunk_typed_limit(uint32_t Ck, uint32_t o, u
 }
 
 // ComputeOctTreeNodeConstColor + ComputeOctTreeNodeType per chunk
-// (VoxelizerKernels.cu 1680-2380, Voxelizer.cu 931-1172), one wave per
-// node: for every chunk the node's stored brick reaches, the chunk's sample
-// (the brick's first interior voxel clamped into the chunk) against the
-// brick's voxels in that chunk that the chunk's typing launch reaches; the
-// node is NON-CONST when any differs (types OR-ed over chunks), and its
-// colour is the sample of the last chunk in visit order.
+// (VoxelizerKernels.cu 1680-2380, Voxelizer.cu 931-1172), one wave per node
+// that k_chunk_node_list kept: for every chunk the node's stored brick
+// reaches, the chunk's sample (the brick's first interior voxel clamped into
+// the chunk) against the brick's voxels in that chunk that the chunk's typing
+// launch reaches; the node is NON-CONST when any differs (types OR-ed over
+// chunks), and its colour is the sample of the last chunk in visit order.
 //
-// A brick window with no active tile under it reads zero everywhere (every
-// sample lies in the window, so the colour is zero too): CONST, colour 0,
-// without further reads.  Otherwise the window's voxel offsets u along
-// each axis map to a chunk slot j (the chunk holding lo + u, counted from
-// the window's first) and to whether that chunk's typing launch reaches
-// them (kChunkTypedBit); the chunks' samples are read once per node (slot
-// triple -> colour) and the wave stops at the first voxel that differs.
-// Windows wider than kChunkAxis or with more than kChunkSamples slot
-// triples read every voxel's sample directly.  The nodes of every depth in
-// one launch, the coarse depths (few nodes, each a long walk) first, so
-// their waves run beside the many waves of the finer depths.
+// The window's voxel offsets u along each axis map to a chunk slot j (the
+// chunk holding lo + u, counted from the window's first) and to whether that
+// chunk's typing launch reaches them (kChunkTypedBit); the chunks' samples are
+// read once per node (slot triple -> colour), and the window's tiles with
+// them.  A voxel's sample and tile then come from the LDS, by the sum of one
+// word per axis, and only its colour (on level 0 beside its stored bits) from
+// memory, for kChunkAhead voxels a lane at once; the wave stops at the first
+// of these steps with a voxel that differs.
+// Windows wider than kChunkAxis or with more than kChunkSamples slot triples
+// read every voxel's sample directly (room for 512 triples costs a workgroup a
+// CU: 249 us where 64 take 216).
 constexpr uint32_t kChunkAxis = 66, kChunkSamples = 64, kChunkTypedBit = 1u << 31;
+constexpr uint32_t kChunkTiles = 1000;   // a window of kChunkAxis reaches 10 tiles an axis
+constexpr int kChunkAhead = 4;
+// An axis word's parts: slot, tile and place in the tile, each times its stride.
+constexpr uint32_t kAxTile = 7, kAxVox = 17, kAxOut = 1u << 28;   // out: past the level's extent
+static_assert(kChunkSamples <= 1u << kAxTile && kChunkTiles < 1u << (kAxVox - kAxTile) &&
+                  kAxVox + 9 <= 28,
+              "the sums of three words' parts stay apart");
 constexpr int kChunkWaves = kBlock / 64;
-__global__ __launch_bounds__(kBlock) void k_chunk_node_type(SampleDepths S, ChunkGeom cg) {
+
+// The nodes with an active tile under their brick window, of every depth, in
+// any order.  The window of any other reads zero everywhere (every sample lies
+// in the window, so the colour is zero too): CONST, colour 0.  A thread per
+// node (18 us for the 300 K nodes of 1024^3, bricks of 16^3, in chunks of
+// 256^3): when a wave each found out first, nine in ten for nothing, the typing
+// took 355 us with VALU and scalar issue full, so 18 + 216.
+__global__ __launch_bounds__(kBlock) void k_chunk_node_list(SampleDepths S, ChunkGeom cg,
+                                                            uint32_t* __restrict__ list,
+                                                            uint32_t* __restrict__ count) {
+    __shared__ uint32_t s_w[kBlock / 64];
+    __shared__ uint32_t s_base;
+    const uint64_t g = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    bool any = false;
+    if (g < S.start[S.L]) {
+        int d = 0;
+        while (g >= S.start[d + 1]) ++d;
+        const uint64_t n = g - S.start[d];
+        const LevelMap& lm = S.lm[d];
+        uint32_t nd[3], t0[3], t1[3];
+        node_xyz(n, (uint32_t)(__ffs(S.Rd[d]) - 1), nd[0], nd[1], nd[2]);
+        bool in = true;
+        for (int a = 0; a < 3; ++a) {
+            const uint32_t sp = nd[a] * S.B[a] + S.border[d][a];
+            const uint32_t cov = cg.nc[a] * (cg.C[a] >> (S.L - 1 - d));
+            in = in && sp - 1u < cov;
+            t0[a] = (sp - 1u) >> 3;
+            t1[a] = min(min(sp + S.B[a], cov - 1u) >> 3, lm.TG[a] - 1u);
+            in = in && t0[a] <= t1[a];
+        }
+        if (in) {
+            const uint32_t nt =
+                (t1[0] - t0[0] + 1u) * (t1[1] - t0[1] + 1u) * (t1[2] - t0[2] + 1u);
+            uint32_t tx = t0[0], ty = t0[1], tz = t0[2];
+            // the loads independent of each other, several in flight
+#pragma unroll 8
+            for (uint32_t k = 0; k < nt; ++k) {
+                any |= lm.tileIdx[((uint64_t)tz * lm.TG[1] + ty) * lm.TG[0] + tx] >= 0;
+                if (++tx > t1[0]) {
+                    tx = t0[0];
+                    if (++ty > t1[1]) { ty = t0[1]; ++tz; }
+                }
+            }
+        }
+        if (!any) {
+            S.cc[d][n] = 0u;
+            S.flag[d][n] = 0u;
+        }
+    }
+    uint32_t total;
+    const uint32_t o = block_excl_scan(any ? 1u : 0u, s_w, &total);
+    if (!total) return;   // uniform
+    if (threadIdx.x == 0) s_base = atomicAdd(count, total);
+    __syncthreads();
+    if (any) list[s_base + o] = (uint32_t)g;
+}
+
+__global__ __launch_bounds__(kBlock) void k_chunk_node_type(
+    SampleDepths S, ChunkGeom cg, const uint32_t* __restrict__ list,
+    const uint32_t* __restrict__ count) {
     __shared__ uint32_t s_ax[kChunkWaves][3][kChunkAxis];
-    __shared__ uint32_t s_sco[kChunkWaves][3][kChunkSamples];
+    __shared__ uint32_t s_sco[kChunkWaves][3][kChunkAxis];
     __shared__ uint32_t s_samp[kChunkWaves][kChunkSamples];
+    __shared__ int32_t s_tile[kChunkWaves][kChunkTiles];
     const uint32_t lane = threadIdx.x & 63u;
     // the wave's index, and below its node and depth, in scalar registers
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t Bv[3] = {S.B[0], S.B[1], S.B[2]};
     const uint32_t e[3] = {Bv[0] + 2u, Bv[1] + 2u, Bv[2] + 2u};
-    const uint64_t total = S.start[S.L];
-    for (uint64_t g = (uint64_t)blockIdx.x * kChunkWaves + wv; g < total;
-         g += (uint64_t)gridDim.x * kChunkWaves) {
+    const uint32_t total = *count;
+    for (uint64_t i = (uint64_t)blockIdx.x * kChunkWaves + wv; i < total;
+         i += (uint64_t)gridDim.x * kChunkWaves) {
+        const uint64_t g = __builtin_amdgcn_readfirstlane(list[i]);
         int dd = 0;   // the node's depth (uniform over the wave)
         while (g >= S.start[dd + 1]) ++dd;
         dd = __builtin_amdgcn_readfirstlane(dd);
@@ -2739,57 +2807,65 @@ __global__ __launch_bounds__(kBlock) void k_chunk_node_type(SampleDepths S, Chun
         uint32_t nd[3];
         node_xyz(n, ld, nd[0], nd[1], nd[2]);
         uint32_t lo[3], hi[3], c0[3], c1[3], sp[3], cov[3], m[3];
-        bool inAny = true;
         for (int a = 0; a < 3; ++a) {
             sp[a] = nd[a] * Bv[a] + bo[a];
             lo[a] = sp[a] - 1u;
             hi[a] = sp[a] + Bv[a];
             cov[a] = cg.nc[a] * Ck[a];
-            c0[a] = lo[a] / Ck[a];
-            c1[a] = min(hi[a] / Ck[a], cg.nc[a] - 1u);
-            m[a] = (lo[a] + e[a] - 1u) / Ck[a] - c0[a] + 1u;
-            if (c0[a] >= cg.nc[a]) inAny = false;
         }
-        // any active tile under the window
-        bool any = false;
-        if (inAny) {
+        const bool narrow = e[0] <= kChunkAxis && e[1] <= kChunkAxis && e[2] <= kChunkAxis;
+        int32_t* tl = s_tile[wv];
+        // the window's tiles
+        uint32_t ntx = 1u, ntxy = 1u;
+        if (narrow) {
             const uint32_t t0[3] = {lo[0] >> 3, lo[1] >> 3, lo[2] >> 3};
             uint32_t t1[3];
             for (int a = 0; a < 3; ++a) t1[a] = min(hi[a], cov[a] - 1u) >> 3;
-            const uint32_t ntx = t1[0] - t0[0] + 1u, nty = t1[1] - t0[1] + 1u;
-            const uint32_t ntl = ntx * nty * (t1[2] - t0[2] + 1u);
-            bool mine = false;
+            ntx = t1[0] - t0[0] + 1u;
+            const uint32_t nty = t1[1] - t0[1] + 1u;
+            ntxy = ntx * nty;
+            const uint32_t ntl = ntxy * (t1[2] - t0[2] + 1u);
+            const float invX = __builtin_amdgcn_rcpf((float)ntx),
+                        invY = __builtin_amdgcn_rcpf((float)nty);
             for (uint32_t q = lane; q < ntl; q += 64u) {
-                const uint32_t qx = q % ntx, qy = (q / ntx) % nty, qz = q / (ntx * nty);
-                const uint32_t tx = t0[0] + qx, ty = t0[1] + qy, tz = t0[2] + qz;
-                if (tx < lm.TG[0] && ty < lm.TG[1] && tz < lm.TG[2] &&
-                    lm.tileIdx[((uint64_t)tz * lm.TG[1] + ty) * lm.TG[0] + tx] >= 0)
-                    mine = true;
+                const uint32_t r = udiv_small(q, ntx, invX), qz = udiv_small(r, nty, invY);
+                const uint32_t tx = t0[0] + q - r * ntx, ty = t0[1] + r - qz * nty,
+                               tz = t0[2] + qz;
+                int32_t t = -1;
+                if (tx < lm.TG[0] && ty < lm.TG[1] && tz < lm.TG[2])
+                    t = lm.tileIdx[((uint64_t)tz * lm.TG[1] + ty) * lm.TG[0] + tx];
+                tl[q] = t;
             }
-            any = __ballot(mine) != 0ull;
         }
-        if (!any) {
-            if (lane == 0) {
-                cc[n] = 0u;
-                flag[n] = 0u;
-            }
-            continue;
+        // coordinates are below 2^16, a divisor's reciprocal is within an ulp
+        float invCk[3];
+        for (int a = 0; a < 3; ++a) {
+            invCk[a] = __builtin_amdgcn_rcpf((float)Ck[a]);
+            c0[a] = udiv_small(lo[a], Ck[a], invCk[a]);
+            const uint32_t ch = udiv_small(hi[a], Ck[a], invCk[a]);
+            c1[a] = min(ch, cg.nc[a] - 1u);
+            m[a] = ch - c0[a] + 1u;
         }
-        const bool tables = e[0] <= kChunkAxis && e[1] <= kChunkAxis && e[2] <= kChunkAxis &&
-                            m[0] * m[1] * m[2] <= kChunkSamples;   // uniform
+        const bool tables = narrow && m[0] * m[1] * m[2] <= kChunkSamples;   // uniform
         bool diff = false;
         if (tables) {
             uint32_t (&ax)[3][kChunkAxis] = s_ax[wv];
-            uint32_t (&sco)[3][kChunkSamples] = s_sco[wv];
+            uint32_t (&sco)[3][kChunkAxis] = s_sco[wv];
             uint32_t* samp = s_samp[wv];
             for (uint32_t t = lane; t < e[0] + e[1] + e[2]; t += 64u) {
                 const int a = t < e[0] ? 0 : (t < e[0] + e[1] ? 1 : 2);
                 const uint32_t u = t - (a == 0 ? 0u : (a == 1 ? e[0] : e[0] + e[1]));
                 const uint32_t P = lo[a] + u;
-                const uint32_t ci = P / Ck[a], o = ci * Ck[a];
+                const uint32_t ci = udiv_small(P, Ck[a], invCk[a]), o = ci * Ck[a];
                 const bool typed = P < cov[a] &&
                                    P - o < chunk_typed_limit(Ck[a], o, bo[a], full[a], a == 0);
-                ax[a][u] = (typed ? kChunkTypedBit : 0u) | (ci - c0[a]);
+                const uint32_t slot = (ci - c0[a]) * (a == 0 ? 1u : (a == 1 ? m[0] : m[0] * m[1]));
+                const uint32_t tile =
+                    ((P >> 3) - (lo[a] >> 3)) * (a == 0 ? 1u : (a == 1 ? ntx : ntxy));
+                ax[a][u] = typed ? kChunkTypedBit | slot | (tile << kAxTile) |
+                                       ((P & 7u) << (kAxVox + 3u * (uint32_t)a)) |
+                                       (P < lm.dims[a] ? 0u : kAxOut)
+                                 : 0u;
             }
             for (uint32_t t = lane; t < m[0] + m[1] + m[2]; t += 64u) {
                 const int a = t < m[0] ? 0 : (t < m[0] + m[1] ? 1 : 2);
@@ -2805,16 +2881,19 @@ __global__ __launch_bounds__(kBlock) void k_chunk_node_type(SampleDepths S, Chun
             const uint32_t mt = m[0] * m[1] * m[2];
             uint32_t myRank = 0u, myCol = 0u;
             bool ranked = false;
+            const float invM0 = __builtin_amdgcn_rcpf((float)m[0]),
+                        invM1 = __builtin_amdgcn_rcpf((float)m[1]);
             for (uint32_t t = lane; t < mt; t += 64u) {
-                const uint32_t j0 = t % m[0], j1 = (t / m[0]) % m[1], j2 = t / (m[0] * m[1]);
+                const uint32_t r = udiv_small(t, m[0], invM0), j2 = udiv_small(r, m[1], invM1);
+                const uint32_t j0 = t - r * m[0], j1 = r - j2 * m[1];
                 const uint32_t c = level_col(lm, col, sco[0][j0], sco[1][j1], sco[2][j2]);
                 samp[t] = c;
                 if (c0[0] + j0 <= c1[0] && c0[1] + j1 <= c1[1] && c0[2] + j2 <= c1[2]) {
-                    const uint32_t r = cg.rank[((uint64_t)(c0[2] + j2) * cg.nc[1] + (c0[1] + j1)) *
-                                                   cg.nc[0] + (c0[0] + j0)];
-                    if (!ranked || r > myRank) {
+                    const uint32_t rk = cg.rank[((uint64_t)(c0[2] + j2) * cg.nc[1] + (c0[1] + j1)) *
+                                                    cg.nc[0] + (c0[0] + j0)];
+                    if (!ranked || rk > myRank) {
                         ranked = true;
-                        myRank = r;
+                        myRank = rk;
                         myCol = c;
                     }
                 }
@@ -2836,25 +2915,44 @@ __global__ __launch_bounds__(kBlock) void k_chunk_node_type(SampleDepths S, Chun
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-            // voxel q = (w * e1 + v) * e0 + u; q / e0 and q / (e0 e1) by
-            // multiply-high with ceil(2^32 / d), exact for q * d < 2^32
-            // (windows of at most 66^3 voxels)
+            // voxel q = (w * e1 + v) * e0 + u: (q + 1/2) / d is at least 1 / (2 d)
+            // from a whole number, 1.1e-4 for d <= 66^2, past the rounding of
+            // its product with 1 / d (2e-5 for quotients up to 66)
             const uint32_t e01 = e[0] * e[1], nv = e01 * e[2];
-            const uint32_t inv0 = (uint32_t)((0x100000000ull + e[0] - 1u) / e[0]);
-            const uint32_t inv01 = (uint32_t)((0x100000000ull + e01 - 1u) / e01);
-            for (uint32_t b = 0; b < nv; b += 64u) {
-                const uint32_t q = b + lane;
-                bool d = false;
-                if (q < nv) {
-                    const uint32_t w = __umulhi(q, inv01), r = q - w * e01;
-                    const uint32_t v = __umulhi(r, inv0), u = r - v * e[0];
-                    const uint32_t ax0 = ax[0][u], ay = ax[1][v], az = ax[2][w];
-                    if (ax0 & ay & az & kChunkTypedBit) {
-                        const uint32_t j0 = ax0 & 0xffffu, j1 = ay & 0xffffu, j2 = az & 0xffffu;
-                        const uint32_t scol = samp[(j2 * m[1] + j1) * m[0] + j0];
-                        d = level_col(lm, col, lo[0] + u, lo[1] + v, lo[2] + w) != scol;
+            const float inv0 = 1.0f / (float)e[0], inv01 = 1.0f / (float)e01;
+            for (uint32_t b = 0; b < nv; b += 64u * kChunkAhead) {
+                uint32_t c[kChunkAhead], want[kChunkAhead], bits[kChunkAhead], at[kChunkAhead];
+#pragma unroll
+                for (int i = 0; i < kChunkAhead; ++i) {
+                    const uint32_t q = b + (uint32_t)i * 64u + lane;
+                    c[i] = want[i] = 0u;
+                    bits[i] = ~0u;
+                    at[i] = 0u;
+                    if (q < nv) {
+                        const uint32_t w = (uint32_t)(((float)q + 0.5f) * inv01),
+                                       r = q - __umul24(w, e01);
+                        const uint32_t v = (uint32_t)(((float)r + 0.5f) * inv0),
+                                       u = r - __umul24(v, e[0]);
+                        const uint32_t ax0 = ax[0][u], ay = ax[1][v], az = ax[2][w];
+                        if (ax0 & ay & az & kChunkTypedBit) {
+                            const uint32_t sum = ax0 + ay + az;
+                            want[i] = samp[sum & ((1u << kAxTile) - 1u)];
+                            const int32_t t = tl[(sum >> kAxTile) & ((1u << (kAxVox - kAxTile)) - 1u)];
+                            at[i] = (sum >> kAxVox) & (kTileVox - 1u);
+                            if (t >= 0 && !((ax0 | ay | az) & kAxOut)) {
+                                c[i] = col[(uint64_t)t * kTileVox + at[i]];
+                                if (lm.defOcc) {   // uniform
+                                    const uint64_t wd = (uint64_t)t * kTileWords + (at[i] >> 5);
+                                    bits[i] = lm.defOcc[wd] | lm.defFill[wd];
+                                }
+                            }
+                        }
                     }
                 }
+                bool d = false;
+#pragma unroll
+                for (int i = 0; i < kChunkAhead; ++i)
+                    d = d || (((bits[i] >> (at[i] & 31u)) & 1u) ? c[i] : 0u) != want[i];
                 if (__ballot(d)) {
                     diff = true;
                     break;
@@ -2922,54 +3020,82 @@ __global__ __launch_bounds__(kBlock) void k_chunk_node_type(SampleDepths S, Chun
 // inside one chunk it is written while that chunk is typed; across chunks
 // it is assembled and written after the last of them, with the other
 // bricks completed there, in (z, y, x) order.
-__global__ void k_chunk_brick_keys(const uint32_t* __restrict__ flag, ChunkGeom cg, int k,
-                                   uint32_t Rd, uint32_t B0, uint32_t B1, uint32_t B2,
-                                   uint32_t bo0, uint32_t bo1, uint32_t bo2,
-                                   unsigned long long* __restrict__ keys,
-                                   uint32_t* __restrict__ nodes, uint32_t* __restrict__ count) {
-    const uint64_t n = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t nn = (uint64_t)Rd * Rd * Rd;
-    if (n >= nn || flag[n] != 1u) return;
-    const uint32_t Ck[3] = {cg.C[0] >> k, cg.C[1] >> k, cg.C[2] >> k}, Bv[3] = {B0, B1, B2},
-                   bo[3] = {bo0, bo1, bo2};
-    const uint32_t ld = (uint32_t)(__ffs(Rd) - 1);
-    uint32_t nd[3];
-    node_xyz(n, ld, nd[0], nd[1], nd[2]);
-    uint32_t c0[3], c1[3];
-    bool inside = true;
-    for (int a = 0; a < 3; ++a) {
-        const uint32_t lo = nd[a] * Bv[a] + bo[a] - 1u, hi = nd[a] * Bv[a] + bo[a] + Bv[a];
-        if (hi >= cg.nc[a] * Ck[a]) return;   // part of it never processed: no brick
-        c0[a] = lo / Ck[a];
-        c1[a] = hi / Ck[a];
-        inside = inside && c0[a] == c1[a];
+// The keys of all depths side by side, each with its depth on top (from bit
+// depthShift), in any order.  A workgroup's nodes are of one depth and take
+// their places with one atomic each on the total and the depth's count (one a
+// node cost 44 us for the 9 K bricks of 1024^3 in chunks of 256^3, with a
+// launch and a sort per depth another 100).
+__global__ __launch_bounds__(kBlock) void k_chunk_brick_keys(SampleDepths S, ChunkGeom cg,
+                                                             uint32_t depthShift,
+                                                             unsigned long long* __restrict__ keys,
+                                                             uint32_t* __restrict__ nodes,
+                                                             uint32_t* __restrict__ count,
+                                                             uint32_t* __restrict__ total) {
+    __shared__ uint32_t s_w[kBlock / 64];
+    __shared__ uint32_t s_base;
+    int d = 0;   // uniform: the workgroup's depth, and its first node there
+    uint64_t b0 = blockIdx.x;
+    for (; d + 1 < S.L; ++d) {
+        const uint64_t blocks = (S.start[d + 1] - S.start[d] + kBlock - 1u) / kBlock;
+        if (b0 < blocks) break;
+        b0 -= blocks;
     }
+    const uint32_t Rd = S.Rd[d];
+    const uint64_t n = b0 * kBlock + threadIdx.x, nn = S.start[d + 1] - S.start[d];
+    const int k = S.L - 1 - d;
+    const uint32_t ld = (uint32_t)(__ffs(Rd) - 1);
+    bool brick = n < nn && S.flag[d][n] == 1u, inside = true;
     uint32_t last = 0u;
-    for (uint32_t k = c0[2]; k <= c1[2]; ++k)
-        for (uint32_t j = c0[1]; j <= c1[1]; ++j)
-            for (uint32_t i = c0[0]; i <= c1[0]; ++i)
-                last = max(last, cg.rank[((uint64_t)k * cg.nc[1] + j) * cg.nc[0] + i]);
-    const uint32_t sh = 3u * ld;
-    const uint32_t slot = atomicAdd(count, 1u);
-    keys[slot] = ((unsigned long long)last << (sh + 1u)) | ((unsigned long long)(inside ? 0u : 1u) << sh) |
-                 (unsigned long long)n;
+    if (brick) {
+        uint32_t nd[3], c0[3], c1[3];
+        node_xyz(n, ld, nd[0], nd[1], nd[2]);
+        for (int a = 0; a < 3; ++a) {
+            const uint32_t Ck = cg.C[a] >> k, sp = nd[a] * S.B[a] + S.border[d][a];
+            const uint32_t lo = sp - 1u, hi = sp + S.B[a];
+            if (hi >= cg.nc[a] * Ck) brick = false;   // part of it never processed: no brick
+            c0[a] = lo / Ck;
+            c1[a] = hi / Ck;
+            inside = inside && c0[a] == c1[a];
+        }
+        if (brick)
+            for (uint32_t z = c0[2]; z <= c1[2]; ++z)
+                for (uint32_t j = c0[1]; j <= c1[1]; ++j)
+                    for (uint32_t i = c0[0]; i <= c1[0]; ++i)
+                        last = max(last, cg.rank[((uint64_t)z * cg.nc[1] + j) * cg.nc[0] + i]);
+    }
+    uint32_t mine;
+    const uint32_t o = block_excl_scan(brick ? 1u : 0u, s_w, &mine);
+    if (!mine) return;   // uniform
+    if (threadIdx.x == 0) {
+        s_base = atomicAdd(total, mine);
+        atomicAdd(&count[d], mine);
+    }
+    __syncthreads();
+    if (!brick) return;
+    const uint32_t sh = 3u * ld, slot = s_base + o;
+    keys[slot] = ((unsigned long long)d << depthShift) | ((unsigned long long)last << (sh + 1u)) |
+                 ((unsigned long long)(inside ? 0u : 1u) << sh) | (unsigned long long)n;
     nodes[slot] = (uint32_t)n;
 }
 
-__global__ void k_chunk_types(uint64_t nn, const uint32_t* __restrict__ flag,
-                              uint8_t* __restrict__ types, uint32_t* __restrict__ bidx) {
+// Every node's type, and no brick yet.
+__global__ void k_chunk_types(DepthOut D, const uint32_t* __restrict__ flag) {
     const uint64_t n = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= nn) return;
-    types[n] = (uint8_t)flag[n];
-    bidx[n] = 0xffffffffu;
+    if (n >= D.off[D.L]) return;
+    int d = 0;
+    while (d + 1 < D.L && n >= D.off[d + 1]) ++d;
+    D.types[d][n - D.off[d]] = (uint8_t)flag[n];
+    D.bidx[d][n - D.off[d]] = 0xffffffffu;
 }
-__global__ void k_chunk_bidx(uint32_t nb, const uint32_t* __restrict__ sorted,
-                             uint32_t* __restrict__ bidx, uint32_t* __restrict__ brickNode) {
+// Brick j - first[d] of depth d is that of node sorted[j].
+__global__ void k_chunk_bidx(DepthOut D, RangeOffs first, const uint32_t* __restrict__ sorted) {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= nb) return;
-    const uint32_t n = sorted[j];
-    bidx[n] = j;
-    brickNode[j] = n;
+    if (j >= first.v[D.L]) return;
+    int d = 0;
+    while (j >= first.v[d + 1]) ++d;
+    const uint32_t n = sorted[j], i = j - (uint32_t)first.v[d];
+    D.bidx[d][n] = i;
+    D.brickNode[d][i] = n;
 }
 
 inline unsigned grid_for(uint64_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
@@ -3317,25 +3443,28 @@ void launch_chunk_mip(hipStream_t st, const LevelMap& src, const LevelMap& dst,
     k_chunk_mip<<<(unsigned)nActive, kBlock, 0, st>>>(src, dst, cg, ks, kd, listDst, colSrc, nrmSrc,
                                                       colDst, qnDst, nrmDst);
 }
-void launch_chunk_node_type(hipStream_t st, const SampleDepths& S, const ChunkGeom& cg) {
+void launch_chunk_node_type(hipStream_t st, const SampleDepths& S, const ChunkGeom& cg,
+                            uint32_t* list, uint32_t* count) {
     const uint64_t nn = S.start[S.L];
     if (nn == 0) return;
-    const unsigned grid = (unsigned)std::min<uint64_t>((nn + kChunkWaves - 1) / kChunkWaves, 1u << 20);
-    k_chunk_node_type<<<grid, kBlock, 0, st>>>(S, cg);
+    k_chunk_node_list<<<grid_for(nn, kBlock), kBlock, 0, st>>>(S, cg, list, count);
+    const unsigned grid = (unsigned)std::min<uint64_t>((nn + kChunkWaves - 1) / kChunkWaves, 1u << 14);
+    k_chunk_node_type<<<grid, kBlock, 0, st>>>(S, cg, list, count);
 }
-void launch_chunk_brick_keys(hipStream_t st, const uint32_t* flag, const ChunkGeom& cg, int k,
-                             uint32_t Rd, const uint32_t B[3], const uint32_t border[3],
-                             unsigned long long* keys, uint32_t* nodes, uint32_t* count) {
-    const uint64_t nn = (uint64_t)Rd * Rd * Rd;
-    k_chunk_brick_keys<<<grid_for(nn, kBlock), kBlock, 0, st>>>(flag, cg, k, Rd, B[0], B[1], B[2],
-                                                                border[0], border[1], border[2],
-                                                                keys, nodes, count);
+void launch_chunk_brick_keys(hipStream_t st, const SampleDepths& S, const ChunkGeom& cg,
+                             uint32_t depthShift, unsigned long long* keys, uint32_t* nodes,
+                             uint32_t* count, uint32_t* total) {
+    uint64_t blocks = 0;
+    for (int d = 0; d < S.L; ++d) blocks += grid_for(S.start[d + 1] - S.start[d], kBlock);
+    if (blocks)
+        k_chunk_brick_keys<<<(unsigned)blocks, kBlock, 0, st>>>(S, cg, depthShift, keys, nodes,
+                                                                count, total);
 }
-void launch_chunk_brick_assign(hipStream_t st, uint64_t nodes, const uint32_t* flag,
-                               const uint32_t* sorted, uint32_t nb, uint8_t* types,
-                               uint32_t* bidx, uint32_t* brickNode) {
-    if (nodes) k_chunk_types<<<grid_for(nodes, kBlock), kBlock, 0, st>>>(nodes, flag, types, bidx);
-    if (nb) k_chunk_bidx<<<grid_for(nb, kBlock), kBlock, 0, st>>>(nb, sorted, bidx, brickNode);
+void launch_chunk_brick_assign(hipStream_t st, const DepthOut& D, const RangeOffs& first,
+                               const uint32_t* flag, const uint32_t* sorted) {
+    const uint64_t nodes = D.off[D.L], bricks = first.v[D.L];
+    if (nodes) k_chunk_types<<<grid_for(nodes, kBlock), kBlock, 0, st>>>(D, flag);
+    if (bricks) k_chunk_bidx<<<grid_for(bricks, kBlock), kBlock, 0, st>>>(D, first, sorted);
 }
 
 }  // namespace voxmi
