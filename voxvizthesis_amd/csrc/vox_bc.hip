@@ -202,7 +202,7 @@ __device__ __forceinline__ void encode_block(const uint32_t* c, const uint32_t* 
 // follow each other in memory, so a workgroup takes as many whole ones as 256
 // threads hold (perWg, of bxn blocks), and copies their texels, one contiguous
 // range, through the LDS: read straight from memory, every load of a wave fell
-// into some 50 cache lines.  Bound by VALU issue (4.6 K bricks of 18^3 texels
+// into some 50 cache lines.  Bound by VALU issue (4.3 K bricks of 18^3 texels
 // of a 512^3 terrain: 142 us with a distance per channel, entry and texel and
 // texels read from memory; 130 us with byte dot products, 91 us now).
 __global__ __launch_bounds__(kWg) void k_bc_bricks(const uint32_t* __restrict__ col,
