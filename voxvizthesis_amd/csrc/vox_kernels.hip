@@ -2722,7 +2722,7 @@ constexpr int kChunkWaves = kBlock / 64;
 // any order.  The window of any other reads zero everywhere (every sample lies
 // in the window, so the colour is zero too): CONST, colour 0.  A thread per
 // node (18 us for the 300 K nodes of 1024^3, bricks of 16^3, in chunks of
-// 256^3): when a wave each found out first, nine in ten for nothing, the typing
+// 256^3): when a wave each found out first, most of them for nothing, the typing
 // took 355 us with VALU and scalar issue full, so 18 + 216.
 __global__ __launch_bounds__(kBlock) void k_chunk_node_list(SampleDepths S, ChunkGeom cg,
                                                             uint32_t* __restrict__ list,
@@ -3023,7 +3023,7 @@ __global__ __launch_bounds__(kBlock) void k_chunk_node_type(
 // The keys of all depths side by side, each with its depth on top (from bit
 // depthShift), in any order.  A workgroup's nodes are of one depth and take
 // their places with one atomic each on the total and the depth's count (one a
-// node cost 44 us for the 9 K bricks of 1024^3 in chunks of 256^3, with a
+// node cost 44 us for the 19 K bricks of 1024^3 in chunks of 256^3, with a
 // launch and a sort per depth another 100).
 __global__ __launch_bounds__(kBlock) void k_chunk_brick_keys(SampleDepths S, ChunkGeom cg,
                                                              uint32_t depthShift,

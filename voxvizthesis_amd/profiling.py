@@ -31,9 +31,11 @@ def kname(s: str) -> str:
     m = re.search(r"wrapped_(\w+?)_config", s)
     if s.startswith("void rocprim") and m:
         return "rocprim " + m.group(1)
+    # a template's instance: "void ", then its arguments after the name
+    s = s.removeprefix("void ")
     for prefix in ("voxmi::(anonymous namespace)::", "(anonymous namespace)::"):
         if s.startswith(prefix):
-            s = s[len(prefix):]
+            return s[len(prefix):].split("(")[0].split("<")[0]
     return s.split("(")[0]
 
 
