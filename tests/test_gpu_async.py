@@ -113,3 +113,20 @@ def test_timing_run_equals_overlapped_run():
             assert any(t.any() for t in ref[1::5])   # some node typed
         finally:
             vz.close()
+
+
+def test_an_earlier_error_of_the_thread_is_not_the_generate_s():
+    """The runtime keeps a failed call's error until it is read: one left by
+    other code of the thread does not refuse a setup pass or a generate."""
+    import ctypes as C
+    hip = C.CDLL("libamdhip64.so")
+    vz = upload(scenes.scene_two_triangles(), 8)
+    try:
+        for _ in range(2):
+            assert hip.hipEventQuery(None) != 0 and hip.hipPeekAtLastError() != 0
+            print("[async] after an error left behind", flush=True)
+            assert vz.computeEdgesFaceNormalsAndBounds(), vz.getErrorMessage()
+            assert hip.hipEventQuery(None) != 0
+            assert vz.generateVoxelsAndOctTree(None) == 1, vz.getErrorMessage()
+    finally:
+        vz.close()

@@ -213,6 +213,12 @@ struct vox_ctx {
         err << m << std::endl;
         return false;
     }
+    // Before the launches of a call whose error it reads at its end: one that
+    // an earlier call of the thread left behind (not ready, a refused capture)
+    // is not this call's.
+    void forget_error() const {
+        if (!replay) (void)hipGetLastError();
+    }
     bool check(hipError_t e, const char* what) {
         if (e == hipSuccess) return true;
         err << what << " failed: " << hipGetErrorString(e) << std::endl;
@@ -819,6 +825,7 @@ int vox_compute_edges_face_normals_and_bounds(vox_ctx* h) {
         return 0;
     uint32_t* cnt = h->binCount.as<uint32_t>();
     uint32_t* start = h->binStart.as<uint32_t>();
+    h->forget_error();
     h->run("fill", [&] {
         const FillSeg z[2] = {{cnt, h->numBins, 0u},
                               {h->counters.as<uint32_t>(), kCounterWords, 0u}};
@@ -865,6 +872,7 @@ int gen_front(vox_ctx* h) {
     hipStream_t st = h->st;
     if (!h->replay) {
         std::memset(&h->stats, 0, sizeof(h->stats));
+        h->forget_error();
         (void)hipEventRecord(h->evStart, st);
     }
 
