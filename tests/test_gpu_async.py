@@ -117,7 +117,7 @@ def test_timing_run_equals_overlapped_run():
 
 def test_an_earlier_error_of_the_thread_is_not_the_generate_s():
     """The runtime keeps a failed call's error until it is read: one left by
-    other code of the thread does not refuse a setup pass or a generate."""
+    other code of the thread refuses no triangle upload, setup pass or generate."""
     import ctypes as C
     hip = C.CDLL("libamdhip64.so")
     vz = upload(scenes.scene_two_triangles(), 8)
@@ -125,6 +125,8 @@ def test_an_earlier_error_of_the_thread_is_not_the_generate_s():
         for _ in range(2):
             assert hip.hipEventQuery(None) != 0 and hip.hipPeekAtLastError() != 0
             print("[async] after an error left behind", flush=True)
+            assert vz.allocateTriangleMemory(), vz.getErrorMessage()
+            assert hip.hipEventQuery(None) != 0
             assert vz.computeEdgesFaceNormalsAndBounds(), vz.getErrorMessage()
             assert hip.hipEventQuery(None) != 0
             assert vz.generateVoxelsAndOctTree(None) == 1, vz.getErrorMessage()

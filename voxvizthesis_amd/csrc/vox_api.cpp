@@ -669,6 +669,7 @@ int vox_allocate_triangle_memory(vox_ctx* h) {
         !h->grpFill.ensure(h->groups.size() * 4 + 4, h->err, "group flags"))
         return 0;
     h->fillFlags.clear();
+    h->forget_error();
     // Concatenate groups (allocateTriangleMemory, Voxelizer.cu 346-457).
     uint64_t to = 0, vo = 0, uo = 0, io = 0;
     h->gargs.clear();
