@@ -771,6 +771,7 @@ int vox_compute_edges_face_normals_and_bounds(vox_ctx* h) {
     if (!h || !h->valid || !idle(h)) return 0;
     if (!h->voxMem && !vox_allocate_voxel_memory(h)) return 0;
     if (!h->triMem && !vox_allocate_triangle_memory(h)) return 0;
+    h->prepared = false;   // until the pass below is queued whole
     VoxParams& P = h->P;
     for (int a = 0; a < 3; ++a) {
         P.offP[a] = h->offP[a];
@@ -1898,6 +1899,7 @@ int vox_batch_capture(vox_batch* b) {
     }
     for (size_t j = 0; j < J; ++j) {
         b->jobs[j]->replay = false;
+        b->jobs[j]->prepared = false;   // a captured setup pass has not run
         b->jobs[j]->st = own[j];
     }
     hipGraph_t g = nullptr;
@@ -1969,6 +1971,9 @@ int vox_batch_launch(vox_batch* b) {
             return b->fail("batch: the triangles of job " + std::to_string(j) +
                            " changed since the capture; capture again"), 0;
     (void)hipEventRecord(b->ev[1], b->st);
+    // the graph's generates use up the counters and bin counts of a setup
+    // pass that a job had queued for its own: a generate after it sets up again
+    for (vox_ctx* h : b->jobs) h->prepared = false;
     if (!b->check(hipGraphLaunch(b->exec, b->st), "graph launch")) return 0;
     (void)hipEventRecord(b->ev[2], b->st);
     if (!b->check(hipStreamSynchronize(b->st), "graph")) return 0;
