@@ -110,3 +110,40 @@ def test_raycast_resident_poses(pos, target, fov):
     finally:
         for o in (srv, rc, t, bp, vz):
             o.close()
+
+
+# a box so thin that its brick step along x is 0 / 0, met by the rays of the
+# centre column (x component 0, every other ray's overflows); a box so long
+# that the root's brick step along y overflows
+@pytest.mark.parametrize("case", ["thin box", "long box"])
+def test_raycast_brick_step_that_is_no_number(case):
+    from voxvizthesis_amd.gvserve import BrickServer
+    scene, (W, H) = scenes.scene_terrain_n(64, 64, 8), (33, 49)
+    vz = voxelize_scene(scene)
+    bp = BrickPool(scene.B, (10, 10, 10))
+    t = OctTree(bp, vz)
+    rc, srv = RayCaster(t, W, H), BrickServer(t)
+    tiny = float(np.finfo(np.float32).smallest_subnormal)
+    try:
+        look, up = look_at((0.5, -0.5, 0.6), (0.5, 0.5, 0.5))
+        cam = dict(position=(0.5, -0.5, 0.6), look=look, up=up, fov_y_deg=60.0, width=W, height=H)
+        prm = dict(vol_min=(0.0,) * 3, vol_max=(1.0,) * 3, jitter_seed=3)
+        for _ in range(20):
+            rc.frame(camera(**cam), raycast_params(**prm))
+            if srv.frame(rc).last_uploads == 0:
+                break
+        if case == "thin box":
+            cam["position"] = (tiny, -0.5, 0.6)
+            prm["vol_max"] = (2 * tiny, 1.0, 1.0)
+        else:
+            cam.update(position=(-0.5, 0.5e38, 0.6), look=(1.0, 0.0, 0.0), up=(0.0, 0.0, 1.0))
+            prm.update(vol_max=(1.0, 1.0e38, 1.0), ray_step=0.45)
+        print(f"[raycast] {case}", flush=True)
+        rc.frame(camera(**cam), raycast_params(**prm))
+        ru, rcol = oracle.raycast(cam, prm, vz.raw_result().levels, scene.B, t.nodes(),
+                                  bp.textures()[0])
+        assert (ru != 0).any() and (rcol != 0).any()
+        assert np.array_equal(rc.usage(), ru) and np.array_equal(rc.rgba(), rcol)
+    finally:
+        for o in (srv, rc, t, bp, vz):
+            o.close()

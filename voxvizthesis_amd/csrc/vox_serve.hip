@@ -52,6 +52,9 @@ struct RayUniforms {
     // brick's texels per axis)
     uint32_t wide, wideSlots;
     float firstTexel[3];     // 1 / poolDim: a wide pool's first interior texel
+    // brickStep is no number, or so large that a sum of it is none: the
+    // kernels' instance for that casts the frame (looked at by the host)
+    uint32_t oddStep;
     float invRayStep;        // about 1 / rayStep
     // Bounds of the level-of-detail test's outcome (lod_range): u about
     // camLeft - camUp, lodU at least its length, and the constants of the
@@ -199,9 +202,9 @@ typedef const __attribute__((address_space(1))) pair32* gpair;
 // whole 256ths.
 // Coordinates are clamped as floats (the texel numbers are whole and below
 // 2^24); a pool has at most 1024 texels per axis, so indices are 24-bit
-// products.  (No coordinate is NaN: a ray that is cast has a direction of
-// numbers, and a volume so small that its brick step would not be one has
-// none, its rays' directions overflowing before.)
+// products.  No coordinate is NaN (which reads as 0): the caller sees to that
+// where RayUniforms::oddStep says that one could be (an instance of the cast
+// for that: a test in the sample loop, uniform as it was, took 3.5 % of a frame).
 __device__ __forceinline__ void load_sample(gu32 __restrict__ col, const RayUniforms& U, v3 s,
                                             uint32_t (&t)[8], float (&w)[3]) {
     const float c[3] = {s.x, s.y, s.z};
@@ -290,6 +293,7 @@ __device__ __forceinline__ uint2 fetch_node(gu32 __restrict__ tex, const RayUnif
 // One pixel's ray through one octree (GigaVoxels.frag main): its FragColor
 // in dst and its node usage list in usage (both start at zero here).
 // Returns whether the ray met the octree's box.
+template <bool kOddStep>
 __device__ __forceinline__ bool cast_pixel(const RayUniforms& U, gu32 __restrict__ tex,
                                            gu32 __restrict__ pool,
                                            const float* __restrict__ jitter, int i, int j,
@@ -453,14 +457,19 @@ __device__ __forceinline__ bool cast_pixel(const RayUniforms& U, gu32 __restrict
                         uint32_t t[8];
                         float w[3];
                         load_sample(bpool, U, cbr, t, w);
-                        // eight empty texels add nothing (0 * weight, blended)
-                        if (((t[0] | t[1]) | (t[2] | t[3])) | ((t[4] | t[5]) | (t[6] | t[7]))) {
+                        // eight empty texels add nothing (0 * weight, blended,
+                        // unless a weight is no number)
+                        if (kOddStep ||
+                            (((t[0] | t[1]) | (t[2] | t[3])) | ((t[4] | t[5]) | (t[6] | t[7])))) {
                             float src[4];
                             weigh_sample(t, w, src);
                             src[3] = 1.0f - (1.0f - src[3]);  // pow(1 - a, 1.0)
                             blend(dst, src);
                         }
                         cbr = add(cbr, brickRayStep);
+                        if (kOddStep)
+                            cbr = mk(cbr.x == cbr.x ? cbr.x : 0.0f, cbr.y == cbr.y ? cbr.y : 0.0f,
+                                     cbr.z == cbr.z ? cbr.z : 0.0f);
                     }
                 }
                 if (nlt >= startPush && nlt < stopPush && pushed < U.maxPush) {
@@ -542,6 +551,7 @@ __device__ __forceinline__ void append_requests(const RequestList& R, const uint
 // pass over the usage lists in a kernel of its own read 100 MB back at
 // 1080p and met few equal ids per wave: 154 us beside a cast of 0.91 ms).
 constexpr int kCastW = 16, kCastH = 4;   // pixels of a wave
+template <bool kOddStep>
 __global__ void __launch_bounds__(kCastW * kCastH)
 k_raycast(RayUniforms U, const uint32_t* __restrict__ tex, const uint32_t* __restrict__ pool,
           const float* __restrict__ jitter, uint32_t* __restrict__ rgbaOut,
@@ -551,7 +561,7 @@ k_raycast(RayUniforms U, const uint32_t* __restrict__ tex, const uint32_t* __res
     uint32_t usage[kMaxUsage];
     if (i < U.rx1 && j < U.ry1) {
         float dst[4];
-        cast_pixel(U, (gu32)tex, (gu32)pool, jitter, i, j, dst, usage);
+        cast_pixel<kOddStep>(U, (gu32)tex, (gu32)pool, jitter, i, j, dst, usage);
         const uint64_t pix = (uint64_t)j * U.W + i;
         uint32_t o = 0;
 #pragma unroll
@@ -595,6 +605,7 @@ struct TreeCast {
 // requests for it.  With resume the pass continues a frame: acc from frame,
 // T from trans (a pass over the octrees in front wrote both); trans, when
 // given, receives each pixel's T for the next pass.
+template <bool kOddStep>
 __global__ void __launch_bounds__(kCastW * kCastH)
 k_raycast_multi(const TreeCast* __restrict__ trees, uint32_t n, const float* __restrict__ jitter,
                 int32_t W, int32_t x0, int32_t y0, int32_t x1, int32_t y1, float tStop,
@@ -623,7 +634,8 @@ k_raycast_multi(const TreeCast* __restrict__ trees, uint32_t n, const float* __r
         float dst[4];
         bool act = want && i >= U.rx0 && i < U.rx1 && j >= U.ry0 && j < U.ry1;
         if (act) {
-            act = cast_pixel(U, (gu32)tc.tex, (gu32)tc.pool, jitter, i, j, dst, usage);
+            act = cast_pixel<kOddStep>(U, (gu32)tc.tex, (gu32)tc.pool, jitter, i, j, dst,
+                                       usage);
         } else {
 #pragma unroll
             for (int q = 0; q < kMaxUsage; ++q) usage[q] = 0u;
@@ -767,6 +779,8 @@ bool ray_uniforms(const vox_camera& cam, const vox_raycast_params& prm, int leve
         // a wide pool is sampled one brick at a time: its texels are the frame
         const uint32_t pd = poolWide ? B[a] + 2u : poolDims[a];
         U.brickStep[a] = (1.0f / (float)pd) * ratio;
+        // (the edge of a box below the smallest floats: 0 / 0)
+        if (!(std::fabs(U.brickStep[a]) < 1.0e30f)) U.oddStep = 1u;
         U.brickDim[a] = (float)B[a];
         U.poolDim[a] = (float)pd;
         U.pdim[a] = pd;
@@ -971,8 +985,10 @@ int vox_raycast_frame(vox_raycaster* rc, const vox_camera* cam, const vox_raycas
     const RequestList R{rc->stamp.as<uint32_t>(), rc->req.as<uint32_t>(),
                         rc->reqTime.as<unsigned long long>(), rc->counts.as<uint32_t>(), rc->tag,
                         rc->maxReq};
-    k_raycast<<<grid, kCastW * kCastH, 0, st>>>(U, tex, o.poolCol, rc->jitter.as<float>(), rc->rgba.as<uint32_t>(),
-                                    rc->rgbaF.as<float4>(), rc->usage.as<uint32_t>(), R);
+    const auto cast = U.oddStep ? k_raycast<true> : k_raycast<false>;
+    cast<<<grid, kCastW * kCastH, 0, st>>>(U, tex, o.poolCol, rc->jitter.as<float>(),
+                                           rc->rgba.as<uint32_t>(), rc->rgbaF.as<float4>(),
+                                           rc->usage.as<uint32_t>(), R);
     rc->rect[0] = U.rx0;
     rc->rect[1] = U.ry0;
     rc->rect[2] = U.rx1;
@@ -1094,10 +1110,13 @@ int vox_raycast_frame_multi(vox_raycaster* const* rcs, uint32_t n, const vox_cam
     (void)hipEventRecord(r0->ev[0], st);
     dim3 grid((unsigned)(ux1 - ux0 + kCastW - 1) / kCastW,
               (unsigned)(uy1 - uy0 + kCastH - 1) / kCastH);
-    k_raycast_multi<<<grid, kCastW * kCastH, 0, st>>>(r0->multiTable.as<TreeCast>(), n, r0->jitter.as<float>(),
-                                          cam->width, ux0, uy0, ux1, uy1, t_stop,
-                                          reinterpret_cast<float4*>(frame), transmittance,
-                                          resume ? 1 : 0);
+    bool odd = false;
+    for (const TreeCast& tc : table) odd = odd || tc.U.oddStep;
+    const auto cast = odd ? k_raycast_multi<true> : k_raycast_multi<false>;
+    cast<<<grid, kCastW * kCastH, 0, st>>>(r0->multiTable.as<TreeCast>(), n, r0->jitter.as<float>(),
+                                           cam->width, ux0, uy0, ux1, uy1, t_stop,
+                                           reinterpret_cast<float4*>(frame), transmittance,
+                                           resume ? 1 : 0);
     (void)hipEventRecord(r0->ev[1], st);
     (void)hipEventRecord(r0->ev[2], st);
     if (!r0->check(hipGetLastError(), "raycast multi kernel")) return 0;
