@@ -203,7 +203,7 @@ def serving_bench(vz, scene, frames: int, W: int, H: int, slots, max_up: int, st
     hi = lo + np.asarray(scene.N, np.float32) * np.asarray(scene.delta, np.float32)
     prm = raycast_params(lo, hi, jitter_seed=5)
     paths = [scenes.flythrough(seed=5 + k, frames=frames) for k in range(streams)]
-    ray_ms, dedup_ms, req = [], [], 0
+    ray_ms, req = [], 0
     t0 = time.perf_counter()
     for f in range(frames):
         for rc, path in zip(rcs, paths):
@@ -213,7 +213,6 @@ def serving_bench(vz, scene, frames: int, W: int, H: int, slots, max_up: int, st
         for rc in rcs:  # waits for the ray casts only
             v = rc.view()
             ray_ms.append(v.ms_raycast)
-            dedup_ms.append(v.ms_requests)
             req += v.nrequests
     st = srv.stats()
     wall = time.perf_counter() - t0
@@ -233,7 +232,6 @@ def serving_bench(vz, scene, frames: int, W: int, H: int, slots, max_up: int, st
         "bricks_per_s": round(st.uploads / wall, 1),
         "frame_ms": round(wall / frames * 1e3, 3),
         "raycast_ms_mean": round(float(np.mean(ray_ms)), 4),
-        "dedup_ms_mean": round(float(np.mean(dedup_ms)), 4),
         "update_ms_mean": round(st.ms_update_total / max(st.frames, 1), 4),
         "latency_p50_ms": round(float(np.percentile(lat, 50)), 4) if len(lat) else None,
         "latency_p99_ms": round(float(np.percentile(lat, 99)), 4) if len(lat) else None,

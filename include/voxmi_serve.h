@@ -9,8 +9,9 @@
  * node texture and brick pool of voxmi_pool.h.  Each pixel records up to 12
  * node ids ((x+1)<<20 | (y+1)<<10 | (z+1) of the node texel, 0 = none,
  * GigaVoxels.frag 508-525) in the 2x2-pixel interleave of the shader
- * (571-577).  The ids are then deduplicated on the device (wave-level first,
- * then one flag per node texel) into the frame's request list, replacing the
+ * (571-577).  A wave that has cast its pixels lists their distinct ids (the
+ * wave's own first, then one flag per node texel) in the frame's request list,
+ * in place of the
  * selection-mask / histopyramid / compaction passes and the host-side
  * std::map of the reference (GigaVoxelsRenderer.cpp 2048-2110,
  * GigaVoxelsOctTree.cpp 430-652).
@@ -83,7 +84,8 @@ typedef struct vox_frame_view {
     uint32_t* requests;         /* device, the frame's distinct node ids     */
     uint32_t  nrequests;        /* capped at max_requests                    */
     uint32_t  nrequests_total;  /* distinct ids before the cap               */
-    double    ms_raycast;       /* HIP-event time of the ray-cast kernel     */
+    double    ms_raycast;       /* HIP-event time of the ray-cast kernel, the
+                                   listing of the requests included          */
     double    ms_requests;      /* 0: the cast lists its requests itself     */
     const float* rgba_f32;      /* device, width*height*4 floats: FragColor  */
 } vox_frame_view;
@@ -96,8 +98,8 @@ vox_raycaster* vox_raycaster_create(vox_octree* tree, int32_t max_width, int32_t
                                     uint32_t max_requests);
 void vox_raycaster_destroy(vox_raycaster* rc);
 const char* vox_raycaster_get_error(vox_raycaster* rc);
-/* One frame: ray cast, then request deduplication, queued on the ray
- * caster's stream. */
+/* One frame, queued on the ray caster's stream: the cast, whose waves list
+ * the frame's distinct node ids as they end. */
 int vox_raycast_frame(vox_raycaster* rc, const vox_camera* cam, const vox_raycast_params* prm);
 /* The last frame's buffers, counts and timings (waits for the frame). */
 int vox_raycaster_get_frame(vox_raycaster* rc, vox_frame_view* out);
@@ -154,7 +156,8 @@ int vox_composite(vox_raycaster* const* rcs, uint32_t n, float* dst, int32_t wid
  *     slots and their node texels get the resident bit and brick pointer.
  * Entries that find no slot stay in the FIFO for later frames.  The latency
  * of an admitted request is the device clock from the ray cast appending it
- * to the end of its brick copy. */
+ * (when the wave that met the node ends, so with part of the frame's cast
+ * still to come) to the end of its brick copy. */
 typedef struct vox_server vox_server;
 
 typedef struct vox_server_stats {

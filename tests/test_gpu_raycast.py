@@ -147,3 +147,21 @@ def test_raycast_brick_step_that_is_no_number(case):
     finally:
         for o in (srv, rc, t, bp, vz):
             o.close()
+
+
+def test_frame_times_hold_no_request_stage():
+    """The cast lists its requests itself: one time, and 0 for a separate pass."""
+    scene = scenes.scene_small_terrain()
+    vz = voxelize_scene(scene)
+    bp = BrickPool(scene.B, (4, 4, 4))
+    t = OctTree(bp, vz)
+    rc = RayCaster(t, 64, 48)
+    try:
+        look, up = look_at((0.5, -0.6, 1.3), (0.5, 0.5, 0.5))
+        for f in range(3):
+            v = rc.frame(camera((0.5, -0.6, 1.3), look, up, 45.0, 64, 48, f),
+                         raycast_params((0.0,) * 3, (1.0,) * 3))
+            assert v.ms_raycast > 0.0 and v.ms_requests == 0.0
+    finally:
+        for o in (rc, t, bp, vz):
+            o.close()

@@ -700,13 +700,13 @@ struct vox_raycaster {
     size_t hostCap[2] = {0, 0};
     hipEvent_t tableCopied[2] = {nullptr, nullptr};
     int tableNext = 0;
-    hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
+    hipEvent_t ev[2] = {nullptr, nullptr};   // round the last frame's cast
     hipEvent_t done = nullptr;  // the last frame's request list is complete
     hipEvent_t read = nullptr;  // a composite has read the last frame
     int32_t rect[4] = {0, 0, 0, 0};  // pixels the last frame wrote
     bool timingPending = false, countsPending = false, haveJitter = false, readPending = false;
     uint64_t jitterSeed = 0;
-    double msRay = 0, msReq = 0;
+    double msRay = 0;
     std::stringstream err;
     std::string errCache;
     bool fail(const std::string& m) {
@@ -932,12 +932,10 @@ namespace {
 // Timings of the frame whose events were recorded last (waits for it).
 void settle_timing(vox_raycaster* rc) {
     if (!rc->timingPending) return;
-    (void)hipEventSynchronize(rc->ev[2]);
-    float a = 0, b = 0;
+    (void)hipEventSynchronize(rc->ev[1]);
+    float a = 0;
     (void)hipEventElapsedTime(&a, rc->ev[0], rc->ev[1]);
-    (void)hipEventElapsedTime(&b, rc->ev[1], rc->ev[2]);
     rc->msRay = a;
-    rc->msReq = b;
     rc->timingPending = false;
 }
 
@@ -993,9 +991,7 @@ int vox_raycast_frame(vox_raycaster* rc, const vox_camera* cam, const vox_raycas
     rc->rect[1] = U.ry0;
     rc->rect[2] = U.rx1;
     rc->rect[3] = U.ry1;
-    // the requests are listed by the cast itself: no time of their own
     (void)hipEventRecord(rc->ev[1], st);
-    (void)hipEventRecord(rc->ev[2], st);
     if (!rc->check(hipGetLastError(), "raycast kernels") ||
         !rc->check(hipEventRecord(rc->done, st), "event record"))
         return 0;
@@ -1118,7 +1114,6 @@ int vox_raycast_frame_multi(vox_raycaster* const* rcs, uint32_t n, const vox_cam
                                            reinterpret_cast<float4*>(frame), transmittance,
                                            resume ? 1 : 0);
     (void)hipEventRecord(r0->ev[1], st);
-    (void)hipEventRecord(r0->ev[2], st);
     if (!r0->check(hipGetLastError(), "raycast multi kernel")) return 0;
     r0->timingPending = true;
     for (uint32_t k = 0; k < n; ++k) {
@@ -1184,7 +1179,7 @@ int vox_raycaster_get_frame(vox_raycaster* rc, vox_frame_view* out) {
     out->nrequests = rc->nreq;
     out->nrequests_total = rc->nreqTotal;
     out->ms_raycast = rc->msRay;
-    out->ms_requests = rc->msReq;
+    out->ms_requests = 0.0;   // listed by the cast itself: no time of their own
     return 1;
 }
 
