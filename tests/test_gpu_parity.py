@@ -109,3 +109,14 @@ def test_brick_wider_than_the_gather_tile_table():
 @pytest.mark.parametrize("N,B", [(32, 8), (36, 9), (78, 39), (80, 40)])
 def test_brick_sizes_at_the_gather_s_edges(N, B):
     _check(scenes.scene_mixed(seed=21, N=N, B=B))
+
+
+# bricks that reach 6 or 7 tiles an axis by where they start (some staged, some
+# read from the maps, in one launch), the widest of them, the next, which
+# always reach 7, and bricks that are flat on one axis
+@pytest.mark.parametrize("N,B", [((176,) * 3, (44,) * 3), ((184,) * 3, (46,) * 3),
+                                 ((188,) * 3, (47,) * 3), ((320, 320, 32), (80, 80, 8))], ids=str)
+def test_bricks_staged_by_the_tiles_they_reach(N, B):
+    cube = scenes.scene_mixed(seed=22, N=max(N), B=max(B))
+    _check(scenes.Scene(meshes=cube.meshes, N=N, B=B, name=f"staged_{B[0]}_{B[2]}",
+                        p=cube.p, delta=cube.delta))

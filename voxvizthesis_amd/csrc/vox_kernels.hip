@@ -1899,9 +1899,10 @@ __global__ void k_brick_assign_all(uint64_t allNodes, const uint32_t* __restrict
 // reads before their stores, so they take a wave each and not a workgroup
 // of four, for more bricks in flight.
 constexpr uint32_t kGatherBatch = 16;
-constexpr uint32_t kGatherTiles = 216;   // tiles under a brick, at most 6 per axis: any B <= 39
+constexpr uint32_t kGatherDirect = 8;    // the same without the tables
+constexpr uint32_t kGatherTiles = 216;   // tiles under a brick, 6 per axis: any B <= 39, some B <= 46
 struct GatherLds {
-    uint32_t tiles, rows, ex;            // capacities
+    uint32_t tiles, rows, ex;            // capacities; a brick over more tiles does without
     __host__ __device__ uint32_t words() const { return tiles * (kTileWords + 1) + rows + ex; }
 };
 template <int kThreads>
@@ -1924,24 +1925,61 @@ __device__ __forceinline__ void brick_gather_at(
     const float invx = __builtin_amdgcn_rcpf((float)ex), invy = __builtin_amdgcn_rcpf((float)ey);
     uint32_t* __restrict__ outC = bcol + j * nvox;
     uint32_t* __restrict__ outN = bnrm + j * nvox;
-    if (cap.tiles == 0u) {
-        // a brick too large for LDS: the tile map and the words from memory
-        // for every voxel
-        for (uint32_t i = tid; i < nvox; i += kThreads) {
-            const uint32_t row = udiv_small(i, ex, invx), z = udiv_small(row, ey, invy);
-            const uint32_t X = r0x + i - row * ex, Y = r0y + row - z * ey, Z = r0z + z;
-            const int64_t ta = tile_of(lm, X, Y, Z);
-            const uint32_t v = vox_of(X, Y, Z);
-            const bool def = ta >= 0 && stored(lm, (uint64_t)ta, v);
-            outC[i] = def ? col[(uint64_t)ta * kTileVox + v] : 0u;
-            outN[i] = def ? qn[(uint64_t)ta * kTileVox + v] : kZeroNormalQ;
-        }
-        return;
-    }
     const uint32_t t0x = r0x >> 3, t0y = r0y >> 3, t0z = r0z >> 3;
     const uint32_t ntx = ((r0x + ex - 1) >> 3) - t0x + 1, nty = ((r0y + ey - 1) >> 3) - t0y + 1,
                    ntz = ((r0z + ez - 1) >> 3) - t0z + 1;
     const uint32_t ntl = ntx * nty * ntz;
+    // voxel i as (x, row), moved on by kThreads
+    uint32_t row = udiv_small(tid, ex, invx), x = tid - row * ex;
+    const uint32_t drow = udiv_small(kThreads, ex, invx), dx = kThreads - drow * ex;
+    if (ntl > cap.tiles) {   // uniform: the brick decides, by the tiles it reaches
+        // the tile map and the words from memory for every voxel: the reads of
+        // kGatherDirect voxels are in flight together, step by step (one voxel
+        // at a time: 1.10 ms for the 64^3 bricks of a 512^3 terrain, so 0.45)
+        for (uint32_t i0 = tid; i0 < nvox; i0 += kGatherDirect * kThreads) {
+            int32_t ta[kGatherDirect];
+            uint32_t v[kGatherDirect], w[kGatherDirect], c[kGatherDirect], q[kGatherDirect];
+#pragma unroll
+            for (uint32_t u = 0; u < kGatherDirect; ++u) {
+                const uint32_t z = udiv_small(row, ey, invy);
+                const uint32_t X = r0x + x, Y = r0y + row - z * ey, Z = r0z + z;
+                v[u] = vox_of(X, Y, Z);
+                ta[u] = -1;
+                if (i0 + u * kThreads < nvox)
+                    ta[u] = lm.tileIdx[((uint64_t)(Z >> 3) * lm.TG[1] + (Y >> 3)) * lm.TG[0] + (X >> 3)];
+                x += dx;
+                row += drow;
+                if (x >= ex) { x -= ex; ++row; }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kGatherDirect; ++u) {
+                w[u] = ta[u] >= 0 ? ~0u : 0u;
+                if (lm.defOcc && ta[u] >= 0) {
+                    const uint64_t o = (uint64_t)ta[u] * kTileWords + (v[u] >> 5);
+                    w[u] = lm.defOcc[o] | lm.defFill[o];
+                }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kGatherDirect; ++u) {
+                c[u] = 0u;
+                q[u] = kZeroNormalQ;
+                if ((w[u] >> (v[u] & 31u)) & 1u) {
+                    const uint64_t o = (uint64_t)ta[u] * kTileVox + v[u];
+                    c[u] = col[o];
+                    q[u] = qn[o];
+                }
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kGatherDirect; ++u) {
+                const uint32_t i = i0 + u * kThreads;
+                if (i < nvox) {
+                    outC[i] = c[u];
+                    outN[i] = q[u];
+                }
+            }
+        }
+        return;
+    }
     const float invTx = __builtin_amdgcn_rcpf((float)ntx), invTy = __builtin_amdgcn_rcpf((float)nty);
     for (uint32_t i = tid; i < ntl * kTileWords; i += kThreads) {
         const uint32_t tl = i / kTileWords, w = i % kTileWords;
@@ -1964,9 +2002,6 @@ __device__ __forceinline__ void brick_gather_at(
     for (uint32_t x = tid; x < ex; x += kThreads)
         s_x[x] = (((r0x + x) >> 3) - t0x) * 512u + ((r0x + x) & 7u);
     __syncthreads();
-    // voxel i as (x, row), moved on by kThreads
-    uint32_t row = udiv_small(tid, ex, invx), x = tid - row * ex;
-    const uint32_t drow = udiv_small(kThreads, ex, invx), dx = kThreads - drow * ex;
     for (uint32_t i0 = tid; i0 < nvox; i0 += kGatherBatch * kThreads) {
         uint32_t c[kGatherBatch], q[kGatherBatch];
 #pragma unroll
@@ -3348,14 +3383,17 @@ void launch_brick_assign_all(hipStream_t st, const uint32_t* flag, const uint32_
 }
 void launch_brick_gather_all(hipStream_t st, const GatherDepths& G) {
     if (G.n <= 0 || G.start[G.n] == 0) return;
-    // tiles a brick's B + 2 voxels reach on an axis, at most
-    uint64_t tiles = 1, nvox = 1;
+    // tiles a brick's B + 2 voxels reach, at most and at least
+    uint64_t tiles = 1, least = 1, nvox = 1;
     for (int a = 0; a < 3; ++a) {
         tiles *= (G.B[a] + (uint64_t)kTile) / kTile + 1u;
+        least *= (G.B[a] + (uint64_t)kTile + 1u) / kTile;
         nvox *= G.B[a] + 2u;
     }
     GatherLds cap{};
-    if (tiles <= kGatherTiles) cap = {(uint32_t)tiles, (G.B[1] + 2u) * (G.B[2] + 2u), G.B[0] + 2u};
+    if (least <= kGatherTiles)
+        cap = {(uint32_t)std::min<uint64_t>(tiles, kGatherTiles), (G.B[1] + 2u) * (G.B[2] + 2u),
+               G.B[0] + 2u};
     // (bricks so flat and wide that their tables take over 32 KB do without)
     if (cap.words() > 8192u) cap = GatherLds{};
     const unsigned bricks = (unsigned)G.start[G.n];
