@@ -2615,17 +2615,27 @@ __device__ __forceinline__ uint32_t chunk_tile_active(const LevelMap& src, const
                     return 1u;
     return 0u;
 }
+// The tile map of a level whose tiles read other source tiles than 2 x 2 x 2:
+// a thread per tile, as a tile's walk over its source tiles (up to 512 where
+// chunks are a voxel wide) is long beside the map's writes, and the levels
+// with such walks are small (480^3 in chunks of 96^3, three such levels: four
+// tiles a thread 61 us a level, so 19).
 __global__ __launch_bounds__(kBlock) void k_chunk_map(LevelMap src, LevelMap dst, ChunkGeom cg,
                                                       int ks, int kd,
                                                       int32_t* __restrict__ tileIdx,
                                                       int32_t* __restrict__ list,
                                                       uint32_t* __restrict__ count) {
-    map_tiles<1>(dst.numTiles, [&](uint64_t t0) {
-        uint32_t m = 0u;
-        for (int k = 0; k < kMapTiles; ++k)
-            if (t0 + k < dst.numTiles && chunk_tile_active(src, dst, cg, ks, kd, t0 + k)) m |= 1u << k;
-        return m;
-    }, tileIdx, list, count);
+    __shared__ uint32_t s_w[kBlock / 64];
+    __shared__ uint32_t s_base;
+    const uint64_t t = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
+    const bool in = t < dst.numTiles;
+    const bool on = in && chunk_tile_active(src, dst, cg, ks, kd, t) != 0u;
+    uint32_t total;
+    const uint32_t o = block_excl_scan(on ? 1u : 0u, s_w, &total);
+    if (threadIdx.x == 0) s_base = total ? atomicAdd(count, total) : 0u;
+    __syncthreads();
+    if (on) list[s_base + o] = (int32_t)t;
+    if (in) tileIdx[t] = on ? (int32_t)(s_base + o) : -1;
 }
 
 // ComputeVoxelMipMap8 (VoxelizerKernels.cu 1520-1663) inside each chunk:
@@ -3470,8 +3480,8 @@ void launch_mip_source_count(hipStream_t st, const LevelMap& src, const LevelMap
 void launch_chunk_map(hipStream_t st, const LevelMap& src, const LevelMap& dst, const ChunkGeom& cg,
                       int ks, int kd, int32_t* tileIdx, int32_t* list, uint32_t* count) {
     if (dst.numTiles == 0) return;
-    k_chunk_map<<<grid_for(dst.numTiles, kMapBlock), kBlock, 0, st>>>(src, dst, cg, ks, kd, tileIdx,
-                                                                      list, count);
+    k_chunk_map<<<grid_for(dst.numTiles, kBlock), kBlock, 0, st>>>(src, dst, cg, ks, kd, tileIdx,
+                                                                   list, count);
 }
 void launch_chunk_mip(hipStream_t st, const LevelMap& src, const LevelMap& dst,
                       const ChunkGeom& cg, int ks, int kd, uint64_t nActive,
