@@ -82,3 +82,29 @@ def test_device_assignment_sizes(ntri, dim, spread):
             assert a.zmin[t] == z.min() and a.zmax[t] == z.max(), f"tile {t}"
         else:
             assert np.isnan(a.zmin[t]) and np.isnan(a.zmax[t]), f"tile {t}"
+
+
+# waves of few boxes (triangles sorted along rows of tiles) and of many (in no
+# order), boxes of a tile or two and boxes over much of the grid, counted in LDS
+# and in memory
+@pytest.mark.parametrize("dim", [(1, 1), (6, 4), (32, 32), (1024, 1), (40, 40), (3, 700)])
+@pytest.mark.parametrize("rows", [True, False])
+@pytest.mark.parametrize("spread", [0.2, 12.0])
+def test_device_assignment_orders(dim, rows, spread):
+    from voxvizthesis_amd import _lib
+    verts = _soup(1500, 7, dim, spread)
+    if rows:
+        c = np.floor(verts.mean(1))
+        verts = np.ascontiguousarray(verts[np.lexsort((c[:, 0], c[:, 1]))])
+    g = _lib.VoxTileGrid()
+    g.origin[:], g.size[:], g.border[:], g.dim[:] = (0.0, 0.0), (1.0, 1.0), (0.1, 0.1), dim
+    print(f"[tiler] {dim} rows={rows} spread={spread}", flush=True)
+    a = TileAssignment(verts, g)
+    ref = ot.assign(verts, (0.0, 0.0), (1.0, 1.0), (0.1, 0.1), dim)
+    assert a.start[-1] == a.tris.size == sum(map(len, ref.values()))
+    for t in range(dim[0] * dim[1]):
+        want = ref.get(t, [])
+        assert a.tile(t).tolist() == want, f"tile {t}"
+        if want:
+            z = verts[want][:, :, 2]
+            assert a.zmin[t] == z.min() and a.zmax[t] == z.max(), f"tile {t}"

@@ -85,13 +85,20 @@ __device__ __forceinline__ int32_t ord(float f) {
 }
 
 // Grids of at most kLdsTiles tiles keep a count per tile and wave and the z
-// extents per tile in LDS (24 bytes per tile and workgroup: 24 KB at the
-// most, six workgroups per CU).
+// extents per tile in LDS: 24 bytes per tile and workgroup beside the 9 KB of
+// staged vertices, 33 KB at the most, four workgroups (one per SIMD and wave)
+// a CU.  There the split takes 134 us for 2 M triangles of a heightfield on 32 x
+// 32 tiles and 500 in no order, the sort on 40 x 40 tiles 260 and 640.
 constexpr uint32_t kLdsTiles = 1024;
 constexpr int kWaves = kB / 64;
 // Waves a split is spread over at most: four per SIMD, and the (tile, wave)
-// counts it scans stay below 2^22.
+// counts it scans are at most 2^22.
 constexpr uint64_t kSplitWaves = 4096;
+
+// Tiles of a box, first | last << 16 per axis.
+__device__ __forceinline__ uint64_t box_tiles(uint32_t xr, uint32_t yr) {
+    return (uint64_t)((xr >> 16) - (xr & 0xffffu) + 1u) * ((yr >> 16) - (yr & 0xffffu) + 1u);
+}
 
 __device__ __forceinline__ int32_t wave_min(int32_t v) {
 #pragma unroll
@@ -103,40 +110,140 @@ __device__ __forceinline__ int32_t wave_min(int32_t v) {
 }
 
 // Every tile that a wave's triangles reach, once: visit(tile, m) with m the
-// lanes whose box holds it.  xr, yr: a lane's box, first | last << 16.  The
-// lanes with one and the same box are taken together (neighbouring triangles
-// mostly share theirs); a tile that the box of an earlier lane holds has been
-// visited with it.
+// lanes whose box holds it.  xr, yr: a lane's box, first | last << 16.  Either
+// box by box, the lanes with one and the same box taken together (neighbouring
+// triangles mostly share theirs; a tile that the box of an earlier lane holds
+// has been visited with it), or every tile of the box round them all, whichever
+// are fewer tiles (2,000 triangles over about half of 32 x 32 tiles each: 4.3 ms
+// a call with box by box alone, so 0.39).
 template <class F>
 __device__ __forceinline__ void each_tile(bool act, uint32_t xr, uint32_t yr, uint32_t dimx,
                                           F visit) {
-    uint64_t pend = __ballot(act);
+    const uint64_t all = __ballot(act);
+    if (!all) return;
+    const int f = __ffsll((unsigned long long)all) - 1;
+    const uint32_t fx = __builtin_amdgcn_readlane(xr, f), fy = __builtin_amdgcn_readlane(yr, f);
+    uint32_t x0 = fx & 0xffffu, x1 = fx >> 16, y0 = fy & 0xffffu, y1 = fy >> 16;
+    uint64_t pend = all & ~__ballot(xr == fx && yr == fy);
+    if (!pend) {   // one box
+        for (uint32_t y = y0; y <= y1; ++y)
+            for (uint32_t x = x0; x <= x1; ++x) visit(y * dimx + x, all);
+        return;
+    }
+    // else the box round them all, and the boxes' own tiles
+    uint64_t tiles = box_tiles(fx, fy);
     while (pend) {
         const int l = __ffsll((unsigned long long)pend) - 1;
         const uint32_t lx = __builtin_amdgcn_readlane(xr, l);
         const uint32_t ly = __builtin_amdgcn_readlane(yr, l);
-        const uint64_t same = __ballot(act && xr == lx && yr == ly);
-        const bool only = same == __ballot(act);
-        pend &= ~same;
+        pend &= ~__ballot(xr == lx && yr == ly);
+        tiles += box_tiles(lx, ly);
+        x0 = min(x0, lx & 0xffffu);
+        x1 = max(x1, lx >> 16);
+        y0 = min(y0, ly & 0xffffu);
+        y1 = max(y1, ly >> 16);
+    }
+    auto holding = [&](uint32_t x, uint32_t y) {
+        return __ballot(act && x >= (xr & 0xffffu) && x <= xr >> 16 && y >= (yr & 0xffffu) &&
+                        y <= yr >> 16);
+    };
+    if (box_tiles(x0 | (x1 << 16), y0 | (y1 << 16)) <= tiles) {
+        for (uint32_t y = y0; y <= y1; ++y)
+            for (uint32_t x = x0; x <= x1; ++x) {
+                const uint64_t m = holding(x, y);
+                if (m) visit(y * dimx + x, m);
+            }
+        return;
+    }
+    pend = all;
+    while (pend) {
+        const int l = __ffsll((unsigned long long)pend) - 1;
+        const uint32_t lx = __builtin_amdgcn_readlane(xr, l);
+        const uint32_t ly = __builtin_amdgcn_readlane(yr, l);
+        pend &= ~__ballot(xr == lx && yr == ly);
         for (uint32_t y = ly & 0xffffu; y <= ly >> 16; ++y)
             for (uint32_t x = lx & 0xffffu; x <= lx >> 16; ++x) {
-                uint64_t m = same;
-                if (!only) {
-                    m = __ballot(act && x >= (xr & 0xffffu) && x <= xr >> 16 &&
-                                 y >= (yr & 0xffffu) && y <= yr >> 16);
-                    if (m & ((1ull << l) - 1ull)) continue;
-                }
-                visit(y * dimx + x, m);
+                const uint64_t m = holding(x, y);
+                if (!(m & ((1ull << l) - 1ull))) visit(y * dimx + x, m);
             }
     }
+}
+
+// The counts and z extents of a wave's triangles, by atomics: add(tile, n, lo,
+// hi).  Two ways, as atomics in LDS cost less than those in memory.  Either has
+// lanes whose boxes few others share walk their own (2 M triangles in no order:
+// 0.94 ms a call on 32 x 32 tiles with the lanes of every tile reduced, so
+// 0.49; on 40 x 40, in memory, 1.14 and 0.64).
+//
+// In LDS: the lanes with one and the same box are reduced and its tiles spread
+// over the lanes; the rest, or what the first kBoxes boxes leave over, walk.
+constexpr int kBoxes = 8, kShared = 8;
+template <class F>
+__device__ __forceinline__ void count_lds(bool act, uint32_t xr, uint32_t yr, int32_t zlo,
+                                          int32_t zhi, uint32_t dimx, F add) {
+    const uint32_t lane = threadIdx.x & 63u;
+    bool alone = act;
+    uint64_t pend = __ballot(act);
+    for (int k = 0; k < kBoxes && pend; ++k) {
+        const int l = __ffsll((unsigned long long)pend) - 1;
+        const uint32_t lx = __builtin_amdgcn_readlane(xr, l);
+        const uint32_t ly = __builtin_amdgcn_readlane(yr, l);
+        const uint64_t same = __ballot(act && xr == lx && yr == ly);
+        pend &= ~same;
+        const int n = __popcll(same);
+        if (n < kShared) continue;
+        const bool in = (same >> lane) & 1ull;
+        alone = alone && !in;
+        const int32_t lo = wave_min(in ? zlo : 0x7fffffff);
+        // the maximum of a as the complement of the minimum of ~a
+        const int32_t hi = ~wave_min(in ? ~zhi : 0x7fffffff);
+        const uint32_t w = (lx >> 16) - (lx & 0xffffu) + 1u, tiles = (uint32_t)box_tiles(lx, ly);
+        for (uint32_t i = lane; i < tiles; i += 64u) {   // at most kLdsTiles
+            const uint32_t y = i / w, x = i - y * w;
+            add(((ly & 0xffffu) + y) * dimx + (lx & 0xffffu) + x, (uint32_t)n, lo, hi);
+        }
+    }
+    if (alone)
+        for (uint32_t y = yr & 0xffffu; y <= yr >> 16; ++y)
+            for (uint32_t x = xr & 0xffffu; x <= xr >> 16; ++x) add(y * dimx + x, 1u, zlo, zhi);
+}
+// In memory: a wave of at most kFew boxes has one atomic a tile, any other's
+// lanes walk (8 boxes: 508 us for 272 for 2 M triangles of a heightfield on
+// 200 x 200 tiles; the boxes reduced one by one as in LDS: 435).
+constexpr int kFew = 16;
+template <class F>
+__device__ __forceinline__ void count_mem(bool act, uint32_t xr, uint32_t yr, int32_t zlo,
+                                          int32_t zhi, uint32_t dimx, F add) {
+    uint64_t pend = __ballot(act);
+    for (int k = 0; k < kFew && pend; ++k) {
+        const int l = __ffsll((unsigned long long)pend) - 1;
+        pend &= ~__ballot(xr == (uint32_t)__builtin_amdgcn_readlane(xr, l) &&
+                          yr == (uint32_t)__builtin_amdgcn_readlane(yr, l));
+    }
+    if (pend) {   // uniform: boxes are left
+        if (act)
+            for (uint32_t y = yr & 0xffffu; y <= yr >> 16; ++y)
+                for (uint32_t x = xr & 0xffffu; x <= xr >> 16; ++x) add(y * dimx + x, 1u, zlo, zhi);
+        return;
+    }
+    const uint32_t lane = threadIdx.x & 63u;
+    each_tile(act, xr, yr, dimx, [&](uint32_t tile, uint64_t m) {
+        const bool in = (m >> lane) & 1ull;
+        if (__popcll(m) == 1) {
+            if (in) add(tile, 1u, zlo, zhi);
+            return;
+        }
+        const int32_t lo = wave_min(in ? zlo : 0x7fffffff);
+        const int32_t hi = ~wave_min(in ? ~zhi : 0x7fffffff);
+        if (lane == 0u) add(tile, (uint32_t)__popcll(m), lo, hi);
+    });
 }
 
 // First pass of the split: each triangle's tile box (ranges), the triangles
 // per (tile, wave), and the tiles' z extents.  Wave w takes the triangles
 // [w * per * 64, (w + 1) * per * 64).  Bound by reading the vertices once
 // (36 bytes a triangle), which are staged through LDS with 16-byte loads,
-// the next 64 triangles' in flight while the current ones are counted; the z
-// extents are reduced in the wave before they meet an atomic.  2.26 M
+// the next 64 triangles' in flight while the current ones are counted.  2.26 M
 // triangles on a 4 x 4 grid: 50 us (81 MB of vertices at 1.6 TB/s).
 __global__ __launch_bounds__(kB) void k_split_count(const float* __restrict__ verts, uint64_t ntri,
                                                     Grid g, uint32_t n, uint32_t per, uint32_t nw,
@@ -197,17 +304,12 @@ __global__ __launch_bounds__(kB) void k_split_count(const float* __restrict__ ve
         if (act) ranges[t] = make_uint2(xr, yr);
         const int32_t zlo = ord(fminf(fminf(v[2], v[5]), v[8]));
         const int32_t zhi = ord(fmaxf(fmaxf(v[2], v[5]), v[8]));
-        each_tile(act, xr, yr, g.dim[0], [&](uint32_t tile, uint64_t m) {
-            const bool in = (m >> lane) & 1ull;
-            const int32_t lo = wave_min(in ? zlo : 0x7fffffff);
-            // the maximum of a as the complement of the minimum of ~a
-            const int32_t hi = ~wave_min(in ? ~zhi : 0x7fffffff);
-            if (lane == 0u) {
-                lds[tile * kWaves + wv] += (uint32_t)__popcll(m);
-                atomicMin(&s_lo[tile], lo);
-                atomicMax(&s_hi[tile], hi);
-            }
-        });
+        count_lds(act, xr, yr, zlo, zhi, g.dim[0],
+                  [&](uint32_t tile, uint32_t k, int32_t lo, int32_t hi) {
+                      atomicAdd(&lds[tile * kWaves + wv], k);
+                      atomicMin(&s_lo[tile], lo);
+                      atomicMax(&s_hi[tile], hi);
+                  });
     }
     __syncthreads();
     for (uint32_t t = tid; t < n; t += kB) {
@@ -255,9 +357,8 @@ __global__ __launch_bounds__(kB) void k_split_write(const uint2* __restrict__ ra
 }
 
 // Counts per tile and per triangle, and the tiles' z extents (grids of more
-// than kLdsTiles tiles).  The lanes of a wave that share a tile reduce their
-// extents before one of them meets the atomics: with an atomic per lane, the
-// same-address traffic took 28.4 ms for 2.26 M triangles on a 4 x 4 grid.
+// than kLdsTiles tiles).  Bound by the atomics: with one per lane and extent,
+// 2.26 M triangles on a 4 x 4 grid took 28.4 ms.
 __global__ void k_tile_count(const float* __restrict__ verts, uint64_t ntri, Grid g,
                              uint32_t* __restrict__ cnt, uint32_t* __restrict__ triCnt,
                              int32_t* __restrict__ zmin, int32_t* __restrict__ zmax) {
@@ -274,25 +375,18 @@ __global__ void k_tile_count(const float* __restrict__ verts, uint64_t ntri, Gri
     if (act0) triCnt[t] = (x1 - x0 + 1u) * (y1 - y0 + 1u);
     const int32_t zlo = ord(fminf(fminf(v[2], v[5]), v[8]));
     const int32_t zhi = ord(fmaxf(fmaxf(v[2], v[5]), v[8]));
-    const uint32_t lane = threadIdx.x & 63u;
-    each_tile(act0, x0 | (x1 << 16), y0 | (y1 << 16), g.dim[0], [&](uint32_t tile, uint64_t m) {
-        const bool in = (m >> lane) & 1ull;
-        if (__popcll(m) == 1) {
-            if (in) {
-                atomicAdd(&cnt[tile], 1u);
-                atomicMin(&zmin[tile], zlo);
-                atomicMax(&zmax[tile], zhi);
-            }
-            return;
-        }
-        const int32_t lo = wave_min(in ? zlo : 0x7fffffff);
-        const int32_t hi = ~wave_min(in ? ~zhi : 0x7fffffff);
-        if (lane == 0u) {
-            atomicAdd(&cnt[tile], (uint32_t)__popcll(m));
-            atomicMin(&zmin[tile], lo);
-            atomicMax(&zmax[tile], hi);
-        }
-    });
+    count_mem(act0, x0 | (x1 << 16), y0 | (y1 << 16), zlo, zhi, g.dim[0],
+              [&](uint32_t tile, uint32_t k, int32_t lo, int32_t hi) {
+                  atomicAdd(&cnt[tile], k);
+                  // a lane of its own looks first: an extent only widens, so
+                  // one that is wide enough already needs no atomic
+                  if (k != 1u || lo < __hip_atomic_load(&zmin[tile], __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_WORKGROUP))
+                      atomicMin(&zmin[tile], lo);
+                  if (k != 1u || hi > __hip_atomic_load(&zmax[tile], __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_WORKGROUP))
+                      atomicMax(&zmax[tile], hi);
+              });
 }
 
 // The (tile, triangle) pairs of triangle t at its offset: pairs in
@@ -559,7 +653,7 @@ int vox_tiler_assign(vox_tiler* t, const float* verts, uint64_t ntri, int32_t de
         return 0;
     k_z_init<<<grid_for(n), kB, 0, st>>>(n, t->zmin.as<int32_t>(), t->zmax.as<int32_t>());
     // The split through LDS wherever the tiles' counters fit there (2.26 M
-    // triangles on a 4 x 4 grid: 108 us a call; the sort's pairs, its three
+    // triangles on a 4 x 4 grid: 103 us a call; the sort's pairs, its three
     // passes and their scans alone took 100 us of device time beside the
     // count); the sort beyond.
     return (ntri && n <= kLdsTiles ? assign_split(t, verts, ntri, g, (uint32_t)n)
