@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import oracle
-from voxvizthesis_amd import scenes
+from voxvizthesis_amd import _lib, scenes
 from voxvizthesis_amd._lib import VOX_OPT_MIP_CHAIN
 from voxvizthesis_amd.gvpool import BrickPool, OctTree
 from voxvizthesis_amd.gvserve import RayCaster, camera, raycast_params
@@ -163,5 +163,37 @@ def test_frame_times_hold_no_request_stage():
                          raycast_params((0.0,) * 3, (1.0,) * 3))
             assert v.ms_raycast > 0.0 and v.ms_requests == 0.0
     finally:
+        for o in (rc, t, bp, vz):
+            o.close()
+
+
+def test_frame_taller_than_a_grid_has_rows_of_workgroups():
+    """A wave casts four rows and a grid holds 65536 workgroups in y: a frame of
+    more rows than both together equals the oracle's."""
+    from voxvizthesis_amd.gvserve import raycast_front_to_back
+    scene, (W, H) = scenes.scene_small_terrain(), (1, 4 * 65536 + 37)
+    vz = voxelize_scene(scene)
+    bp = BrickPool(scene.B, (4, 4, 4))
+    t = OctTree(bp, vz)
+    rc = RayCaster(t, W, H)
+    frame = _lib.DeviceArray.alloc(16 * W * H)
+    try:
+        look, up = look_at((0.5, -0.6, 1.3), (0.5, 0.5, 0.5))
+        cam = dict(position=(0.5, -0.6, 1.3), look=look, up=up, fov_y_deg=45.0, width=W, height=H)
+        prm = dict(vol_min=(0.0,) * 3, vol_max=(1.0,) * 3, jitter_seed=3)
+        print(f"[raycast] {W}x{H}", flush=True)
+        rc.frame(camera(**cam), raycast_params(**prm))
+        ru, rcol = oracle.raycast(cam, prm, vz.raw_result().levels, scene.B, t.nodes(),
+                                  bp.textures()[0])
+        assert (ru != 0).any()
+        assert np.array_equal(rc.usage(), ru) and np.array_equal(rc.rgba(), rcol)
+        # front to back over the one octree: the same frame times its alpha
+        own, f = rc.rgba_f32(), np.full((H, W, 4), -1.0, np.float32)
+        raycast_front_to_back([rc], camera(**cam), [raycast_params(**prm)], frame.ptr)
+        rc.requests()   # waits for the frame
+        assert rc._L.vox_device_download(f.ctypes.data, frame.ptr, 0, f.nbytes)
+        assert np.array_equal(f, own * own[..., 3:])
+    finally:
+        frame.close()
         for o in (rc, t, bp, vz):
             o.close()

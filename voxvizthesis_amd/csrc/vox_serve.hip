@@ -551,13 +551,21 @@ __device__ __forceinline__ void append_requests(const RequestList& R, const uint
 // pass over the usage lists in a kernel of its own read 100 MB back at
 // 1080p and met few equal ids per wave: 154 us beside a cast of 0.91 ms).
 constexpr int kCastW = 16, kCastH = 4;   // pixels of a wave
+// Workgroups over w x h pixels; rows of them past a grid's 65536 go on in z.
+dim3 cast_grid(uint32_t w, uint32_t h) {
+    const uint32_t rows = (h + kCastH - 1) / kCastH, y = std::min(rows, 32768u);
+    return dim3((w + kCastW - 1) / kCastW, y, (rows + y - 1) / y);
+}
+__device__ __forceinline__ int cast_row() {
+    return (int)((blockIdx.z * gridDim.y + blockIdx.y) * kCastH + threadIdx.x / kCastW);
+}
 template <bool kOddStep>
 __global__ void __launch_bounds__(kCastW * kCastH)
 k_raycast(RayUniforms U, const uint32_t* __restrict__ tex, const uint32_t* __restrict__ pool,
           const float* __restrict__ jitter, uint32_t* __restrict__ rgbaOut,
           float4* __restrict__ rgbaF, uint32_t* __restrict__ usageOut, RequestList R) {
     const int i = U.rx0 + (int)blockIdx.x * kCastW + (int)(threadIdx.x % kCastW);
-    const int j = U.ry0 + (int)blockIdx.y * kCastH + (int)(threadIdx.x / kCastW);
+    const int j = U.ry0 + cast_row();
     uint32_t usage[kMaxUsage];
     if (i < U.rx1 && j < U.ry1) {
         float dst[4];
@@ -612,7 +620,7 @@ k_raycast_multi(const TreeCast* __restrict__ trees, uint32_t n, const float* __r
                 float4* __restrict__ frame, float* __restrict__ trans, int resume) {
     // pixels of the union of the octrees' rectangles, [x0, x1) x [y0, y1)
     const int i = x0 + (int)blockIdx.x * kCastW + (int)(threadIdx.x % kCastW);
-    const int j = y0 + (int)blockIdx.y * kCastH + (int)(threadIdx.x / kCastW);
+    const int j = y0 + cast_row();
     const bool in = i < x1 && j < y1;
     const uint64_t pix = (uint64_t)j * W + i;
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -979,7 +987,7 @@ int vox_raycast_frame(vox_raycaster* rc, const vox_camera* cam, const vox_raycas
     }
     launch_fill_u32(st, rc->counts.as<uint32_t>(), 2, 0u);
     (void)hipEventRecord(rc->ev[0], st);
-    dim3 grid((rw + kCastW - 1) / kCastW, (rh + kCastH - 1) / kCastH);
+    const dim3 grid = cast_grid(rw, rh);
     const RequestList R{rc->stamp.as<uint32_t>(), rc->req.as<uint32_t>(),
                         rc->reqTime.as<unsigned long long>(), rc->counts.as<uint32_t>(), rc->tag,
                         rc->maxReq};
@@ -1104,8 +1112,7 @@ int vox_raycast_frame_multi(vox_raycaster* const* rcs, uint32_t n, const vox_cam
         !r0->check(hipEventRecord(r0->tableCopied[b], st), "event record"))
         return 0;
     (void)hipEventRecord(r0->ev[0], st);
-    dim3 grid((unsigned)(ux1 - ux0 + kCastW - 1) / kCastW,
-              (unsigned)(uy1 - uy0 + kCastH - 1) / kCastH);
+    const dim3 grid = cast_grid((uint32_t)(ux1 - ux0), (uint32_t)(uy1 - uy0));
     bool odd = false;
     for (const TreeCast& tc : table) odd = odd || tc.U.oddStep;
     const auto cast = odd ? k_raycast_multi<true> : k_raycast_multi<false>;
