@@ -83,6 +83,27 @@ def test_device_tile_windows(x0, y0, cw, ch, off):
         t.close()
 
 
+def test_height_ranges_of_many_short_threads():
+    """Ranges of windows on more threads at once than pairs are kept for, each
+    thread ending after its own."""
+    from concurrent.futures import ThreadPoolExecutor
+    t = DeviceTerrain(300, 1.0, 11)
+    try:
+        g = t.grid()
+
+        def one(k):
+            x, y, w, h = k, 2 * k, 1 + 5 * k, 1 + 3 * k
+            win = g[y:y + h, x:x + w]
+            return t.range(x, y, w, h) == (win.min(), win.max())
+
+        for _ in range(2):
+            print("[terrain] ranges on threads", flush=True)
+            with ThreadPoolExecutor(24) as ex:
+                assert all(ex.map(one, range(48)))
+    finally:
+        t.close()
+
+
 def snapshot(vz):
     r = vz.result()
     out = [r["occupancy"]]

@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -263,6 +264,35 @@ __global__ __launch_bounds__(256) void k_range(const float* __restrict__ H, uint
         out[2 * blockIdx.x + 1] = hi;
     }
 }
+
+// The pairs of one call, for its length: kept for the next call of any thread
+// (at most kPairsKept, the rest freed), not by a thread, whose end would then
+// free them after the runtime's own state of the thread is gone, and wait for
+// the device.
+constexpr size_t kPairsKept = 16;
+std::mutex g_pairsMu;
+std::vector<int32_t*> g_pairs;
+struct Pairs {
+    int32_t* p = nullptr;
+    Pairs() {
+        std::lock_guard<std::mutex> lk(g_pairsMu);
+        if (g_pairs.empty()) return;
+        p = g_pairs.back();
+        g_pairs.pop_back();
+    }
+    ~Pairs() {
+        if (!p) return;
+        {
+            std::lock_guard<std::mutex> lk(g_pairsMu);
+            if (g_pairs.size() < kPairsKept) {
+                g_pairs.push_back(p);
+                return;
+            }
+        }
+        (void)hipHostFree(p);
+    }
+};
+
 float from_ordered(int32_t o) {
     const int32_t b = o >= 0 ? o : (int32_t)(0x80000000u - (uint32_t)o - 1u);
     float f;
@@ -311,15 +341,8 @@ int vox_terrain_range(const float* heights, uint32_t n1, uint32_t x0, uint32_t y
     if (!heights || !out_minmax || w == 0 || h == 0 || (uint64_t)x0 + w > n1 ||
         (uint64_t)y0 + h > n1)
         return fail("vox_terrain_range: window outside the grid"), 0;
-    // the workgroups' pairs, in pinned host memory that the kernel writes
-    // itself: one buffer per calling thread, given back when it ends
-    struct Pairs {
-        int32_t* p = nullptr;
-        ~Pairs() {
-            if (p) (void)hipHostFree(p);
-        }
-    };
-    thread_local Pairs pairs;
+    // the workgroups' pairs, in pinned host memory that the kernel writes itself
+    Pairs pairs;
     if (!pairs.p && !check(hipHostMalloc(reinterpret_cast<void**>(&pairs.p), 8 * kRangeBlocks,
                                          hipHostMallocDefault),
                            "vox_terrain_range"))
