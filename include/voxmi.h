@@ -106,7 +106,8 @@ typedef struct vox_stats {
     uint64_t active_tiles[VOX_MAX_LEVELS]; /* 8^3 voxel tiles per mip level    */
     uint64_t occupied_voxels;
     uint64_t bricks_total;
-    double   ms_total;                /* HIP-event time of the device pipeline  */
+    double   ms_total;                /* HIP-event time of vox_generate's device
+                                         work (without the setup pass)          */
     int32_t  nkernels;
     char     kernel_name[64][32];
     double   kernel_ms[64];           /* summed per kernel name                */
@@ -179,7 +180,10 @@ void vox_deallocate_voxel_memory(vox_ctx* h);
 int  vox_allocate_triangle_memory(vox_ctx* h);
 void vox_deallocate_triangle_memory(vox_ctx* h);
 /* cuda::Voxelizer::computeEdgesFaceNormalsAndBounds (Voxelizer.cu 459-489):
- * per-triangle setup and binning of triangles to 8^3 voxel tiles. */
+ * per-triangle setup and the count of triangles per 8^3 voxel tile, queued on
+ * the handle's stream: the call does not wait for them.  An error of their run,
+ * and of the memory for the tiles' triangle lists (which vox_generate sizes and
+ * fills), is reported by the vox_generate that follows. */
 int vox_compute_edges_face_normals_and_bounds(vox_ctx* h);
 /* cuda::Voxelizer::generateVoxelsAndOctTree (Voxelizer.cu 2180-2814).
  * Returns 1 ok, 0 error, -1 no group overlaps the grid.  out_dir may be NULL

@@ -82,6 +82,7 @@ public:
     void deallocateTriangleMemory() { vox_deallocate_triangle_memory(_h); }
     bool allocateVoxelMemory() { return vox_allocate_voxel_memory(_h) == 1; }
     void deallocateVoxelMemory() { vox_deallocate_voxel_memory(_h); }
+    // Queued, not waited for: generateVoxelsAndOctTree reports errors of its run.
     bool computeEdgesFaceNormalsAndBounds() {
         return vox_compute_edges_face_normals_and_bounds(_h) == 1;
     }

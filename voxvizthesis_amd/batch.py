@@ -101,7 +101,8 @@ def make_job(scene, B: int, persistent_blocks: int = 0, options: int = 0) -> Vox
 
 def autotune(scene, edges=(8, 16, 32), blocks_per_cu=(4, 8, 16), cus: int = 256, reps: int = 2,
              keep: bool = False):
-    """Time eager generates of the scene for every brick edge and persistent
+    """Time eager generates of the scene (with the setup pass, which is queued
+    before each and runs into it) for every brick edge and persistent
     launch shape (one voxelizer per brick edge, its launch shape changed
     between timings); return (B, persistent_blocks, ms) of the fastest, and
     with keep=True also that voxelizer, set to the chosen shape (the caller
@@ -118,9 +119,9 @@ def autotune(scene, edges=(8, 16, 32), blocks_per_cu=(4, 8, 16), cus: int = 256,
                         raise RuntimeError(vz.getErrorMessage())
                     t = math.inf
                     for _ in range(reps):
-                        vz.computeEdgesFaceNormalsAndBounds()
                         t0 = time.perf_counter()
-                        if vz.generateVoxelsAndOctTree(None) == 0:
+                        if not vz.computeEdgesFaceNormalsAndBounds() or \
+                                vz.generateVoxelsAndOctTree(None) == 0:
                             raise RuntimeError(vz.getErrorMessage())
                         t = min(t, (time.perf_counter() - t0) * 1e3)
                     if best is None or t < best[2]:

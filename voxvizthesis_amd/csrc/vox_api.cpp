@@ -2,9 +2,9 @@
 //
 // Mirrors cuda::Voxelizer (Voxelizer.h 22-244, Voxelizer.cu): the same
 // call sequence and return conventions, but the whole pipeline runs on one
-// HIP stream with everything resident in HBM.  Host round trips are limited
-// to three small counter reads per vox_generate (bin entries, active tiles
-// per level, bricks per level) that size the next allocations.
+// HIP stream with everything resident in HBM.  Beside the wait for its end, a
+// vox_generate waits twice for counts that size the next allocations (bin
+// entries and active tiles per level, bricks per level).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -92,6 +92,8 @@ class Voxelizer:
         self._keep = []
 
     def computeEdgesFaceNormalsAndBounds(self) -> bool:
+        """Queue the setup pass (not waited for: errors of its run are
+        reported by generateVoxelsAndOctTree)."""
         return bool(self._L.vox_compute_edges_face_normals_and_bounds(self._h))
 
     def generateVoxelsAndOctTree(self, outputDir=None, outputBinary=True,
