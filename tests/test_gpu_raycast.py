@@ -197,3 +197,44 @@ def test_frame_taller_than_a_grid_has_rows_of_workgroups():
         frame.close()
         for o in (rc, t, bp, vz):
             o.close()
+
+
+# deeper trees in boxes off the unit cube, long on one axis, and far from the
+# origin, resident in texture pools and in wide ones; bricks whose side in the
+# pool is no power of two.  The level-of-detail test, the step counts and the
+# quotients by the pool's sides then take values that the unit box does not.
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("N,B,lo,size", [
+    (256, 8, (0.0, 0.0, 0.0), (1.0, 1.0, 1.0)), (256, 8, (3.25, -7.5, 0.125), (4.0, 4.0, 4.0)),
+    (192, 12, (-700.0, 300.0, 40.0), (32.0, 8.0, 2.0)), (224, 7, (0.1, 0.2, 0.3), (0.7, 0.9, 0.05))])
+def test_raycast_boxes_and_deep_trees(N, B, lo, size, wide):
+    from voxvizthesis_amd.gvserve import BrickServer
+    scene, (W, H) = scenes.scene_terrain_n(128, N, B), (97, 61)
+    vz = voxelize_scene(scene)
+    slots = 16 * (N // B) ** 2 + 64
+    k = int(np.ceil(slots ** (1 / 3)))
+    bp = BrickPool(scene.B, wide_slots=slots, normals=False) if wide else BrickPool(scene.B, (k,) * 3)
+    t = OctTree(bp, vz)
+    rc, srv = RayCaster(t, W, H), BrickServer(t)
+    lo, size = np.asarray(lo, np.float32), np.asarray(size, np.float32)
+    prm = dict(vol_min=lo, vol_max=lo + size, jitter_seed=3)
+    try:
+        for n, (pos, target, fov) in enumerate([((0.5, -0.6, 1.3), (0.5, 0.5, 0.5), 45.0),
+                                                ((0.41, 0.37, 0.56), (0.6, 0.52, 0.5), 75.0),
+                                                ((6.0, 5.0, 4.0), (0.5, 0.5, 0.5), 10.0)]):
+            pos, target = (lo + size * np.asarray(q) for q in (pos, target))
+            look, up = look_at(pos, target)
+            cam = dict(position=pos, look=look, up=up, fov_y_deg=fov, width=W, height=H, frame=n)
+            print(f"[raycast] N={N} B={B} box {lo} {size} wide={wide} pose {n}", flush=True)
+            for _ in range(40):
+                rc.frame(camera(**cam), raycast_params(**prm))
+                if srv.frame(rc).last_uploads == 0:
+                    break
+            rc.frame(camera(**cam), raycast_params(**prm))
+            ru, rcol = oracle.raycast(cam, prm, vz.raw_result().levels, scene.B, t.nodes(),
+                                      bp.textures()[0], wide=wide)
+            assert (ru != 0).any()
+            assert np.array_equal(rc.usage(), ru) and np.array_equal(rc.rgba(), rcol)
+    finally:
+        for o in (srv, rc, t, bp, vz):
+            o.close()

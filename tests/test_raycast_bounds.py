@@ -3,145 +3,153 @@
 The device decides a node's level-of-detail test from a range of voxel half
 sizes (lod_range) and a node's step count from products with reciprocals
 (exit_steps) wherever rounding cannot change the outcome, and takes c / 255,
-quotients by the pool's sides and the trilinear weights from products.  Restated here in fp32 and compared with the stated
-arithmetic on drawn rays."""
-import ctypes
-import math
+quotients by the pool's sides and the trilinear weights from products.  The
+functions and constants that the kernels are built from (vox_raymath.h), built
+here without a device, against the stated arithmetic on drawn rays, with square
+roots and reciprocals one unit in the last place off either way."""
+import ctypes as C
+import os
+import subprocess
 
 import numpy as np
 import pytest
 
+from voxvizthesis_amd import _lib
+from voxvizthesis_amd.gvserve import camera, raycast_params
+
 f = np.float32
-LIBM = ctypes.CDLL("libm.so.6")
-LIBM.fmaf.restype = ctypes.c_float
-LIBM.fmaf.argtypes = [ctypes.c_float] * 3
-U24 = 2.0 ** -24
+HERE = os.path.dirname(os.path.abspath(__file__))
 
 
-def dot(a, b):
-    return ((a[..., 0] * b[..., 0] + a[..., 1] * b[..., 1]) + a[..., 2] * b[..., 2]).astype(f)
+@pytest.fixture(scope="module")
+def rm(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("raymath") / "raymath_check.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off",
+                    "-Wall", "-Wno-unknown-pragmas", os.path.join(HERE, "cpp", "raymath_check.cpp"),
+                    "-o", so], check=True)
+    L = C.CDLL(so)
+    L.rm_uniforms.restype = C.c_void_p
+    L.rm_uniforms.argtypes = [C.POINTER(_lib.VoxCamera), C.POINTER(_lib.VoxRaycastParams), C.c_int,
+                              C.c_uint32, C.c_uint32, C.c_uint32]
+    for name, args in (("rm_free", [C.c_void_p]), ("rm_odd_step", [C.c_void_p]),
+                       ("rm_lod", [C.c_void_p, C.c_int, C.c_void_p, C.c_int] + [C.c_void_p] * 2),
+                       ("rm_exit", [C.c_void_p, C.c_int] + [C.c_void_p] * 4 + [C.c_int] +
+                        [C.c_void_p] * 4),
+                       ("rm_div_by", [C.c_int, C.c_void_p, C.c_float, C.c_void_p]),
+                       ("rm_weigh", [C.c_int] + [C.c_void_p] * 4), ("rm_unorm8_256", [C.c_uint32])):
+        getattr(L, name).argtypes = args
+    L.rm_unorm8_256.restype = C.c_float
+    return L
 
 
-def normalize(v):
-    return (v * (f(1) / np.sqrt(dot(v, v)))[..., None]).astype(f)
+def ptr(*arrays):
+    return [a.ctypes.data for a in arrays]
 
 
-def lod_constants(up, left, vol, cam, root_half, pixel, lod):
-    M = max(abs(float(v)) for v in vol) + max(abs(float(c)) for c in cam)
-    M += 2.0 * root_half * (np.abs(up).max() + np.abs(left).max())
-    tau = max(0.0, pixel / lod) * (1 + 1e-5) + 2.0 ** -20
-    return (f(1.001 * (np.linalg.norm(up) + np.linalg.norm(left))),
-            f(1.03 * math.sqrt(2.18 * tau) / 1.6),
-            f(1.03 * 2 * math.pi * 7 * M * U24 / 1.6))
+def uniforms(rm, pos, look, up, fov, W, H, lo, hi, levels=7, brick=16, pool=144, wide=0, step=0.0):
+    U = rm.rm_uniforms(C.byref(camera(pos, look, up, fov, W, H)),
+                       C.byref(raycast_params(lo, hi, ray_step=step)), levels, brick, pool, wide)
+    assert U
+    return U
 
 
 # a camera in the volume, beside it, far off; wide and narrow pixels; a volume
-# off the unit cube
-@pytest.mark.parametrize("spread,fov,height,shift", [
-    (0.5, 60.0, 1080, 0.0), (0.05, 60.0, 1080, 0.0), (0.002, 70.0, 64, 0.0),
-    (3.0, 35.0, 720, 0.0), (40.0, 20.0, 1440, 0.0), (0.5, 60.0, 1080, 3.25)])
-def test_lod_range_never_decides_against_the_test(spread, fov, height, shift):
+# off the unit cube, and ones that are long on one axis
+@pytest.mark.parametrize("spread,fov,height,shift,size", [
+    (0.5, 60.0, 1080, 0.0, (1, 1, 1)), (0.05, 60.0, 1080, 0.0, (1, 1, 1)),
+    (0.002, 70.0, 64, 0.0, (1, 1, 1)), (3.0, 35.0, 720, 0.0, (1, 1, 1)),
+    (40.0, 20.0, 1440, 0.0, (1, 1, 1)), (0.5, 60.0, 1080, 3.25, (1, 1, 1)),
+    (0.5, 60.0, 1080, -700.0, (32, 8, 2)), (0.5, 60.0, 480, 0.0, (0.01, 0.01, 4))])
+def test_lod_range_never_decides_against_the_test(rm, spread, fov, height, shift, size):
     rng = np.random.default_rng(int(1000 * spread) + height)
-    n, decided, total = 4000, 0, 0
+    n, levels, decided, total = 4000, 10, 0, 0
+    size = np.array(size, np.float64)
     for _ in range(12):
         look = rng.normal(size=3)
         look /= np.linalg.norm(look)
         up = np.cross(look, rng.normal(size=3))
-        up = (up / np.linalg.norm(up)).astype(f)
-        look = look.astype(f)
-        left = np.cross(up, look).astype(f)
-        p = (rng.random((n, 3)) + shift).astype(f)
-        cam = (0.5 + shift + spread * rng.normal(size=3)).astype(f)
-        pixel = 1.0 - math.cos(math.sqrt(2) * 2 * math.tan(math.radians(fov) / 2) / height)
-        pixel, lod = float(f(pixel)), 10.0
-        root = f(1.0 / 16 * 0.5)
-        lu, k1, k2 = lod_constants(up, left, (shift, 1 + shift), cam, float(root), pixel, lod)
-        d = (p - cam).astype(f)
-        u = (left - up).astype(f)
-        c = np.stack([d[:, 1] * u[2] - d[:, 2] * u[1], d[:, 2] * u[0] - d[:, 0] * u[2],
-                      d[:, 0] * u[1] - d[:, 1] * u[0]], -1).astype(f)
-        A, C2 = dot(d, d), dot(c, c)
-        ok = C2 >= f(1e-6) * A * lu * lu
-        with np.errstate(divide="ignore", invalid="ignore"):
-            # the device's square roots and reciprocals are approximate: one
-            # unit in the last place, on the side that decides more
-            rA = np.sqrt(A)
-            lo = np.where(ok, (A * k1 + rA * k2) / np.sqrt(C2) * f(1 - 2.0 ** -21), np.inf)
-            hi = np.where(ok, rA * f(0.49) / lu * f(1 + 2.0 ** -21), 0.0)
-        for k in range(10):
-            h = f(float(root) * 0.5 ** k)
-            sure = (h >= lo) & (h <= hi)
-            ll = normalize((((p - up * h) + left * h) - cam).astype(f))
-            ur = normalize((((p + up * h) - left * h) - cam).astype(f))
-            proj = (f(1) - dot(ll, ur)) * f(lod)
-            assert not (sure & (f(pixel) > proj)).any()
-            decided += int(sure.sum())
-            total += n
+        up /= np.linalg.norm(up)
+        lo = np.full(3, shift)
+        pos = lo + size * (0.5 + spread * rng.normal(size=3))
+        U = uniforms(rm, pos, look, up, fov, height * 16 // 9, height, lo, lo + size)
+        p = rng.random((n, 3)).astype(f)   # unit-volume coordinates
+        sure, stop = np.empty((2, n, levels), np.uint8)
+        for ulp in (-1, 0, 1):
+            rm.rm_ulp(ulp)
+            rm.rm_lod(U, n, *ptr(p), levels, *ptr(sure, stop))
+            assert not (sure & stop).any()
+        decided += int(sure.sum())
+        total += sure.size
+        rm.rm_free(U)
     print(f"decided {decided} of {total}")
-    assert spread > 1 or decided > 0.2 * total
+    assert spread > 1 or max(size) / min(size) > 4 or decided > 0.2 * total
 
 
 @pytest.mark.parametrize("levels", [2, 5, 8])
-def test_exit_steps_equal_the_divided_ones(levels):
+def test_exit_steps_equal_the_divided_ones(rm, levels):
     rng = np.random.default_rng(levels)
-    n = 400000
-    step = f(0.5 / (16 << (levels - 1)))
-    x = np.abs(rng.random((n, 3)) * rng.choice([1.0, 0.1, 1e-3, 0.0], (n, 1))).astype(f)
-    x[rng.random((n, 3)) < 0.02] = 0
-    x[: n // 50] *= f(-1)                 # a point just outside the node
-    # many quotients at and near whole numbers
-    k = rng.integers(1, 60, n // 4)
+    n = 200000
+    U = uniforms(rm, (0.5, -1.0, 0.5), (0, 1, 0), (0, 0, 1), 60.0, 64, 64, (0,) * 3, (1,) * 3,
+                 levels)
+    step = 0.5 / (16 << (levels - 1))
     d = rng.normal(size=(n, 3))
-    d = np.abs(d / np.linalg.norm(d, axis=1, keepdims=True)).astype(f)
+    d = (d / np.linalg.norm(d, axis=1, keepdims=True)).astype(f)
     d[rng.random((n, 3)) < 0.02] = 0
-    x[: n // 4] = (d[: n // 4] * (k * float(step))[:, None]).astype(f)
-    with np.errstate(divide="ignore", invalid="ignore", over="ignore"):
-        t = np.where((d > 0) & (x != 0), x / d, f(np.inf)).astype(f)
-        want = (np.minimum(f(4), t.min(1)) / step).astype(np.float32)
-        want = np.trunc(want).astype(np.int64) + 1
-        for ulp in (-1, 0, 1):            # a reciprocal may be one off
-            r = np.where(d != 0, (f(1) / d), f(0)).astype(f)
-            r = (r * f(1 + ulp * 2.0 ** -23)).astype(f)
-            tx = (x * r).astype(f)
-            q = np.minimum(f(4), np.where(tx != 0, tx, f(np.inf)).min(1))
-            q = (q * (f(1) / step)).astype(f)
-            e = (np.abs(q) * f(1e-6)).astype(f)
-            a, b = np.trunc(q - e), np.trunc(q + e)
-            sure = (a == b) & (np.abs(q) < 1e6) & (r.max(1) < 1e30)
-            assert (a[sure].astype(np.int64) + 1 == want[sure]).all()
-            # (a quarter of the rows lie on every face: the quotient of the
-            # limit 4 by the step, a whole number, which is divided out)
-            assert sure[n // 4:].mean() > 0.74
+    d[rng.random((n, 3)) < 0.01] *= f(1e-40)             # reciprocals that overflow
+    size = rng.choice([1.0, 0.125, 2.0 ** -6], (n, 1))
+    mn = (np.floor(rng.random((n, 3)) / size) * size).astype(f)
+    mx = (mn + size).astype(f)
+    p = (mn + size * rng.random((n, 3))).astype(f)
+    p = np.where(rng.random((n, 3)) < 0.02, mn, p)       # on a face, and just outside
+    p[: n // 50] = np.nextafter(mx[: n // 50], f(2))
+    # quotients at and near whole numbers: k steps before the exit face in x
+    k = rng.integers(1, 60, n // 4)[:, None] * step
+    m = slice(n - n // 4, n)
+    p[m] = np.where(d[m] > 0, mx[m] - d[m] * k, mn[m] - d[m] * k).astype(f)
+    for e in (0, 1, levels - 1):
+        for ulp in (-1, 0, 1):
+            rm.rm_ulp(ulp)
+            fast, want, used = np.empty((3, n), np.int32)
+            sure = np.empty(n, np.uint8)
+            rm.rm_exit(U, n, *ptr(p, d, mn, mx), e, *ptr(fast, sure, want, used))
+            assert (used == want).all() and (fast == want)[sure != 0].all()
+            assert sure[: n // 2].mean() > 0.7
+    rm.rm_free(U)
 
 
-def fma(a, b, c):
-    """Fused multiply-add in fp32 of scalars (the C library's)."""
-    return LIBM.fmaf(float(a), float(b), float(c))
-
-
-def test_unorm8_is_the_rounded_quotient():
-    k = float.fromhex("0x1.010102p-8")
+def test_unorm8_is_the_rounded_quotient(rm):
     for c in range(256):
-        assert f(fma(c, k, c)) == f(256) * (f(c) / f(255))
+        assert f(rm.rm_unorm8_256(c)) == f(256) * (f(c) / f(255))
 
 
 # brick texels per axis of wide pools (B + 2) and of texture pools
 @pytest.mark.parametrize("b", [3, 6, 9, 18, 34, 66, 100, 144, 288, 720, 1023, 1024])
-def test_div_by_is_the_rounded_quotient(b):
+def test_div_by_is_the_rounded_quotient(rm, b):
     rng = np.random.default_rng(b)
-    r = f(1) / f(b)
-    a = np.concatenate([rng.random(4000) * 16, np.exp2(rng.uniform(-80, 10, 4000)),
-                        np.arange(1024)]).astype(f)
-    for x in a:
-        q = x * r
-        assert f(fma(fma(-q, b, x), r, q)) == x / f(b)
+    a = np.concatenate([rng.random(40000) * 16, np.exp2(rng.uniform(-149, 10, 40000)),
+                        np.arange(1024), [0.0]]).astype(f)
+    out = np.empty_like(a)
+    rm.rm_div_by(a.size, *ptr(a), b, *ptr(out))
+    assert np.array_equal(out, a / f(b))
 
 
-def test_weight_products_are_exact():
-    w = np.arange(257)
+def test_weighed_samples_equal_the_products(rm):
     rng = np.random.default_rng(1)
-    x, y, z = (rng.choice(w, 20000) for _ in range(3))
-    want = ((x / 256).astype(f) * (y / 256).astype(f)) * (z / 256).astype(f)
-    got = (x.astype(f) * y.astype(f)) * (z.astype(f) * f(2.0 ** -32))
-    assert (got * f(256) == want).all()
-    assert (want.astype(np.float64) == x * y * z / 2.0 ** 24).all()
+    n = 20000
+    t = rng.integers(0, 2 ** 32, (n, 8), dtype=np.uint32) * (rng.random((n, 8)) < 0.7)
+    t = np.ascontiguousarray(t, np.uint32)
+    w = rng.integers(0, 257, (n, 3)).astype(f)
+    got, want = np.empty((2, n, 4), f)
+    rm.rm_weigh(n, *ptr(t, w, got, want))
+    assert np.array_equal(got, want)
+
+
+def test_brick_steps_that_are_no_number_are_found(rm):
+    tiny = float(np.finfo(f).smallest_subnormal)
+    view = ((0.5, -1.0, 0.5), (0, 1, 0), (0, 0, 1), 60.0, 65, 65)
+    for lo, hi, step, odd in [((0,) * 3, (1,) * 3, 0.0, 0), ((0,) * 3, (2 * tiny, 1, 1), 0.0, 1),
+                              ((0,) * 3, (1, 1e38, 1), 0.45, 1), ((0,) * 3, (1, 1e-30, 1), 0.0, 0)]:
+        for wide in (0, 1):
+            U = uniforms(rm, *view, lo, hi, levels=4, brick=8, pool=100, wide=wide, step=step)
+            assert rm.rm_odd_step(U) == odd
+            rm.rm_free(U)
