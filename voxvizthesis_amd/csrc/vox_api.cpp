@@ -915,7 +915,7 @@ int gen_front(vox_ctx* h) {
         std::memcpy(act, h->planAct, sizeof(act));
         h->pairs = h->planPairs;
     } else {
-        h->run("tile_map", [&] {
+        h->run("counts", [&] {
             launch_map_counts(st, ctr, L, h->binStart.as<uint32_t>() + h->numBins,
                               h->pin + kPinTiles);
         });
@@ -1193,7 +1193,7 @@ int gen_back(vox_ctx* h, const char* out_dir, int binary) {
     // the counts the host needs, left in pinned memory
     auto counts = [&](const uint32_t* excl, const uint64_t* offs, const uint32_t* cnt) {
         if (h->replay) return;
-        h->run("scan", [&] {
+        h->run("counts", [&] {
             launch_generate_counts(st, excl, offs, cnt, L, reinterpret_cast<uint32_t*>(satc),
                                    ctr + kScanErrWord, h->pin + kPinCounts);
         });

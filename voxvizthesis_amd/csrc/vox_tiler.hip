@@ -244,7 +244,7 @@ __device__ __forceinline__ void count_mem(bool act, uint32_t xr, uint32_t yr, in
 // [w * per * 64, (w + 1) * per * 64).  Bound by reading the vertices once
 // (36 bytes a triangle), which are staged through LDS with 16-byte loads,
 // the next 64 triangles' in flight while the current ones are counted.  2.26 M
-// triangles on a 4 x 4 grid: 50 us (81 MB of vertices at 1.6 TB/s).
+// triangles on a 4 x 4 grid: 45 us (81 MB of vertices at 1.8 TB/s).
 __global__ __launch_bounds__(kB) void k_split_count(const float* __restrict__ verts, uint64_t ntri,
                                                     Grid g, uint32_t n, uint32_t per, uint32_t nw,
                                                     int aligned, uint2* __restrict__ ranges,
