@@ -772,7 +772,7 @@ def main():
         if name == "voxelize":
             # fraction above is of HBM bandwidth; what bounds this kernel is
             # VALU issue (SQ counters, profiles/full_octree_traffic.md)
-            out["limiter"] = "VALU issue: ~75 % of the SIMDs' VALU issue rate (SQ counters)"
+            out["limiter"] = "VALU issue: 67 % of the busy CUs' issue slots (SQ counters)"
         return out
 
     # The roofline names k_voxelize (one launch per triangle group), the
