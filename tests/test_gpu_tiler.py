@@ -86,8 +86,10 @@ def test_device_assignment_sizes(ntri, dim, spread):
 
 # waves of few boxes (triangles sorted along rows of tiles) and of many (in no
 # order), boxes of a tile or two and boxes over much of the grid, counted in LDS
-# and in memory
-@pytest.mark.parametrize("dim", [(1, 1), (6, 4), (32, 32), (1024, 1), (40, 40), (3, 700)])
+# and in memory; grids at the 32 tiles from which the lists are written by a lane
+# per tile, and of one and several rows in its 64
+@pytest.mark.parametrize("dim", [(1, 1), (6, 4), (31, 1), (8, 4), (13, 5), (65, 2), (32, 32),
+                                 (1024, 1), (40, 40), (3, 700)])
 @pytest.mark.parametrize("rows", [True, False])
 @pytest.mark.parametrize("spread", [0.2, 12.0])
 def test_device_assignment_orders(dim, rows, spread):

@@ -87,8 +87,8 @@ __device__ __forceinline__ int32_t ord(float f) {
 // Grids of at most kLdsTiles tiles keep a count per tile and wave and the z
 // extents per tile in LDS: 24 bytes per tile and workgroup beside the 9 KB of
 // staged vertices, 33 KB at the most, four workgroups (one per SIMD and wave)
-// a CU.  There the split takes 134 us for 2 M triangles of a heightfield on 32 x
-// 32 tiles and 500 in no order, the sort on 40 x 40 tiles 260 and 640.
+// a CU.  There the split takes 137 us for 2 M triangles of a heightfield on 32 x
+// 32 tiles and 384 in no order, the sort on 40 x 40 tiles 263 and 693.
 constexpr uint32_t kLdsTiles = 1024;
 constexpr int kWaves = kB / 64;
 // Waves a split is spread over at most: four per SIMD, and the (tile, wave)
@@ -109,16 +109,21 @@ __device__ __forceinline__ int32_t wave_min(int32_t v) {
     return v;
 }
 
-// Every tile that a wave's triangles reach, once: visit(tile, m) with m the
-// lanes whose box holds it.  xr, yr: a lane's box, first | last << 16.  Either
-// box by box, the lanes with one and the same box taken together (neighbouring
-// triangles mostly share theirs; a tile that the box of an earlier lane holds
-// has been visited with it), or every tile of the box round them all, whichever
-// are fewer tiles (2,000 triangles over about half of 32 x 32 tiles each: 4.3 ms
-// a call with box by box alone, so 0.39).
-template <class F>
-__device__ __forceinline__ void each_tile(bool act, uint32_t xr, uint32_t yr, uint32_t dimx,
-                                          F visit) {
+// The lanes whose box (xr, yr: first | last << 16) holds tile (x, y).
+__device__ __forceinline__ uint64_t lanes_at(bool act, uint32_t xr, uint32_t yr, uint32_t x,
+                                             uint32_t y) {
+    return __ballot(act && x >= (xr & 0xffffu) && x <= xr >> 16 && y >= (yr & 0xffffu) &&
+                    y <= yr >> 16);
+}
+
+// Every tile that a wave's triangles reach, once: visit(x, y, m) with m the
+// lanes whose box holds it.  Box by box, the lanes with one and the same box
+// taken together (neighbouring triangles mostly share theirs; a tile that the
+// box of an earlier lane holds has been visited with it), or, where the box round
+// them all has no more tiles than the boxes, tile by tile of that one.  From
+// kSweep tiles round them all, sweep(x0, x1, y0, y1) over those instead.
+template <uint64_t kSweep, class V, class W>
+__device__ __forceinline__ void each_tile(bool act, uint32_t xr, uint32_t yr, V visit, W sweep) {
     const uint64_t all = __ballot(act);
     if (!all) return;
     const int f = __ffsll((unsigned long long)all) - 1;
@@ -127,10 +132,9 @@ __device__ __forceinline__ void each_tile(bool act, uint32_t xr, uint32_t yr, ui
     uint64_t pend = all & ~__ballot(xr == fx && yr == fy);
     if (!pend) {   // one box
         for (uint32_t y = y0; y <= y1; ++y)
-            for (uint32_t x = x0; x <= x1; ++x) visit(y * dimx + x, all);
+            for (uint32_t x = x0; x <= x1; ++x) visit(x, y, all);
         return;
     }
-    // else the box round them all, and the boxes' own tiles
     uint64_t tiles = box_tiles(fx, fy);
     while (pend) {
         const int l = __ffsll((unsigned long long)pend) - 1;
@@ -143,15 +147,16 @@ __device__ __forceinline__ void each_tile(bool act, uint32_t xr, uint32_t yr, ui
         y0 = min(y0, ly & 0xffffu);
         y1 = max(y1, ly >> 16);
     }
-    auto holding = [&](uint32_t x, uint32_t y) {
-        return __ballot(act && x >= (xr & 0xffffu) && x <= xr >> 16 && y >= (yr & 0xffffu) &&
-                        y <= yr >> 16);
-    };
-    if (box_tiles(x0 | (x1 << 16), y0 | (y1 << 16)) <= tiles) {
+    const uint64_t round = box_tiles(x0 | (x1 << 16), y0 | (y1 << 16));
+    if (round >= kSweep) {
+        sweep(x0, x1, y0, y1);
+        return;
+    }
+    if (round <= tiles) {
         for (uint32_t y = y0; y <= y1; ++y)
             for (uint32_t x = x0; x <= x1; ++x) {
-                const uint64_t m = holding(x, y);
-                if (m) visit(y * dimx + x, m);
+                const uint64_t m = lanes_at(act, xr, yr, x, y);
+                if (m) visit(x, y, m);
             }
         return;
     }
@@ -163,8 +168,8 @@ __device__ __forceinline__ void each_tile(bool act, uint32_t xr, uint32_t yr, ui
         pend &= ~__ballot(xr == lx && yr == ly);
         for (uint32_t y = ly & 0xffffu; y <= ly >> 16; ++y)
             for (uint32_t x = lx & 0xffffu; x <= lx >> 16; ++x) {
-                const uint64_t m = holding(x, y);
-                if (!(m & ((1ull << l) - 1ull))) visit(y * dimx + x, m);
+                const uint64_t m = lanes_at(act, xr, yr, x, y);
+                if (!(m & ((1ull << l) - 1ull))) visit(x, y, m);
             }
     }
 }
@@ -173,7 +178,7 @@ __device__ __forceinline__ void each_tile(bool act, uint32_t xr, uint32_t yr, ui
 // hi).  Two ways, as atomics in LDS cost less than those in memory.  Either has
 // lanes whose boxes few others share walk their own (2 M triangles in no order:
 // 0.94 ms a call on 32 x 32 tiles with the lanes of every tile reduced, so
-// 0.49; on 40 x 40, in memory, 1.14 and 0.64).
+// 0.50; on 40 x 40, in memory, 1.19 and 0.69).
 //
 // In LDS: the lanes with one and the same box are reduced and its tiles spread
 // over the lanes; the rest, or what the first kBoxes boxes leave over, walk.
@@ -207,36 +212,44 @@ __device__ __forceinline__ void count_lds(bool act, uint32_t xr, uint32_t yr, in
         for (uint32_t y = yr & 0xffffu; y <= yr >> 16; ++y)
             for (uint32_t x = xr & 0xffffu; x <= xr >> 16; ++x) add(y * dimx + x, 1u, zlo, zhi);
 }
-// In memory: a wave of at most kFew boxes has one atomic a tile, any other's
-// lanes walk (8 boxes: 508 us for 272 for 2 M triangles of a heightfield on
-// 200 x 200 tiles; the boxes reduced one by one as in LDS: 435).
+// In memory: a wave of at most kFew boxes, each of four lanes or more on average,
+// has one atomic a tile, any other's lanes walk (2 M triangles of a heightfield
+// on 200 x 200 tiles 272 us; with 8 boxes 508, the boxes reduced one by one as in
+// LDS 435).
 constexpr int kFew = 16;
+// Lanes of small boxes look at a tile's extents first: those only widen, so one
+// that is wide enough already needs no atomic (2 M triangles in no order on 40 x
+// 40 tiles: 0.91 ms without).  Over a large box the looks would be a chain of waits
+// that the atomics are not.
+constexpr uint32_t kLook = 4;
+constexpr uint32_t kFirst = 2048;   // workgroups that start together find nothing set
 template <class F>
 __device__ __forceinline__ void count_mem(bool act, uint32_t xr, uint32_t yr, int32_t zlo,
                                           int32_t zhi, uint32_t dimx, F add) {
-    uint64_t pend = __ballot(act);
-    for (int k = 0; k < kFew && pend; ++k) {
+    const uint64_t all = __ballot(act);
+    uint64_t pend = all;
+    int k = 0;
+    for (; k < kFew && pend; ++k) {
         const int l = __ffsll((unsigned long long)pend) - 1;
         pend &= ~__ballot(xr == (uint32_t)__builtin_amdgcn_readlane(xr, l) &&
                           yr == (uint32_t)__builtin_amdgcn_readlane(yr, l));
     }
-    if (pend) {   // uniform: boxes are left
+    if (pend || 4 * k > __popcll(all)) {   // uniform
+        const bool look = blockIdx.x >= kFirst && box_tiles(xr, yr) <= kLook;
         if (act)
             for (uint32_t y = yr & 0xffffu; y <= yr >> 16; ++y)
-                for (uint32_t x = xr & 0xffffu; x <= xr >> 16; ++x) add(y * dimx + x, 1u, zlo, zhi);
+                for (uint32_t x = xr & 0xffffu; x <= xr >> 16; ++x)
+                    add(y * dimx + x, 1u, zlo, zhi, look);
         return;
     }
     const uint32_t lane = threadIdx.x & 63u;
-    each_tile(act, xr, yr, dimx, [&](uint32_t tile, uint64_t m) {
+    auto visit = [&](uint32_t x, uint32_t y, uint64_t m) {
         const bool in = (m >> lane) & 1ull;
-        if (__popcll(m) == 1) {
-            if (in) add(tile, 1u, zlo, zhi);
-            return;
-        }
         const int32_t lo = wave_min(in ? zlo : 0x7fffffff);
         const int32_t hi = ~wave_min(in ? ~zhi : 0x7fffffff);
-        if (lane == 0u) add(tile, (uint32_t)__popcll(m), lo, hi);
-    });
+        if (lane == 0u) add(y * dimx + x, (uint32_t)__popcll(m), lo, hi, false);
+    };
+    each_tile<~0ull>(act, xr, yr, visit, [](uint32_t, uint32_t, uint32_t, uint32_t) {});
 }
 
 // First pass of the split: each triangle's tile box (ranges), the triangles
@@ -324,7 +337,13 @@ __global__ __launch_bounds__(kB) void k_split_count(const float* __restrict__ ve
 
 // Second pass: the wave's places in every tile's list (the scan of its
 // counts), handed out in triangle order.  Entries at or past cap are not
-// written (the host then grows the lists and runs the pass again).
+// written (the host then grows the lists and runs the pass again).  A wave
+// goes tile by tile, each a read and a write of a place that the next waits for,
+// or, over kSweepTiles tiles and more, a lane takes a tile and its triangles one
+// after the other (100 triangles in no order on 934 tiles 60 us and 19; 2 M on 32 x
+// 32 tiles 0.50 ms a call and 0.39; swept from 16 tiles on, 4 x 4 tiles take 205 us
+// for 153).
+constexpr uint64_t kSweepTiles = 32;
 __global__ __launch_bounds__(kB) void k_split_write(const uint2* __restrict__ ranges, uint64_t ntri,
                                                     uint32_t dimx, uint32_t n, uint32_t per,
                                                     uint32_t nw, const uint32_t* __restrict__ excl,
@@ -345,14 +364,44 @@ __global__ __launch_bounds__(kB) void k_split_write(const uint2* __restrict__ ra
         const bool act = t < t1;
         const uint2 cur = r;
         if (t + 64u < t1) r = ranges[t + 64u];
-        each_tile(act, cur.x, cur.y, dimx, [&](uint32_t tile, uint64_t m) {
+        auto visit = [&](uint32_t x, uint32_t y, uint64_t m) {
+            const uint32_t tile = y * dimx + x;
             const uint32_t at = place[tile * kWaves + wv];
             const uint64_t o = (uint64_t)at + (uint64_t)__popcll(m & ((1ull << lane) - 1ull));
             if (((m >> lane) & 1ull) && o < cap) tris[o] = (uint32_t)t;
             __builtin_amdgcn_wave_barrier();
             if (lane == 0u) place[tile * kWaves + wv] = at + (uint32_t)__popcll(m);
             __builtin_amdgcn_wave_barrier();
-        });
+        };
+        auto sweep = [&](uint32_t x0, uint32_t x1, uint32_t y0, uint32_t y1) {
+            const uint32_t w = x1 - x0 + 1u, tiles = w * (y1 - y0 + 1u);   // at most kLdsTiles
+            for (uint32_t i0 = 0; i0 < tiles; i0 += 64u) {
+                // the triangles whose boxes reach these 64 tiles' rows and, in
+                // one row, columns
+                const uint32_t i1 = min(i0 + 63u, tiles - 1u), ya = i0 / w, yb = i1 / w;
+                const uint32_t xa = ya == yb ? x0 + i0 - ya * w : x0;
+                const uint32_t xb = ya == yb ? x0 + i1 - yb * w : x1;
+                uint64_t left = __ballot(act && (cur.x & 0xffffu) <= xb && cur.x >> 16 >= xa &&
+                                         (cur.y & 0xffffu) <= y0 + yb && cur.y >> 16 >= y0 + ya);
+                if (!left) continue;
+                const uint32_t i = i0 + lane, dy = i / w, x = x0 + i - dy * w, y = y0 + dy;
+                const uint32_t tile = i < tiles ? y * dimx + x : 0u;
+                uint32_t at = place[tile * kWaves + wv];
+                for (; left; left &= left - 1ull) {
+                    const int l = __ffsll((unsigned long long)left) - 1;
+                    const uint32_t lx = __builtin_amdgcn_readlane(cur.x, l);
+                    const uint32_t ly = __builtin_amdgcn_readlane(cur.y, l);
+                    if (i < tiles && x >= (lx & 0xffffu) && x <= lx >> 16 && y >= (ly & 0xffffu) &&
+                        y <= ly >> 16) {
+                        if (at < cap) tris[at] = (uint32_t)(b + (uint32_t)l);
+                        ++at;
+                    }
+                }
+                if (i < tiles) place[tile * kWaves + wv] = at;
+                __builtin_amdgcn_wave_barrier();   // other lanes read it next
+            }
+        };
+        each_tile<kSweepTiles>(act, cur.x, cur.y, visit, sweep);
     }
 }
 
@@ -376,16 +425,17 @@ __global__ void k_tile_count(const float* __restrict__ verts, uint64_t ntri, Gri
     const int32_t zlo = ord(fminf(fminf(v[2], v[5]), v[8]));
     const int32_t zhi = ord(fmaxf(fmaxf(v[2], v[5]), v[8]));
     count_mem(act0, x0 | (x1 << 16), y0 | (y1 << 16), zlo, zhi, g.dim[0],
-              [&](uint32_t tile, uint32_t k, int32_t lo, int32_t hi) {
+              [&](uint32_t tile, uint32_t k, int32_t lo, int32_t hi, bool look) {
                   atomicAdd(&cnt[tile], k);
-                  // a lane of its own looks first: an extent only widens, so
-                  // one that is wide enough already needs no atomic
-                  if (k != 1u || lo < __hip_atomic_load(&zmin[tile], __ATOMIC_RELAXED,
-                                                        __HIP_MEMORY_SCOPE_WORKGROUP))
-                      atomicMin(&zmin[tile], lo);
-                  if (k != 1u || hi > __hip_atomic_load(&zmax[tile], __ATOMIC_RELAXED,
-                                                        __HIP_MEMORY_SCOPE_WORKGROUP))
-                      atomicMax(&zmax[tile], hi);
+                  bool low = true, high = true;
+                  if (look) {
+                      low = lo < __hip_atomic_load(&zmin[tile], __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+                      high = hi > __hip_atomic_load(&zmax[tile], __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_WORKGROUP);
+                  }
+                  if (low) atomicMin(&zmin[tile], lo);
+                  if (high) atomicMax(&zmax[tile], hi);
               });
 }
 
